@@ -28,11 +28,10 @@
 // Its logits are kept in base-2 units (q, the key bias and the pair bias
 // carry a factor log2(e)), which changes nothing but the rounding:
 // exp2(log2(e) x) = exp(x). Any other head dimension, or f32 precision, runs
-// a one-thread-per-query kernel in f32 on the natural units.
+// the same two products on the f32 MFMA, on the natural units.
 #include <algorithm>
 #include <cmath>
 #include <cstddef>
-#include <utility>
 
 #include "dma.h"
 #include "gemm.h"
@@ -411,56 +410,201 @@ struct FlashArgs {
   float clamp;
 };
 
-// One thread per (b, h, q), f32 arithmetic: the reference's recurrence
-// (attention.ts:688-723) with the query and the accumulator in registers,
-// one instance per head dimension D.
-template <typename CT, int D>
-__global__ __launch_bounds__(256) void attention_flash_generic_kernel(FlashArgs a) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t total = (int64_t)a.B * a.H * a.Q;
-  if (t >= total) return;
-  const int q = (int)(t % a.Q);
-  const int h = (int)((t / a.Q) % a.H);
-  const int64_t b = t / ((int64_t)a.Q * a.H);
-  const CT* base = reinterpret_cast<const CT*>(a.qkvg);
-  const int64_t ld4 = 4 * (int64_t)a.C;
-  const CT* qr = base + (b * a.Q + q) * ld4 + h * D;
-  float qv[D], acc[D];
+// f32 arithmetic at any head dimension up to 32: one wave per 32 queries of one
+// (b, h), keys in blocks of 32, on the f32 MFMA. S^T = K Q^T leaves a lane one
+// query's logits for 16 keys, 8 (v / 4) + 4 (lane / 32) + v % 4; step v of
+// O^T = V^T P^T takes exactly that key from each lane half (B = its
+// probability, A = V of the same key), so the probabilities never move between
+// lanes. The reference's terms and clamp (attention.ts:688-723): the S product
+// accumulates onto the key bias (0 for a live key), then the pair bias is
+// added. The running maximum is replaced by an offset that moves only when a
+// logit exceeds it by more than kF32Slack, which scales numerator and
+// denominator alike; the slack is small because a weight's relative error
+// grows with its exponent.
+//
+// Bound: the f32 MFMA. A block is DP / 2 + 16 instructions of 64 cycles a wave
+// (2,048 cycles at head dimension 32) against ~800 of vector work, so the
+// kernel needs nothing but loads that land in time: K, V and the biases come
+// straight from global memory in the MFMA's own layouts (whole 16-byte chunks
+// of a key's channels, 128-byte rows of V), each fetched one block ahead into
+// the registers its last use just freed. No LDS, no barrier, up to four waves
+// a SIMD. Four waves of a workgroup take consecutive query blocks, so K and V
+// reach a CU about once; workgroup ids give each XCD a contiguous range.
+// Measured, column attention over 508 sequences x 59 residues, 8 heads of 32
+// (15.6 GFLOP, 101 us at the f32 rate of a large product): 163 us; one thread
+// a query took 1,493 us.
+constexpr int kF32Waves = 4;
+constexpr float kF32Slack = 2.0f;
+constexpr float kDropped = -1e30f;    // the logit of a key past the end
+
+// DP: the head dimension padded to 8, 16 or 32 (channels past it are zero in
+// the products). VEC: head dimension a multiple of four, so a lane's channels
+// load in 16-byte chunks (f32). OFF: 32-bit byte offsets within a batch
+// entry's rows where those fit, 64-bit otherwise.
+template <typename CT, int DP, bool VEC, bool BIAS, typename OFF>
+__global__ __launch_bounds__(64 * kF32Waves) void attention_flash_f32_kernel(FlashArgs a, int qtiles, int64_t tiles,
+                                                                          int64_t per_xcd) {
+  static_assert(!VEC || sizeof(CT) == 4, "16-byte chunks of f32 channels");
+  constexpr int HD = DP / 2;  // channels a lane half takes: [HD hi, HD hi + HD)
+  const int lane = threadIdx.x & 63, col = lane & 31, hi = lane >> 5;
+  const int64_t group = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const int64_t t = group * kF32Waves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (t >= tiles) return;  // the whole wave
+  const int q0 = 32 * (int)(t % qtiles);
+  const int h = (int)(t / qtiles % a.H);
+  const int64_t b = t / qtiles / a.H;
+  const int Q = a.Q, d = a.d;
+  const OFF ldb = (OFF)(4 * sizeof(CT)) * (OFF)a.C;  // bytes between rows
+  const char* rows = reinterpret_cast<const char*>(a.qkvg) + b * Q * 4 * a.C * (int64_t)sizeof(CT) +
+                     (int64_t)h * d * sizeof(CT);
+  const char* keys = rows + (int64_t)a.C * sizeof(CT);
+  const char* vals = keys + (int64_t)a.C * sizeof(CT);
+
+  // A lane's HD channels of the row at `off`.
+  auto load_half = [&](const char* base, OFF off, float (&f)[HD]) {
+    const CT* p = reinterpret_cast<const CT*>(base + off);
+    if constexpr (VEC) {
 #pragma unroll
-  for (int e = 0; e < D; e++) {
-    qv[e] = (float)qr[e];
-    acc[e] = 0.0f;
+      for (int i = 0; i < HD / 4; i++) {
+        // a chunk past the head dimension lies in the row's next columns
+        const float4 w = *reinterpret_cast<const float4*>(p + HD * hi + 4 * i);
+        const bool in = HD * hi + 4 * i < d;
+        f[4 * i] = in ? w.x : 0.0f, f[4 * i + 1] = in ? w.y : 0.0f;
+        f[4 * i + 2] = in ? w.z : 0.0f, f[4 * i + 3] = in ? w.w : 0.0f;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < HD; e++) {
+        const float w = (float)p[min(HD * hi + e, d - 1)];
+        f[e] = HD * hi + e < d ? w : 0.0f;
+      }
+    }
+  };
+  const OFF last = (OFF)(Q - 1) * ldb;
+  auto load_keys = [&](int k0, float (&f)[HD]) {  // keys past the end repeat the last (their logits are dropped)
+    const OFF off = (OFF)(k0 + col) * ldb;
+    load_half(keys, off < last ? off : last, f);
+  };
+  // Channels past the head dimension repeat the last (those rows of O^T are not stored).
+  const OFF chan = (OFF)sizeof(CT) * (OFF)min(col, d - 1);
+  const OFF val0 = (OFF)(4 * hi) * ldb + chan, val_last = last + chan;
+  auto load_vals = [&](int k0, float (&f)[16]) {
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+      const OFF off = val0 + (OFF)(k0 + 8 * (v >> 2) + (v & 3)) * ldb;
+      f[v] = (float)*reinterpret_cast<const CT*>(vals + (off < val_last ? off : val_last));
+    }
+  };
+  // Biases of keys k0 + 8 g + 4 hi + [0, 4): rows are padded to whole float4s.
+  const int myq = q0 + col, qc = min(myq, Q - 1);
+  const float* kb_row = a.key_bias + b * a.stride;
+  const float* pb_row = BIAS ? a.bias + ((int64_t)h * Q + qc) * a.stride : nullptr;
+  auto load_bias = [&](const float* row, int k0, floatx16& f) {
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const float4 w = *reinterpret_cast<const float4*>(row + min(k0 + 8 * g + 4 * hi, a.stride - 4));
+      f[4 * g] = w.x, f[4 * g + 1] = w.y, f[4 * g + 2] = w.z, f[4 * g + 3] = w.w;
+    }
+  };
+
+  float qf[HD], kf[HD], vf[16];
+  floatx16 kb, pb;
+  load_keys(0, kf);
+  load_half(rows, (OFF)qc * ldb, qf);
+  load_bias(kb_row, 0, kb);
+  if constexpr (BIAS) load_bias(pb_row, 0, pb);
+  // The loop's order of loads: were V's issued before the biases here, the
+  // loop's wait for the biases would have to cover V's loads as well.
+  __builtin_amdgcn_sched_barrier(0);
+  load_vals(0, vf);
+  __builtin_amdgcn_sched_barrier(0);
+
+  floatx16 o = {};
+  float m = -1e30f, offset = 0.0f;
+  float sum = 0.0f;  // over this lane half's keys
+  for (int k0 = 0; k0 < Q; k0 += 32) {
+    floatx16 s = kb;
+#pragma unroll
+    for (int e = 0; e < HD; e++) s = mfma_f32(kf[e], qf[e], s);
+    load_keys(k0 + 32, kf);
+    float x[16];
+#pragma unroll
+    for (int v = 0; v < 16; v++) x[v] = __builtin_amdgcn_fmed3f(BIAS ? s[v] + pb[v] : s[v], -a.clamp, a.clamp);
+    load_bias(kb_row, k0 + 32, kb);
+    if constexpr (BIAS) load_bias(pb_row, k0 + 32, pb);
+    if (k0 + 32 > Q) {
+#pragma unroll
+      for (int v = 0; v < 16; v++)
+        if (k0 + 8 * (v >> 2) + 4 * hi + (v & 3) >= Q) x[v] = kDropped;
+    }
+    float mx = x[0];
+#pragma unroll
+    for (int v = 1; v < 16; v++) mx = fmaxf(mx, x[v]);
+    if (__builtin_amdgcn_ballot_w64(mx > m + kF32Slack)) {
+      const float to = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)));
+      const float f = __builtin_amdgcn_exp2f((m - to) * kLog2e);
+      sum *= f;
+#pragma unroll
+      for (int v = 0; v < 16; v++) o[v] *= f;
+      m = to;
+      offset = -to * kLog2e;
+    }
+    // e^(x - m) with one rounding of the exponent; the rounding of `offset`
+    // scales every weight of the row alike and drops out.
+#pragma unroll
+    for (int v = 0; v < 16; v++) x[v] = __builtin_amdgcn_exp2f(fmaf(x[v], kLog2e, offset));
+    sum += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])) +
+           (((x[8] + x[9]) + (x[10] + x[11])) + ((x[12] + x[13]) + (x[14] + x[15])));
+#pragma unroll
+    for (int v = 0; v < 16; v++) o = mfma_f32(vf[v], x[v], o);
+    load_vals(k0 + 32, vf);
   }
-  float run_max = -1e30f, run_sum = 0.0f;
-  for (int k = 0; k < a.Q; k++) {
-    const CT* kr = base + (b * a.Q + k) * ld4 + a.C + h * D;
-    float dot = 0.0f;
+  sum += __shfl_xor(sum, 32);
+  if (myq >= Q) return;
+  const CT* gr = reinterpret_cast<const CT*>(rows + (OFF)myq * ldb) + 3 * (int64_t)a.C;
+  const int64_t src = a.transpose ? (int64_t)myq * a.B + b : b * Q + myq;
+  CT* out = reinterpret_cast<CT*>(a.weighted) + src * a.C + h * d;
 #pragma unroll
-    for (int e = 0; e < D; e++) dot += qv[e] * (float)kr[e];
-    float logit = dot + a.key_bias[b * a.stride + k];
-    if (a.bias) logit += a.bias[((int64_t)h * a.Q + q) * a.stride + k];
-    logit = fminf(fmaxf(logit, -a.clamp), a.clamp);
-    const float new_max = fmaxf(run_max, logit);
-    const float scale = expf(run_max - new_max), weight = expf(logit - new_max);
-    run_sum = run_sum * scale + weight;
-    run_max = new_max;
-    const CT* vr = kr + a.C;
+  for (int g = 0; g < 4; g++) {
+    const int c = 8 * g + 4 * hi;
+    if constexpr (VEC) {
+      if (c >= d) break;
+      const float4 gv = *reinterpret_cast<const float4*>(gr + c);
+      *reinterpret_cast<float4*>(out + c) = make_float4(o[4 * g] / sum * gv.x, o[4 * g + 1] / sum * gv.y,
+                                                        o[4 * g + 2] / sum * gv.z, o[4 * g + 3] / sum * gv.w);
+    } else {
 #pragma unroll
-    for (int e = 0; e < D; e++) acc[e] = acc[e] * scale + weight * (float)vr[e];
+      for (int i = 0; i < 4; i++)
+        if (c + i < d) out[c + i] = (CT)(o[4 * g + i] / sum * (float)gr[c + i]);
+    }
   }
-  const CT* gr = qr + 3 * a.C;
-  const int64_t src = a.transpose ? (int64_t)q * a.B + b : b * a.Q + q;
-  CT* out = reinterpret_cast<CT*>(a.weighted) + src * a.C + h * D;
-#pragma unroll
-  for (int e = 0; e < D; e++) out[e] = (CT)(acc[e] / run_sum * (float)gr[e]);
 }
 
-template <typename CT, int... Ds>
-int launch_flash_generic(const FlashArgs& fa, hipStream_t st, std::integer_sequence<int, Ds...>) {
-  using Kernel = void (*)(FlashArgs);
-  static constexpr Kernel table[] = {attention_flash_generic_kernel<CT, Ds + 1>...};
-  const int64_t threads = (int64_t)fa.B * fa.H * fa.Q;
-  return launch("attention.flash", table[fa.d - 1], dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0, st, fa);
+template <typename CT, int DP, bool VEC, typename OFF = uint32_t>
+int launch_flash_f32_as(const FlashArgs& fa, hipStream_t st) {
+  const int qtiles = (int)ceil_div(fa.Q, 32);
+  const int64_t tiles = (int64_t)fa.B * fa.H * qtiles, per_xcd = ceil_div(tiles, 8 * kF32Waves);
+  AFHIP_REQUIRE(per_xcd < ((int64_t)1 << 28), "attention grid too large");
+  auto k = fa.bias ? attention_flash_f32_kernel<CT, DP, VEC, true, OFF>
+                   : attention_flash_f32_kernel<CT, DP, VEC, false, OFF>;
+  return launch("attention.flash", k, dim3((unsigned)(8 * per_xcd)), dim3(64 * kF32Waves), 0, st, fa, qtiles, tiles,
+                per_xcd);
+}
+
+template <typename CT> int launch_flash_f32(const FlashArgs& fa, hipStream_t st) {
+  // The fetch ahead reaches offset (Q + 63) rows before it is cut back to the last row.
+  if (((int64_t)fa.Q + 64) * 4 * fa.C * (int64_t)sizeof(CT) > (int64_t)UINT32_MAX)
+    return launch_flash_f32_as<CT, 32, false, uint64_t>(fa, st);
+  if constexpr (sizeof(CT) == 4) {
+    // Rows of 4 C floats from a 256-byte aligned workspace: heads of a
+    // multiple of four channels start on 16 bytes.
+    if (fa.d % 4 == 0) {
+      if (fa.d <= 8) return launch_flash_f32_as<CT, 8, true>(fa, st);
+      if (fa.d <= 16) return launch_flash_f32_as<CT, 16, true>(fa, st);
+      return launch_flash_f32_as<CT, 32, true>(fa, st);
+    }
+  }
+  return launch_flash_f32_as<CT, 32, false>(fa, st);
 }
 
 // f16 operands, head_dim 32: one wave per 32 queries of one (b, h), keys in
@@ -1298,8 +1442,7 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
                : launch("attention.flash", attention_flash_f16_kernel<false>, dim3((unsigned)groups),
                         dim3(kFlashThreads), 0, st, fa);
     } else {
-      s = f16 ? launch_flash_generic<half_t>(fa, st, std::make_integer_sequence<int, 32>{})
-              : launch_flash_generic<float>(fa, st, std::make_integer_sequence<int, 32>{});
+      s = f16 ? launch_flash_f32<half_t>(fa, st) : launch_flash_f32<float>(fa, st);
     }
     if (s) return s;
   }

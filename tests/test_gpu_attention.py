@@ -335,3 +335,22 @@ def test_f16_mfma_narrow_heads(dev, name, C, H):
     expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
     got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb, precision="f16", out_dtype="f16")
     assert np.abs(got - expect).max() <= 1e-2 * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("C,H,precision", [(64, 16, "f32"), (36, 3, "f32"), (40, 2, "f32"), (84, 3, "f32"), (64, 2, "f32"),
+                                           (10, 1, "f32"), (21, 3, "f16")])
+@pytest.mark.parametrize("name,S,L", [("msa_column", 33, 2), ("msa_column", 65, 3), ("triangle_end", 0, 32),
+                                      ("msa_row", 2, 31), ("msa_row", 3, 1)])
+def test_f32_mfma_flash_edges(dev, name, S, L, C, H, precision):
+    # The f32 flash kernel at the edges of its 32-query and 32-key blocks and
+    # of its channel paddings (head dimensions 4, 12, 20, 28, 32, 10; 7 in
+    # f16 storage). The query weights are scaled up so that logits
+    # spread over tens of units and the softmax offset moves in later
+    # blocks. f32: 16 roundings of logits below 128 (2^-18 each) move a weight
+    # by at most 6e-5, the rest is the 1e-5 of the other f32 tests; f16
+    # storage: the general f16 bound.
+    x, mask, B, Q, tr, w, pb = case(name, S, L, C, H, Cp=12)
+    w["queryWeight"] = w["queryWeight"] * 4
+    expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
+    got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb, precision=precision)
+    assert np.abs(got - expect).max() <= (7e-5 if precision == "f32" else 1e-2) * np.abs(expect).max()
