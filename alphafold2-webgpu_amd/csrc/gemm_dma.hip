@@ -86,7 +86,7 @@ constexpr int kEpiOpmFused = 1;
 
 template <int BM, int BN, int STAGES, int WM, int WN, bool PIPE, typename TC, int EPI = kEpiGeneric, int LW = 16,
           bool AK = false, bool AF = false, bool FP32 = false>
-__global__ __launch_bounds__(64 * WM * WN, WM * WN == 4 ? 2 : 1) void gemm_dma_kernel(gemm_detail::KernelArgs ka) {
+__global__ __launch_bounds__(64 * WM * WN, FP32 && STAGES == 2 ? 4 : WM * WN == 4 ? 2 : 1) void gemm_dma_kernel(gemm_detail::KernelArgs ka) {
   constexpr int WAVES = WM * WN;
   constexpr int kThreads = 64 * WAVES;
   constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -663,16 +663,20 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN == 4 ? 2 : 1) void gemm_dma_k
       return;
     }
   }
-  if ((g.flags & ~gemm_detail::kRowwiseEpilogue) == 0 && !g.c_column_major) {
-    // Row-wise epilogues (plain, scale, bias, ReLU, residual, the
-    // outer-product-mean output's bias / (eps + count)) straight from the
-    // accumulators: lane holds row m0 + wm + 32 i + lane % 32 and, per group
+  // The attention blocks lengthen the row-wise epilogue of every call; the
+  // four-stage f32 tiles, whose calls take 10 us, leave them out (launch_typed
+  // sends no such call there).
+  constexpr bool kAttention = !FP32 || STAGES == 2;
+  if (gemm_detail::rowwise_epilogue(g) && (kAttention || !(g.flags & AFHIP_EPILOGUE_ATTENTION))) {
+    // Row-wise epilogues (plain, scale, bias, attention blocks, ReLU,
+    // residual, the outer-product-mean output's bias / (eps + count)) straight
+    // from the accumulators: lane holds row m0 + wm + 32 i + lane % 32 and, per group
     // g4, columns n0 + wn + 32 j + 8 g4 + 4 (lane / 32) + [0, 4).
     auto aligned4 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & (4 * sizeof(TC) - 1)) == 0; };
     const bool vec4 = (g.ldc & 3) == 0 && (g.sc & 3) == 0 && aligned4(g.c) &&
                       (!(g.flags & AFHIP_EPILOGUE_RESIDUAL) || aligned4(g.residual));
     if (!(g.flags & EPILOGUE_OPM_OUTPUT) && vec4 && m0 + BM <= g.M && n0 + BN <= g.N) {
-      // A whole tile with scale, bias, ReLU and residual at most: no global
+      // A whole tile without a count to read: no global
       // read waits behind a store. The output may alias the residual (and,
       // as far as the compiler knows, the scale and bias), so it keeps such a
       // read after any earlier store; interleaved, that was one memory round
@@ -682,7 +686,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN == 4 ? 2 : 1) void gemm_dma_k
       // later writes. The arithmetic is epilogue_row4's, step for step.
 #pragma clang fp contract(off)
       typedef TC tc4 __attribute__((ext_vector_type(4)));
-      const uint32_t flags = g.flags;
+      const uint32_t flags = kAttention ? g.flags : g.flags & ~(uint32_t)AFHIP_EPILOGUE_ATTENTION;
       float* const bl = reinterpret_cast<float*>(smem);
       float* const sl = bl + BN;
       const TC* R = reinterpret_cast<const TC*>(g.residual) + (int64_t)bt * g.sc;
@@ -724,12 +728,14 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN == 4 ? 2 : 1) void gemm_dma_k
 #pragma unroll
           for (int g4 = 0; g4 < 4; g4++) {
             const int col = n0 + wn + 32 * j + 8 * g4 + 4 * (lane >> 5);
+            const int block = flags & AFHIP_EPILOGUE_ATTENTION ? gemm_detail::attention_block4(g, col) : 0;
             tc4 v;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
               float y = acc[i][j][4 * g4 + e];
               if (flags & AFHIP_EPILOGUE_SCALE) y *= sl[wn + 32 * j + 8 * g4 + 4 * (lane >> 5) + e];
               if (flags & AFHIP_EPILOGUE_BIAS) y += bl[wn + 32 * j + 8 * g4 + 4 * (lane >> 5) + e];
+              if (block) y = block == 1 ? y * g.q_scale : sigmoidf_(y);
               if (flags & AFHIP_EPILOGUE_RELU) y = fmaxf(y, 0.0f);
               if (flags & AFHIP_EPILOGUE_RESIDUAL) y += (float)res[j][g4][e];
               v[e] = (TC)y;
@@ -869,11 +875,20 @@ bool dma_wide(const GemmArgs& g) {
 template <typename TC>
 int launch_typed(const GemmArgs& g, const GemmTypes& t, int tm, int tn, const char* label, hipStream_t s) {
   // f32 arithmetic (dma_eligible: f32 operands in 16-byte rows) on 64 x 64
-  // tiles whatever the selection: four 16 KiB stages, three in flight, two
-  // workgroups a CU; the f32 MFMA's rate makes the small tile's operand
-  // traffic no limit.
-  if (t.precision == AFHIP_PRECISION_F32)
+  // tiles whatever the selection; the f32 MFMA's rate makes the small tile's
+  // operand traffic no limit. A tile's ramp-up and output drain overlap only
+  // other workgroups' MFMAs, so with more than two tiles a CU two 16 KiB
+  // stages and four workgroups a CU are best; with fewer, nothing would run
+  // beside them, and four stages bring up to 128 k at once. Measured on
+  // MI355X (four stages, two workgroups / three, three / two, four), us:
+  // 29972 x 256 x 1024 with attention blocks 179 / 162 / 148, 29972 x 1024 x
+  // 256 153 / 149 / 138, 4096 x 128 x 512 10.4 / 11.3 / 11.7.
+  if (t.precision == AFHIP_PRECISION_F32) {
+    const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    if (ceil_div(g.M, 64) * ceil_div(g.N, 64) * g.batch > 2 * cus || (g.flags & AFHIP_EPILOGUE_ATTENTION))
+      return launch_tile<64, 64, 2, 2, 2, false, TC, 16, false, false, true>(g, label, s);
     return launch_tile<64, 64, 4, 2, 2, false, TC, 16, false, false, true>(g, label, s);
+  }
   const bool a_f32 = t.a_dtype == AFHIP_F32;
   // An f32 A (dma_eligible: 16-byte rows) on 128 x 128 tiles whatever the
   // selection: three stages of 24 KiB keep two workgroups a CU, where

@@ -215,9 +215,22 @@ __device__ __forceinline__ void epilogue_store(const GemmArgs& g, int b, int row
 }
 
 // Epilogue flags that act on one output row elementwise (everything but
-// ATTENTION, whose column blocks differ, and OPM_CONTRACT, which scatters).
+// OPM_CONTRACT, which scatters). ATTENTION's column blocks differ, but a group
+// of four aligned columns lies in one block where head_cols is a multiple of
+// four (rowwise_epilogue).
 constexpr uint32_t kRowwiseEpilogue = AFHIP_EPILOGUE_SCALE | AFHIP_EPILOGUE_BIAS | AFHIP_EPILOGUE_RELU |
-                                      AFHIP_EPILOGUE_RESIDUAL | EPILOGUE_OPM_OUTPUT;
+                                      AFHIP_EPILOGUE_RESIDUAL | AFHIP_EPILOGUE_ATTENTION | EPILOGUE_OPM_OUTPUT;
+
+__device__ __forceinline__ bool rowwise_epilogue(const GemmArgs& g) {
+  return (g.flags & ~kRowwiseEpilogue) == 0 && !g.c_column_major &&
+         (!(g.flags & AFHIP_EPILOGUE_ATTENTION) || g.head_cols % 4 == 0);
+}
+
+// The attention block of a group of four columns from `col` (a multiple of
+// four): 1 for q (scaled), 2 for the gate (sigmoid), 0 for any other.
+__device__ __forceinline__ int attention_block4(const GemmArgs& g, int col) {
+  return col < g.head_cols ? 1 : col >= 3 * g.head_cols && col < 4 * g.head_cols ? 2 : 0;
+}
 
 // epilogue_store for `n` (<= 4) consecutive columns of one row, the same
 // steps in the same order with the same roundings, written with one vector
@@ -229,12 +242,14 @@ __device__ __forceinline__ void epilogue_row4(const GemmArgs& g, int b, int row,
   const uint32_t flags = g.flags;
   float denom = 0.0f;
   if (flags & EPILOGUE_OPM_OUTPUT) denom = g.opm_eps + g.opm_count[(int64_t)g.opm_row0 + row];
+  const int block = flags & AFHIP_EPILOGUE_ATTENTION ? attention_block4(g, col) : 0;
 #pragma unroll
   for (int e = 0; e < 4; e++) {
     if (e >= n) break;
     if (flags & AFHIP_EPILOGUE_SCALE) y[e] *= g.scale[col + e];
     if (flags & AFHIP_EPILOGUE_BIAS) y[e] += g.bias[col + e];
     if (flags & EPILOGUE_OPM_OUTPUT) y[e] += g.bias[col + e] / denom;
+    if (block) y[e] = block == 1 ? y[e] * g.q_scale : sigmoidf_(y[e]);
     if (flags & AFHIP_EPILOGUE_RELU) y[e] = fmaxf(y[e], 0.0f);
   }
   const int64_t at = (int64_t)b * g.sc + (int64_t)row * g.ldc + col;

@@ -461,3 +461,33 @@ def test_invalid_plan_raises_range_error(dev):
         gemm.TiledGemm(0, 4, 4)
     with pytest.raises(_lib.RangeError):
         gemm.TiledGemm(4, 4, 4, precision="f32", w_dtype="i8")
+
+
+@pytest.mark.parametrize("precision,out_dtype,heads,head_dim,rows", [
+    ("f32", "f32", 8, 32, 300), ("f32", "f32", 2, 8, 77), ("f32", "f32", 1, 6, 129),
+    ("f16", "f16", 8, 8, 1000), ("f16", "f32", 3, 4, 259), ("f16", "f16", 1, 7, 130)])
+def test_lds_dma_attention_blocks_match_register_kernel_bitwise(dev, precision, out_dtype, heads, head_dim, rows):
+    # The ATTENTION blocks in the row-wise epilogue: whole and ragged tiles,
+    # block edges inside a tile, and head columns that are no multiple of four
+    # (the element-wise epilogue). The same steps and roundings as the
+    # register-staged kernel, so the same bits.
+    from afhip import gemm
+
+    K, N = 64, 4 * heads * head_dim
+    a, w = ref.normal(71, (rows, K)), ref.normal(72, (N, K), 1 / K)
+    b = ref.normal(73, (N,), 0.1)
+    ad, wd, bd = to_dev(a, dev), to_dev(w, dev), to_dev(b, dev)
+    if precision == "f16":
+        ad, wd = ad.half(), wd.half()
+    got = {}
+    for kernel in ("register", "lds_dma"):
+        gemm.force_variant(gemm.GemmVariant(precision, 128, 128, source="pinned", kernel=kernel))
+        try:
+            plan = gemm.TiledGemm(rows, K, N, precision=precision, a_dtype=precision, w_dtype=precision, w_layout="k",
+                                  out_dtype=out_dtype, epilogue=("bias", "attention"), heads=heads, head_dim=head_dim)
+            assert plan.variant().kernel == kernel
+            got[kernel] = plan.run(ad, wd, bias=bd).float().cpu().numpy()
+        finally:
+            gemm.force_variant(None)
+    assert np.isfinite(got["register"]).all()
+    assert np.array_equal(got["register"], got["lds_dma"])
