@@ -45,6 +45,54 @@ struct GemmArgs {
 constexpr uint32_t EPILOGUE_OPM_CONTRACT = 1u << 16;
 constexpr uint32_t EPILOGUE_OPM_OUTPUT = 1u << 17;
 
+// f32 matrices as pairs of f16 (the pair GEMM, gemm_dma.hip): x = h + l with
+// h = f16(x), l = f16(x - h), 22 to 24 bits of x wherever |x| <= 65504 and x is
+// not tiny beside 2^-14, which the callers see to with power-of-two scales. A
+// row keeps each 16 consecutive k as 16 h, then 16 l (64 bytes); a matrix takes
+// the bytes it takes in f32. K is a multiple of 16.
+__host__ __device__ inline int64_t pair_index(int64_t k) { return 32 * (k >> 4) + (k & 15); }  // of h; l is 16 on
+// The empty asm keeps x a rounded f32: contracted into the conversion
+// (v_fma_mixlo_f16), the operation that made x would round h from its exact
+// result in one place and from x in another, and l would belong to another h.
+__device__ __forceinline__ void pair_split(float x, half_t& h, half_t& l) {
+  asm("" : "+v"(x));
+  h = (half_t)x;
+  l = (half_t)(x - (float)h);
+}
+__device__ __forceinline__ void pair_store(half_t* row, int64_t k, float x) {
+  half_t h, l;
+  pair_split(x, h, l);
+  row[pair_index(k)] = h;
+  row[pair_index(k) + 16] = l;
+}
+// The power of two (its exponent) that takes values of magnitude up to `most`
+// into (-2^15, 2^15), the largest past 2^14; 0 where there are none or they are
+// not finite. Bounded so that the exponents a result adds up stay in f32.
+__device__ __forceinline__ int pair_exponent(float most) {
+  if (!(most > 0.0f) || !isfinite(most)) return 0;
+  int p;
+  frexpf(most, &p);  // most = m 2^p, m in [1/2, 1)
+  return min(max(15 - p, -110), 110);
+}
+// A LayerNorm's output before its affine: C values of magnitude at most
+// sqrt(C), stored times 2^pair_norm_exponent(C), at most 2^15.
+inline int pair_norm_exponent(int C) {
+  int root = 0;
+  while ((int64_t)1 << (2 * root) < C) root++;  // sqrt(C) <= 2^root
+  return 15 - root;
+}
+// The output as pairs (rows of ldc elements, 2 ldc halves) instead of TC.
+constexpr uint32_t EPILOGUE_PAIRS = 1u << 18;
+
+// C = epilogue(sum_k (A_h B_h + A_h B_l + A_l B_h)) over pair rows: A [M], B [N]
+// rows of K elements, f32 accumulation, epilogue SCALE, BIAS, ATTENTION (the
+// gate's sigmoid; q as it is), RELU and RESIDUAL (f32 or f16 outputs only) in
+// that order. N, ldc and head_cols multiples of 16, operands on 4 bytes (16 for
+// the wide loads), no batch. Against 64 bits its error is no larger than the f32 MFMA's from
+// K = 64 on: the dropped l l term is 2^-24 of a product, a third as many f32
+// roundings accumulate.
+int run_gemm_pairs(const GemmArgs& args, int c_dtype, const char* label, hipStream_t stream);
+
 struct GemmTypes {
   int precision;  // AFHIP_PRECISION_*
   int a_dtype;    // AFHIP_F32 | AFHIP_F16

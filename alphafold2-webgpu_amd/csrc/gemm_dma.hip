@@ -10,6 +10,11 @@
 // dispatches it once per channel along z, src/triangle/shaders.ts:452-496),
 // the outer-product-mean contraction and the f16 projections.
 //
+// PAIRS: f32 operands held as pairs of f16 (gemm.h), three products on the f16
+// MFMA: 96 cycles for 32 x 32 x 16 against 512 of the f32 MFMA. Bound by the
+// LDS reads beside the MFMAs (8 KiB a wave for 384 cycles of MFMA) and, with
+// pairs or f32 out, the output's bytes.
+//
 // Design:
 //  - One workgroup of WM x WN wave64s owns a BM x BN output tile (each wave
 //    (BM/WM) x (BN/WN) in 32 x 32 v_mfma_f32_32x32x16_f16 tiles) and walks
@@ -85,8 +90,8 @@ constexpr int kEpiGeneric = 0;
 constexpr int kEpiOpmFused = 1;
 
 template <int BM, int BN, int STAGES, int WM, int WN, bool PIPE, typename TC, int EPI = kEpiGeneric, int LW = 16,
-          bool AK = false, bool AF = false, bool FP32 = false>
-__global__ __launch_bounds__(64 * WM * WN, FP32 && STAGES == 2 ? 4 : WM * WN == 4 ? 2 : 1) void gemm_dma_kernel(gemm_detail::KernelArgs ka) {
+          bool AK = false, bool AF = false, bool FP32 = false, bool PAIRS = false>
+__global__ __launch_bounds__(64 * WM * WN, FP32 && STAGES == 2 ? 4 : PAIRS && STAGES == 3 ? 3 : WM * WN == 4 ? 2 : 1) void gemm_dma_kernel(gemm_detail::KernelArgs ka) {
   constexpr int WAVES = WM * WN;
   constexpr int kThreads = 64 * WAVES;
   constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -379,13 +384,137 @@ __global__ __launch_bounds__(64 * WM * WN, FP32 && STAGES == 2 ? 4 : WM * WN == 
     block_barrier<false>();  // this loop writes no LDS itself
     if (ks + STAGES - 1 < nk) issue(ks + STAGES - 1, (ks + STAGES - 1) % STAGES);
     const unsigned char* st = smem + (ks % STAGES) * STAGE_BYTES;
+    if constexpr (PAIRS) {
+      // The stage row's two halves are 16 k's h and the same k's l.
+      Frag ah[TM], bh[TN], al[TM], bl[TN];
+      read_frags(st, 0, ah, bh);
+      read_frags(st, 1, al, bl);
+      mfmas(ah, bh);
+      mfmas(ah, bl);
+      mfmas(al, bh);
+    } else {
 #pragma unroll
-    for (int kk = 0; kk < 2; kk++) {
-      Frag af[TM], bf[TN];
-      read_frags(st, kk, af, bf);
-      mfmas(af, bf);
+      for (int kk = 0; kk < 2; kk++) {
+        Frag af[TM], bf[TN];
+        read_frags(st, kk, af, bf);
+        mfmas(af, bf);
+      }
     }
     asm volatile("" ::: "memory");
+  }
+
+  if constexpr (PAIRS) {
+    // Scale, bias, the gate, ReLU, then f32 or pairs through a square of LDS of
+    // the wave's own, 32 rows at a time, so that every store instruction
+    // writes whole rows of the wave's columns (four 256-byte pieces) instead of
+    // 32-byte ones: lane holds row m0 + wm + 32 i + lane % 32 and, per group
+    // g4, columns wn + 32 j + 8 g4 + 4 (lane / 32) + [0, 4). A row of the
+    // square keeps 16-byte chunk c (of 4 columns, or of 8 h or l) at slot
+    // c ^ (row % CPR). The residual joins where the rows leave; its reads are
+    // all issued before the first store.
+    const uint32_t flags = g.flags;
+    constexpr int ROWB = 4 * WTN, CPR = ROWB / 16, RPI = 64 / CPR, IT = 32 / RPI;  // rows a store instruction covers
+    static_assert(CPR <= 64 && 64 % CPR == 0 && CPR % 8 == 0, "whole rows a store instruction");
+    static_assert(2 * BN * 4 + WAVES * 32 * ROWB <= STAGES * STAGE_BYTES, "the squares fit the stage memory");
+    float* const bias = reinterpret_cast<float*>(smem);
+    float* const scale = bias + BN;
+    block_barrier<false>();  // every wave is done reading the stages
+    for (int c = threadIdx.x; c < BN; c += kThreads) {
+      const bool in = n0 + c < g.N;
+      bias[c] = in && (flags & AFHIP_EPILOGUE_BIAS) ? g.bias[n0 + c] : 0.0f;
+      scale[c] = in && (flags & AFHIP_EPILOGUE_SCALE) ? g.scale[n0 + c] : 1.0f;
+    }
+    block_barrier();
+    unsigned char* const sq = smem + 2 * BN * 4 + wave * 32 * ROWB;
+    const bool pairs_out = (flags & EPILOGUE_PAIRS) != 0, residual = (flags & AFHIP_EPILOGUE_RESIDUAL) != 0;
+    typedef TC tc4 __attribute__((ext_vector_type(4)));
+    const bool vec4 = (reinterpret_cast<uintptr_t>(g.c) & (4 * sizeof(TC) - 1)) == 0;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      const int r = lane & 31;
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; g4++) {
+          const int c = 32 * j + 8 * g4 + 4 * (lane >> 5);
+          const bool gate = (flags & AFHIP_EPILOGUE_ATTENTION) && gemm_detail::attention_block4(g, n0 + wn + c) == 2;
+          floatx4 y;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            y[e] = fmaf(acc[i][j][4 * g4 + e], scale[wn + c + e], bias[wn + c + e]);
+            if (gate) y[e] = sigmoidf_(y[e]);
+            if (flags & AFHIP_EPILOGUE_RELU) y[e] = fmaxf(y[e], 0.0f);
+          }
+          if (pairs_out) {
+            half4 h, l;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              half_t he, le;
+              pair_split(y[e], he, le);
+              h[e] = he, l[e] = le;
+            }
+            const int chunk = (int)pair_index(c) >> 3;
+            unsigned char* p = sq + r * ROWB + 8 * (lane >> 5);
+            *reinterpret_cast<half4*>(p + 16 * (chunk ^ (r % CPR))) = h;
+            *reinterpret_cast<half4*>(p + 16 * ((chunk + 2) ^ (r % CPR))) = l;
+          } else {
+            *reinterpret_cast<floatx4*>(sq + r * ROWB + 16 * ((c >> 2) ^ (r % CPR))) = y;
+          }
+        }
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the square is written
+      __builtin_amdgcn_wave_barrier();
+      const int c = lane % CPR, col = n0 + wn + 4 * c;
+      auto row_of = [&](int t) { return RPI * t + lane / CPR; };
+      const int row0 = m0 + wm + 32 * i;
+      if (pairs_out) {
+#pragma unroll
+        for (int t = 0; t < IT; t++) {
+          const int rr = row_of(t);
+          u32x4 v = *reinterpret_cast<const u32x4*>(sq + rr * ROWB + 16 * (c ^ (rr % CPR)));
+          // 4 ldc bytes a row, 64 a block of 16 columns: chunk c is 16 bytes at 4 col
+          if (row0 + rr < g.M && col < g.N)
+            *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(g.c) + ((int64_t)(row0 + rr) * g.ldc + col) * 4) = v;
+          stores_read(v);
+        }
+      } else {
+        float old[IT][4] = {};
+        if (residual) {
+#pragma unroll
+          for (int t = 0; t < IT; t++)
+            if (row0 + row_of(t) < g.M && col < g.N) {
+              const TC* p = reinterpret_cast<const TC*>(g.residual) + (int64_t)(row0 + row_of(t)) * g.ldc + col;
+              if (vec4) {
+                const tc4 o = *reinterpret_cast<const tc4*>(p);
+#pragma unroll
+                for (int e = 0; e < 4; e++) old[t][e] = (float)o[e];
+              } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) old[t][e] = (float)p[e];
+              }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < IT; t++) {
+          const int rr = row_of(t);
+          const floatx4 y = *reinterpret_cast<const floatx4*>(sq + rr * ROWB + 16 * (c ^ (rr % CPR)));
+          if (row0 + rr < g.M && col < g.N) {
+            TC* p = reinterpret_cast<TC*>(g.c) + (int64_t)(row0 + rr) * g.ldc + col;
+            tc4 v;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = (TC)(residual ? y[e] + old[t][e] : y[e]);
+            if (vec4) {
+              *reinterpret_cast<tc4*>(p) = v;
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; e++) p[e] = v[e];
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // the square is read before the next rows overwrite it
+      __builtin_amdgcn_wave_barrier();
+    }
+    return;
   }
 
   if constexpr (EPI == kEpiOpmFused) {
@@ -828,7 +957,7 @@ __global__ __launch_bounds__(64 * WM * WN, FP32 && STAGES == 2 ? 4 : WM * WN == 
 }
 
 template <int BM, int BN, int STAGES, int WM, int WN, bool PIPE, typename TC, int LW = 16, bool AK = false,
-          bool AF = false, bool FP32 = false>
+          bool AF = false, bool FP32 = false, bool PAIRS = false>
 int launch_tile(const GemmArgs& g, const char* label, hipStream_t s) {
   gemm_detail::KernelArgs ka;
   ka.g = g;
@@ -839,7 +968,7 @@ int launch_tile(const GemmArgs& g, const char* label, hipStream_t s) {
   ka.total_tiles = (int)total;
   ka.per_xcd = (int)ceil_div(total, 8);
   const size_t shared = (size_t)STAGES * dma_stage_bytes(BM, BN, AF || FP32, FP32);
-  auto kernel = gemm_dma_kernel<BM, BN, STAGES, WM, WN, PIPE, TC, kEpiGeneric, LW, AK, AF, FP32>;
+  auto kernel = gemm_dma_kernel<BM, BN, STAGES, WM, WN, PIPE, TC, kEpiGeneric, LW, AK, AF, FP32, PAIRS>;
   if (int st = allow_lds((const void*)kernel, shared)) return st;
   return launch(label, kernel, dim3((unsigned)(ka.per_xcd * 8)), dim3(64 * WM * WN), shared, s, ka);
 }
@@ -998,6 +1127,38 @@ int run_opm_fused(const GemmArgs& g, int c_dtype, const char* label, hipStream_t
     return set_error(AFHIP_ERR_INVALID_ARGUMENT, "fused outer-product-mean launch outside its shape");
   if (c_dtype == AFHIP_F16) return launch_opm_fused_tile<half_t>(g, label, s);
   return launch_opm_fused_tile<float>(g, label, s);
+}
+
+namespace {
+template <typename TC> int launch_pairs(const GemmArgs& g, const char* label, hipStream_t s) {
+  // 128 x 128 tiles, three stages and three workgroups a CU. Measured on
+  // MI355X (29972 x 256 x 1024 pairs out / 29972 x 1024 x 256 f32 out), us:
+  // 69 / 60; four stages and two workgroups 76 / 61; 256 x 128 over eight
+  // waves 83 / 58; 256 x 256 87 / 81 (both 32-byte stores); the f32 MFMA
+  // 144 / 138.
+  auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  if (!al16(g.a) || !al16(g.b))  // 4-byte loads, as for f16 rows off 16 bytes
+    return launch_tile<128, 128, 5, 2, 2, false, TC, 4, false, false, false, true>(g, label, s);
+  return launch_tile<128, 128, 3, 2, 2, false, TC, 16, false, false, false, true>(g, label, s);
+}
+}  // namespace
+
+int run_gemm_pairs(const GemmArgs& args, int c_dtype, const char* label, hipStream_t s) {
+  auto al4 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0; };
+  const uint32_t allowed = AFHIP_EPILOGUE_SCALE | AFHIP_EPILOGUE_BIAS | AFHIP_EPILOGUE_ATTENTION | AFHIP_EPILOGUE_RELU |
+                           AFHIP_EPILOGUE_RESIDUAL | EPILOGUE_PAIRS;
+  const bool pairs_out = args.flags & EPILOGUE_PAIRS;
+  if (args.M <= 0 || args.N <= 0 || args.K <= 0 || args.K % 16 || args.N % 16 || args.ldc % 16 || args.ldc < args.N ||
+      args.batch != 1 || !al4(args.a) || !al4(args.b) || (args.flags & ~allowed) || args.c_column_major ||
+      (pairs_out && (!al4(args.c) || (args.flags & AFHIP_EPILOGUE_RESIDUAL))) ||
+      ((args.flags & AFHIP_EPILOGUE_ATTENTION) && args.head_cols % 16) ||
+      (int64_t)256 * args.K * 4 >= (int64_t)kOutOfRange)
+    return set_error(AFHIP_ERR_INVALID_ARGUMENT, "pair GEMM outside its shape");
+  GemmArgs g = args;
+  g.K = 2 * args.K;  // in halves
+  g.lda = g.ldb = g.K;
+  if (c_dtype == AFHIP_F16) return launch_pairs<half_t>(g, label, s);
+  return launch_pairs<float>(g, label, s);
 }
 
 int run_gemm_dma(const GemmArgs& g, const GemmTypes& t, int tm, int tn, const char* label, hipStream_t s) {

@@ -20,7 +20,14 @@ namespace {
 
 struct TransitionWeights {
   size_t scale, offset, w1, b1, w2, b2, msa, total;
+  size_t s1, s2, shift;  // the pair path's output scales and hidden exponents
 };
+
+// The pair path (f32 precision): whole 16-channel blocks both ways.
+bool pair_shape(const afhip_transition_desc& d) {
+  return d.precision == AFHIP_PRECISION_F32 && d.channels % 16 == 0 && d.hidden % 16 == 0 && d.channels <= (1 << 16) &&
+         d.hidden <= (1 << 20);
+}
 
 TransitionWeights layout(const afhip_transition_desc& d) {
   TransitionWeights w{};
@@ -37,6 +44,11 @@ TransitionWeights layout(const afhip_transition_desc& d) {
   w.b1 = take(4 * (size_t)d.hidden);
   w.w2 = take(es * (size_t)d.channels * d.hidden);  // [C][H]
   w.b2 = take(4 * (size_t)d.channels);
+  if (pair_shape(d)) {
+    w.s1 = take(4 * (size_t)d.hidden);
+    w.s2 = take(4 * (size_t)d.channels);
+    w.shift = take(4 * (size_t)d.hidden);
+  }
   w.msa = transition_msa_shape(d) ? take(transition_msa_weight_bytes()) : 0;
   w.total = at;
   return w;
@@ -115,6 +127,182 @@ __global__ void transition_prepare_kernel(const float* __restrict__ packed, int 
       else b2[j - 2 * C - H] = gb[j - 2 * C - H];
     }
   }
+}
+
+// Weights of the pair path, one workgroup a row of W1 [H][C], then of W2 [C][H].
+// With x_hat = (x - mean) rstd, |x_hat|_2 <= sqrt(C) for any row:
+//   W1'[h] = W1[h] diag(gamma) in double, scaled by 2^e to fill f16 (largest
+//   element in [2^14, 2^15)); x_hat is stored times 2^x_shift(C) <= 2^15;
+//   b1' = b1 + W1 beta; the hidden unit h stays below
+//   B = sqrt(C) |W1'[h]|_2 + |b1'|, so its pairs hold it times 2^-u, B 2^-u in
+//   (2^14, 2^15]; W2's column h takes 2^u back.
+// The first linear's scale and bias carry 2^-u (it commutes with the ReLU).
+__global__ __launch_bounds__(256) void pair_first_kernel(const float* __restrict__ packed, int C, int H, int x_exp,
+                                                         half_t* __restrict__ w1, float* __restrict__ s1,
+                                                         float* __restrict__ b1, int* __restrict__ shift) {
+  const float* gamma = packed;
+  const float* beta = gamma + C;
+  const float* f = beta + C;  // [C][H]
+  const int h = blockIdx.x;
+  float most = 0.0f;
+  double squares = 0.0, offset = 0.0;
+  for (int c = threadIdx.x; c < C; c += 256) {
+    const double w = f[(size_t)c * H + h], g = w * gamma[c];
+    most = fmaxf(most, fabsf((float)g));
+    squares += g * g;
+    offset += w * beta[c];
+  }
+  __shared__ float m_part[4];
+  __shared__ double s_part[4], o_part[4];
+  for (int o = 32; o > 0; o >>= 1) {
+    most = fmaxf(most, __shfl_xor(most, o));
+    squares += __shfl_xor(squares, o);
+    offset += __shfl_xor(offset, o);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    m_part[threadIdx.x >> 6] = most;
+    s_part[threadIdx.x >> 6] = squares;
+    o_part[threadIdx.x >> 6] = offset;
+  }
+  __syncthreads();
+  most = fmaxf(fmaxf(m_part[0], m_part[1]), fmaxf(m_part[2], m_part[3]));
+  squares = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+  const double bias = f[(size_t)C * H + h] + ((o_part[0] + o_part[1]) + (o_part[2] + o_part[3]));
+  const int e = pair_exponent(most);
+  const int u = -pair_exponent((float)(sqrt((double)C * squares) + fabs(bias)));
+  for (int c = threadIdx.x; c < C; c += 256)
+    pair_store(w1 + (int64_t)h * 2 * C, c, (float)ldexp((double)f[(size_t)c * H + h] * gamma[c], e));
+  if (threadIdx.x == 0) {
+    s1[h] = ldexpf(1.0f, -(x_exp + e + u));
+    b1[h] = (float)ldexp(bias, -u);
+    shift[h] = u;
+  }
+}
+
+__global__ __launch_bounds__(256) void pair_second_kernel(const float* __restrict__ packed, int C, int H,
+                                                          const int* __restrict__ shift, half_t* __restrict__ w2,
+                                                          float* __restrict__ s2, float* __restrict__ b2) {
+  const float* g = packed + 2 * (size_t)C + (size_t)C * H + H;  // [H][C]
+  const int c = blockIdx.x;
+  float most = 0.0f;
+  for (int h = threadIdx.x; h < H; h += 256) most = fmaxf(most, fabsf(ldexpf(g[(size_t)h * C + c], shift[h])));
+  __shared__ float part[4];
+  for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = most;
+  __syncthreads();
+  const int e = pair_exponent(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
+  for (int h = threadIdx.x; h < H; h += 256)
+    pair_store(w2 + (int64_t)c * 2 * H, h, ldexpf(g[(size_t)h * C + c], shift[h] + e));
+  if (threadIdx.x == 0) {
+    s2[c] = ldexpf(1.0f, -e);
+    b2[c] = g[(size_t)H * C + c];
+  }
+}
+
+// The LayerNorm without its affine, rows written as pairs of x_hat 2^x_exp;
+// the statistics of layer_norm_kernel. C = 8 LANES channels with 16-byte
+// accesses (aligned rows), four rows in flight a lane.
+template <typename IT, int LANES>
+__global__ __launch_bounds__(256) void pair_norm_rows_kernel(const IT* __restrict__ x, int64_t rows, float eps,
+                                                             float x_scale, half_t* __restrict__ y) {
+  constexpr int C = 8 * LANES, RPW = 64 / LANES;
+  constexpr int U = 4, LOADS = sizeof(IT) / 2;
+  const int lane = threadIdx.x & 63, sub = lane / LANES, part = lane % LANES;
+  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int64_t waves = ((int64_t)gridDim.x * blockDim.x) >> 6;
+  for (int64_t base = wave * RPW * U; base < rows; base += waves * RPW * U) {
+    u32x4 raw[U][LOADS];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int64_t row = base + u * RPW + sub;
+#pragma unroll
+      for (int l = 0; l < LOADS; l++)
+        raw[u][l] = row < rows ? reinterpret_cast<const u32x4*>(x + row * C + 8 * part)[l] : u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      float v[8];
+      if constexpr (sizeof(IT) == 2) {
+        const half8 h = __builtin_bit_cast(half8, raw[u][0]);
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = (float)h[e];
+      } else {
+#pragma unroll
+        for (int l = 0; l < 2; l++) {
+          const floatx4 f = __builtin_bit_cast(floatx4, raw[u][l]);
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[4 * l + e] = f[e];
+        }
+      }
+      float s = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; e++) s += v[e];
+      const float mean = lane_sum<LANES>(s) / (float)C;
+      float d2 = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        v[e] -= mean;
+        d2 += v[e] * v[e];
+      }
+      const float rstd = fast_rsqrt(lane_sum<LANES>(d2) / (float)C + eps) * x_scale;
+      half8 h, l;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        half_t he, le;
+        pair_split(v[e] * rstd, he, le);
+        h[e] = he, l[e] = le;
+      }
+      u32x4 hb = __builtin_bit_cast(u32x4, h), lb = __builtin_bit_cast(u32x4, l);
+      const int64_t row = base + u * RPW + sub;
+      if (row < rows) {
+        half_t* p = y + row * 2 * C + pair_index(8 * part);
+        *reinterpret_cast<u32x4*>(p) = hb;
+        *reinterpret_cast<u32x4*>(p + 16) = lb;
+      }
+      stores_read(hb, lb);
+    }
+  }
+}
+
+// The same for any width and alignment, one wave64 a row.
+template <typename IT>
+__global__ __launch_bounds__(256) void pair_norm_kernel(const IT* __restrict__ x, int64_t rows, int C, float eps,
+                                                        float x_scale, half_t* __restrict__ y) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const IT* xr = x + row * C;
+  float s = 0.0f;
+  for (int c = lane; c < C; c += 64) s += (float)xr[c];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  const float mean = s / (float)C;
+  float v = 0.0f;
+  for (int c = lane; c < C; c += 64) {
+    float d = (float)xr[c] - mean;
+    v += d * d;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  const float rstd = fast_rsqrt(v / (float)C + eps) * x_scale;
+  for (int c = lane; c < C; c += 64) pair_store(y + row * 2 * C, c, ((float)xr[c] - mean) * rstd);
+}
+
+template <typename IT>
+int launch_pair_norm(const void* x, int64_t rows, int C, float eps, void* y, hipStream_t st) {
+  const float x_scale = ldexpf(1.0f, pair_norm_exponent(C));
+  const IT* xi = (const IT*)x;
+  half_t* yo = (half_t*)y;
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const unsigned grid = (unsigned)std::min<int64_t>(ceil_div(rows, 4 * (64 / std::max(1, C / 8)) * 4), (int64_t)cus * 8);
+  const char* label = "transition.layer_norm";
+  if ((reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
+    if (C == 64) return launch(label, pair_norm_rows_kernel<IT, 8>, dim3(grid), dim3(256), 0, st, xi, rows, eps, x_scale, yo);
+    if (C == 128) return launch(label, pair_norm_rows_kernel<IT, 16>, dim3(grid), dim3(256), 0, st, xi, rows, eps, x_scale, yo);
+    if (C == 256) return launch(label, pair_norm_rows_kernel<IT, 32>, dim3(grid), dim3(256), 0, st, xi, rows, eps, x_scale, yo);
+  }
+  return launch(label, pair_norm_kernel<IT>, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, st, xi, rows, C, eps,
+                x_scale, yo);
 }
 
 int validate(const afhip_transition_desc* d) {
@@ -260,6 +448,14 @@ int afhip_transition_prepare_weights(const afhip_transition_desc* desc, const fl
     if (transition_msa_shape(d)) return prepare_transition_msa(packed, b + w.msa, st);
     return AFHIP_OK;
   }
+  if (pair_shape(d)) {
+    if (int s = launch("transition.prepare", pair_first_kernel, dim3(d.hidden), dim3(256), 0, st, packed, d.channels,
+                       d.hidden, pair_norm_exponent(d.channels), (half_t*)(b + w.w1), (float*)(b + w.s1),
+                       (float*)(b + w.b1), (int*)(b + w.shift)))
+      return s;
+    return launch("transition.prepare", pair_second_kernel, dim3(d.channels), dim3(256), 0, st, packed, d.channels,
+                  d.hidden, (const int*)(b + w.shift), (half_t*)(b + w.w2), (float*)(b + w.s2), (float*)(b + w.b2));
+  }
   return launch("transition.prepare", transition_prepare_kernel<float>, dim3(1024), dim3(256), 0, st, packed,
                 d.channels, d.hidden, (float*)(b + w.scale), (float*)(b + w.offset), (float*)(b + w.w1),
                 (float*)(b + w.b1), (float*)(b + w.w2), (float*)(b + w.b2));
@@ -317,6 +513,37 @@ int afhip_transition_run(const afhip_transition_desc* desc, const void* activati
     const float* sc = (const float*)(wb + w.scale);
     const float* of = (const float*)(wb + w.offset);
     int s;
+    if (pair_shape(d)) {
+      s = d.in_dtype == AFHIP_F32 ? launch_pair_norm<float>(x, rows, d.channels, d.epsilon, normalized, st)
+                                  : launch_pair_norm<half_t>(x, rows, d.channels, d.epsilon, normalized, st);
+      if (s) return s;
+      GemmArgs g1;
+      g1.a = normalized;
+      g1.b = wb + w.w1;
+      g1.c = hidden;
+      g1.scale = (const float*)(wb + w.s1);
+      g1.bias = (const float*)(wb + w.b1);
+      g1.M = (int)rows;
+      g1.N = d.hidden;
+      g1.K = d.channels;
+      g1.ldc = d.hidden;
+      g1.flags = AFHIP_EPILOGUE_SCALE | AFHIP_EPILOGUE_BIAS | AFHIP_EPILOGUE_RELU | EPILOGUE_PAIRS;
+      if ((s = run_gemm_pairs(g1, AFHIP_F32, "transition.first", st))) return s;
+      GemmArgs g2;
+      g2.a = hidden;
+      g2.b = wb + w.w2;
+      g2.c = (char*)out + oe * (size_t)r0 * d.channels;
+      g2.residual = g2.c;
+      g2.scale = (const float*)(wb + w.s2);
+      g2.bias = (const float*)(wb + w.b2);
+      g2.M = (int)rows;
+      g2.N = d.channels;
+      g2.K = d.hidden;
+      g2.ldc = d.channels;
+      g2.flags = AFHIP_EPILOGUE_SCALE | AFHIP_EPILOGUE_BIAS | (d.residual ? AFHIP_EPILOGUE_RESIDUAL : 0u);
+      if ((s = run_gemm_pairs(g2, d.out_dtype, "transition.second", st))) return s;
+      continue;
+    }
     if (d.in_dtype == AFHIP_F32)
       s = f16 ? launch_ln<float, half_t>(x, rows, d.channels, sc, of, d.epsilon, normalized, st)
               : launch_ln<float, float>(x, rows, d.channels, sc, of, d.epsilon, normalized, st);

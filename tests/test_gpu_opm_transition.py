@@ -339,3 +339,48 @@ def test_invalid_opm_and_transition_raise(dev):
     inp["rows"] = 0
     with pytest.raises(_lib.RangeError):
         transition.TransitionGpu().run(inp)
+
+
+@pytest.mark.parametrize("rows,c,h,in_dt,out_dt,residual,shift", [
+    (1, 16, 16, "f32", "f32", False, 0), (31, 16, 48, "f32", "f32", True, 1), (129, 48, 80, "f32", "f32", False, 1),
+    (300, 64, 256, "f16", "f32", True, 0), (257, 128, 512, "f32", "f16", True, 1), (130, 256, 1024, "f32", "f32", True, 0),
+    (65, 40, 64, "f32", "f32", False, 0)])
+def test_transition_f32_pairs(dev, rows, c, h, in_dt, out_dt, residual, shift):
+    # f32 precision on the f16 matrix units: ragged row and column tiles, both
+    # LayerNorm kernels, activations and outputs off 16-byte alignment (shift
+    # elements; the workspace and the weights then lie on 4 bytes), f16 in or out, the residual; the last shape keeps the f32 GEMM
+    # (40 channels). The LayerNorm scales, the first linear's columns and the
+    # second's rows carry factors of 1e-6 to 1e6 that cancel in the result, as
+    # any weight may: the powers of two that the pairs are stored with follow
+    # them. f32 out: the f32 bound of the other tests; f16 out: half an ulp of
+    # the largest value besides.
+    import torch
+
+    from afhip import transition
+
+    inp = transition_case(rows, c, h, 7 * rows + c)
+    w = {k: np.array(v, np.float64) for k, v in inp["weights"].items()}
+    fc, fh = 10.0 ** ref.uniform(81, (c,), -6, 6), 10.0 ** ref.uniform(82, (h,), -6, 6)
+    w["layerNormScale"] *= fc
+    w["layerNormOffset"] *= fc
+    w["firstWeight"] *= fh[None, :] / fc[:, None]
+    w["firstBias"] *= fh
+    w["secondWeight"] /= fh[:, None]
+    w = {k: v.astype(np.float32) for k, v in w.items()}
+    tdt = {"f32": torch.float32, "f16": torch.float16}
+    x = ref.round_f16(inp["activations"])
+    old = ref.round_f16(ref.normal(5, (rows, c)))
+    expect = ref.transition(x, w) + (old if residual else 0)
+    op = transition.Transition(rows, c, h, in_dtype=in_dt, out_dtype=out_dt, residual=residual)
+    for name in ("workspace", "prepared"):
+        buffer = getattr(op, name)
+        setattr(op, name, torch.empty(buffer.numel() + 16, dtype=torch.uint8, device=dev)[4 * shift:][:buffer.numel()])
+    op.prepare(w)
+
+    def place(a, dtype):
+        flat = torch.zeros(rows * c + shift, dtype=tdt[dtype], device=dev)
+        flat[shift:] = torch.from_numpy(a).to(dev).reshape(-1)
+        return flat[shift:].reshape(rows, c)
+
+    out = op(place(x, in_dt), out=place(old, out_dt)).float().cpu().numpy()
+    assert np.abs(out - expect).max() <= (1e-5 if out_dt == "f32" else 1e-5 + 2.0 ** -11) * np.abs(expect).max()
