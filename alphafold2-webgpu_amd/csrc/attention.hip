@@ -27,11 +27,17 @@
 // which hands each lane its channel's keys in the order of those registers.
 // Its logits are kept in base-2 units (q, the key bias and the pair bias
 // carry a factor log2(e)), which changes nothing but the rounding:
-// exp2(log2(e) x) = exp(x). Any other head dimension, or f32 precision, runs
-// the same two products on the f32 MFMA, on the natural units.
+// exp2(log2(e) x) = exp(x).
+//
+// At f32 precision with channels a multiple of 16 every product runs on the
+// f16 MFMA over pairs of f16 (gemm.h), the scales powers of two from bounds
+// that hold for any input (attention_pair_*_kernel). Any other width, or f16
+// precision with another head dimension, runs the two products of the
+// attention on the f32 MFMA, on the natural units.
 #include <algorithm>
 #include <cmath>
 #include <cstddef>
+#include <type_traits>
 
 #include "dma.h"
 #include "gemm.h"
@@ -48,9 +54,20 @@ bool fast_path(const afhip_attention_desc& d) {
   return d.precision == AFHIP_PRECISION_F16 && (d.channels / d.heads) % 8 == 0;
 }
 
+// f32 precision over pairs: whole 16-channel blocks, and byte offsets within a
+// batch entry's f32 q, k, v, g rows in 32 bits (the flash kernel's, which
+// fetches up to 63 rows past the last before it cuts an offset back).
+bool pair_path(const afhip_attention_desc& d) {
+  return d.precision == AFHIP_PRECISION_F32 && d.channels % 16 == 0 &&
+         ((int64_t)d.queries + 64) * 16 * d.channels <= (int64_t)UINT32_MAX;
+}
+
 // Prepared weights: everything the kernels read, in their dtypes.
 struct AttentionWeights {
   size_t ln_scale, ln_offset, w_proj, b_proj, w_out, b_out, pair_scale, pair_offset, w_bias, total;
+  // The pair path: output scales of the two products, each head's logit scale
+  // and value exponent, and the bounds they were taken from.
+  size_t s_proj, s_out, logit_scale, v_exp, bound;
 };
 
 AttentionWeights weights_layout(const afhip_attention_desc& d) {
@@ -73,6 +90,13 @@ AttentionWeights weights_layout(const afhip_attention_desc& d) {
   w.pair_scale = take(4 * pc);
   w.pair_offset = take(4 * pc);
   w.w_bias = take(4 * pc * d.heads);  // [channel][head]
+  if (pair_path(d)) {
+    w.s_proj = take(4 * 4 * C);
+    w.s_out = take(4 * C);
+    w.logit_scale = take(4 * (size_t)d.heads);
+    w.v_exp = take(4 * (size_t)d.heads);
+    w.bound = take(4 * 4 * C);
+  }
   w.total = at;
   return w;
 }
@@ -203,6 +227,125 @@ __global__ void attention_prepare_kernel(const float* __restrict__ packed, int C
   }
 }
 
+struct AttentionPairOut {
+  half_t* w_out;
+  float *s_out, *b_out, *ln_scale, *ln_offset, *pair_scale, *pair_offset, *w_bias;
+};
+
+// The pair path's projections, one workgroup a row n of [4C][C] (q, k, v, g):
+// W'[n] = W[n] diag(gamma) (q rows over sqrt(d) too) in double, stored as pairs
+// times 2^e with the largest element in [2^14, 2^15); bias' = W beta (+ the
+// gating bias). x_hat, whose 2-norm is at most sqrt(C), is stored times 2^x_exp,
+// so s_proj = 2^-(x_exp + e) gives the output, and no output exceeds
+// bound[n] = sqrt(C) |W'[n]|_2 + |bias'|.
+__global__ __launch_bounds__(256) void attention_pair_project_kernel(const float* __restrict__ packed, int C, int H,
+                                                                     int x_exp, half_t* __restrict__ w_proj,
+                                                                     float* __restrict__ s_proj,
+                                                                     float* __restrict__ b_proj,
+                                                                     float* __restrict__ bound) {
+  const float* gamma = packed;
+  const float* beta = gamma + C;
+  const int n = blockIdx.x, part = n / C, col = n - part * C;
+  const float* w = beta + C + (int64_t)part * C * C + col;  // [k][C]
+  const double unit = part == 0 ? 1.0 / sqrt((double)(C / H)) : 1.0;
+  float most = 0.0f;
+  double squares = 0.0, offset = 0.0;
+  for (int k = threadIdx.x; k < C; k += 256) {
+    const double wk = w[(int64_t)k * C] * unit, g = wk * gamma[k];
+    most = fmaxf(most, fabsf((float)g));
+    squares += g * g;
+    offset += wk * beta[k];
+  }
+  __shared__ float m_part[4];
+  __shared__ double s_part[4], o_part[4];
+  for (int o = 32; o > 0; o >>= 1) {
+    most = fmaxf(most, __shfl_xor(most, o));
+    squares += __shfl_xor(squares, o);
+    offset += __shfl_xor(offset, o);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    m_part[threadIdx.x >> 6] = most;
+    s_part[threadIdx.x >> 6] = squares;
+    o_part[threadIdx.x >> 6] = offset;
+  }
+  __syncthreads();
+  const int e = pair_exponent(fmaxf(fmaxf(m_part[0], m_part[1]), fmaxf(m_part[2], m_part[3])));
+  for (int k = threadIdx.x; k < C; k += 256)
+    pair_store(w_proj + (int64_t)n * 2 * C, k, (float)ldexp(w[(int64_t)k * C] * unit * gamma[k], e));
+  if (threadIdx.x == 0) {
+    double bias = (o_part[0] + o_part[1]) + (o_part[2] + o_part[3]);
+    if (part == 3) bias += packed[2 * (int64_t)C + 4 * (int64_t)C * C + col];
+    squares = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+    s_proj[n] = ldexpf(1.0f, -(x_exp + e));
+    b_proj[n] = (float)bias;
+    bound[n] = (float)(sqrt((double)C * squares) + fabs(bias));
+  }
+}
+
+// One wave a head: q, k and v leave the projection times the power of two that
+// takes the head's largest bound to [2^14, 2^15], so the flash kernel's pairs
+// hold them whatever the input; the logits carry 2^(q + k) back, and v's
+// exponent, which the attention's output keeps, goes into the output weights.
+__global__ __launch_bounds__(64) void attention_pair_heads_kernel(int C, int H, const float* __restrict__ bound,
+                                                                  float* __restrict__ s_proj,
+                                                                  float* __restrict__ b_proj,
+                                                                  float* __restrict__ logit_scale,
+                                                                  int* __restrict__ v_exp) {
+  const int h = blockIdx.x, lane = threadIdx.x, d = C / H;  // d <= 32
+  int exps[3];
+#pragma unroll
+  for (int part = 0; part < 3; part++) {
+    const int n = part * C + h * d + lane;
+    float most = lane < d ? bound[n] : 0.0f;
+    for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
+    exps[part] = pair_exponent(most);
+    if (lane < d) {
+      s_proj[n] = ldexpf(s_proj[n], exps[part]);
+      b_proj[n] = ldexpf(b_proj[n], exps[part]);
+    }
+  }
+  if (lane == 0) {
+    logit_scale[h] = ldexpf(1.0f, min(max(-(exps[0] + exps[1]), -120), 120));
+    v_exp[h] = exps[2];
+  }
+}
+
+// The output projection, one workgroup a row n of [C][C], and the tensors that
+// are kept as they are (pair LayerNorm, pair bias weights) in row 0's.
+__global__ __launch_bounds__(256) void attention_pair_output_kernel(const float* __restrict__ packed, int C, int H, int pc,
+                                                                    int separate, int has_bias,
+                                                                    const int* __restrict__ v_exp,
+                                                                    AttentionPairOut o) {
+  const int n = blockIdx.x, d = C / H;
+  const float* w = packed + 3 * (int64_t)C + 4 * (int64_t)C * C;  // [k][C]
+  auto value = [&](int k) { return ldexpf(w[(int64_t)k * C + n], -v_exp[k / d]); };
+  float most = 0.0f;
+  for (int k = threadIdx.x; k < C; k += 256) most = fmaxf(most, fabsf(value(k)));
+  __shared__ float part[4];
+  for (int s = 32; s > 0; s >>= 1) most = fmaxf(most, __shfl_xor(most, s));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = most;
+  __syncthreads();
+  const int e = pair_exponent(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
+  for (int k = threadIdx.x; k < C; k += 256) pair_store(o.w_out + (int64_t)n * 2 * C, k, ldexpf(value(k), e));
+  const float* b = w + (int64_t)C * C;
+  if (threadIdx.x == 0) {
+    o.s_out[n] = ldexpf(1.0f, -e);
+    o.b_out[n] = b[n];
+    o.ln_scale[n] = packed[n];
+    o.ln_offset[n] = packed[C + n];
+  }
+  if (n != 0 || !has_bias) return;
+  const float* p = b + C;
+  if (separate) {
+    for (int c = threadIdx.x; c < pc; c += 256) {
+      o.pair_scale[c] = p[c];
+      o.pair_offset[c] = p[pc + c];
+    }
+    p += 2 * (int64_t)pc;
+  }
+  for (int64_t i = threadIdx.x; i < (int64_t)pc * H; i += 256) o.w_bias[i] = p[i];
+}
+
 // One row pass over [rows][C]: LayerNorm (two-pass mean and biased variance,
 // eps inside the root, attention.ts:312-324) and, as asked, the normalised
 // row, the row's key bias key_scale (mask - 1) (:688-690), and the pair bias
@@ -215,6 +358,7 @@ struct RowsArgs {
   const float* offset;
   float eps;
   void* out;                // [rows][C] in attention order, or null
+  float x_scale;            // pairs out: they hold the rows before the affine times this
   const float* mask;        // source order, or null (no key bias)
   float* key_bias;          // [B][stride] f32, or null
   float key_scale;
@@ -254,6 +398,10 @@ __device__ __forceinline__ void pair_bias_store(const RowsArgs& a, int h, int64_
   if (q == a.Q - 1)
     for (int k = a.Q; k < a.stride; k++) row[k] = 0.0f;
 }
+
+struct pair_t {
+  uint32_t bits;
+};  // an f32 element of a pair row, in size and as a type's name
 
 template <typename T> __device__ __forceinline__ void load8(const T* p, float (&v)[8]) {
   if constexpr (sizeof(T) == 2) {
@@ -340,8 +488,25 @@ __global__ __launch_bounds__(256) void attention_rows_kernel(RowsArgs a) {
     }
     const float rstd = 1.0f / sqrtf(lane_sum<LANES>(var) / (float)C + a.eps);
 #pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = (v[e] - mean) * rstd * sc[e] + of[e];
-    if (a.out && live) store8(reinterpret_cast<OT*>(a.out) + rr * C + 8 * j, v);
+    for (int e = 0; e < 8; e++) v[e] = (v[e] - mean) * rstd;
+    if constexpr (std::is_same<OT, pair_t>::value) {
+      if (a.out && live) {
+        half8 h, l;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          half2v h2, l2;
+          pair_split2(v[e] * a.x_scale, v[e + 1] * a.x_scale, h2, l2);
+          h[e] = h2[0], h[e + 1] = h2[1], l[e] = l2[0], l[e + 1] = l2[1];
+        }
+        half_t* p = reinterpret_cast<half_t*>(a.out) + rr * 2 * C + pair_index(8 * j);
+        *reinterpret_cast<half8*>(p) = h;
+        *reinterpret_cast<half8*>(p + 16) = l;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = v[e] * sc[e] + of[e];
+    if constexpr (!std::is_same<OT, pair_t>::value)
+      if (a.out && live) store8(reinterpret_cast<OT*>(a.out) + rr * C + 8 * j, v);
     if (a.mask && live && j == 0) key_bias_store(a, b, q, a.mask[src]);
     if (a.w) {
       float acc[HB] = {};
@@ -386,8 +551,12 @@ __global__ __launch_bounds__(256) void attention_rows_any_kernel(RowsArgs a) {
   for (int o = 32; o > 0; o >>= 1) var += __shfl_xor(var, o);
   const float rstd = 1.0f / sqrtf(var / (float)C + a.eps);
   if (a.out)
-    for (int c = lane; c < C; c += 64)
-      reinterpret_cast<OT*>(a.out)[r * C + c] = (OT)((ld(xr, c) - mean) * rstd * a.scale[c] + a.offset[c]);
+    for (int c = lane; c < C; c += 64) {
+      if constexpr (std::is_same<OT, pair_t>::value)
+        pair_store(reinterpret_cast<half_t*>(a.out) + r * 2 * C, c, (ld(xr, c) - mean) * rstd * a.x_scale);
+      else
+        reinterpret_cast<OT*>(a.out)[r * C + c] = (OT)((ld(xr, c) - mean) * rstd * a.scale[c] + a.offset[c]);
+    }
   if (a.mask && lane == 0) key_bias_store(a, b, q, a.mask[src]);
   if (a.w) {
     for (int h = 0; h < a.H; h++) {
@@ -406,6 +575,7 @@ struct FlashArgs {
   const half_t* key_mask; // [B][code_stride] codes (f16 kernels)
   const float* bias;      // [H][Q][stride] or null
   void* weighted;         // [B Q][C] in source order
+  const float* logit_scale; // [H] (pair kernel)
   int B, Q, C, H, d, transpose, stride, code_stride;
   float clamp;
 };
@@ -605,6 +775,218 @@ template <typename CT> int launch_flash_f32(const FlashArgs& fa, hipStream_t st)
     }
   }
   return launch_flash_f32_as<CT, 32, false>(fa, st);
+}
+
+// The same attention over pairs of f16 (f32 precision): q, k and v arrive in f32,
+// scaled by powers of two that keep them below 2^15 (attention_pair_heads_kernel),
+// and are split into h + l as they are loaded; the weights e^(x - m) are split
+// times 2^kPairWeight. Three products (h h, h l, l h) a step of 16 on the f16 MFMA, 384
+// cycles a block at head dimension 32 against 2,048. Loads, key order, clamp and
+// offset as in the f32 kernel above; the output, still times v's power of two,
+// leaves as pairs for the output projection.
+// Bound: the loads (20 instructions a block over 32 rows each, for every wave
+// its own). Column attention over 508 sequences x 59 residues, 8 heads of 32:
+// 115 us, the f32 kernel 163; dropping a third of the vector instructions
+// (v_fma_mix_f32 in the split, no per-load bound) left it at 117.
+// log2: keeps small weights' l out of f16's last digits. A weight is at most
+// 2^(kPairWeight + 2.9) (the slack), times 2^8 where every key is masked: there
+// x = m = -1e8, and the rounding of `offset` is up to 8. That is below 65504.
+constexpr float kPairWeight = 4.0f;
+
+// LOAD: a lane's channels element by element (0), in 16-byte chunks (1, head
+// dimension a multiple of four) or in whole steps (2, exactly 16 STEPS channels).
+template <int STEPS, int LOAD, bool BIAS>
+__global__ __launch_bounds__(64 * kF32Waves) void attention_flash_pair_kernel(FlashArgs a, int qtiles, int64_t tiles,
+                                                                              int64_t per_xcd) {
+  const int lane = threadIdx.x & 63, col = lane & 31, hi = lane >> 5;
+  const int64_t group = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const int64_t t = group * kF32Waves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (t >= tiles) return;  // the whole wave
+  const int q0 = 32 * (int)(t % qtiles);
+  const int h = (int)(t / qtiles % a.H);
+  const int64_t b = t / qtiles / a.H;
+  const int Q = a.Q, d = a.d;
+  const uint32_t ldb = 16u * (uint32_t)a.C;  // bytes between rows
+  const char* rows = reinterpret_cast<const char*>(a.qkvg) + (b * Q * 4 * a.C + (int64_t)h * d) * 4;
+  const char* keys = rows + (int64_t)a.C * 4;
+  const char* vals = keys + (int64_t)a.C * 4;
+  const float unit = a.logit_scale[h];
+
+  // A lane's channels of the row at `off`: 16 s + 8 hi + [0, 8) of step s.
+  auto load_row = [&](const char* base, uint32_t off, float (&f)[8 * STEPS]) {
+    const float* p = reinterpret_cast<const float*>(base + off);
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+      if constexpr (LOAD) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const int c = 16 * s + 8 * hi + 4 * i;
+          const float4 w = *reinterpret_cast<const float4*>(p + c);  // past the head: the row's next columns
+          const bool in = LOAD == 2 || c < d;
+          f[8 * s + 4 * i] = in ? w.x : 0.0f, f[8 * s + 4 * i + 1] = in ? w.y : 0.0f;
+          f[8 * s + 4 * i + 2] = in ? w.z : 0.0f, f[8 * s + 4 * i + 3] = in ? w.w : 0.0f;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const int c = 16 * s + 8 * hi + e;
+          const float w = p[min(c, d - 1)];
+          f[8 * s + e] = c < d ? w : 0.0f;
+        }
+      }
+    }
+  };
+  auto split8 = [&](const float* f, half8& hh, half8& ll) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      half2v h2, l2;
+      pair_split2(f[e], f[e + 1], h2, l2);
+      hh[e] = h2[0], hh[e + 1] = h2[1], ll[e] = l2[0], ll[e + 1] = l2[1];
+    }
+  };
+  // Whole blocks add their uniform offset to the (scalar) base; in the last
+  // one, and past it, keys past the end repeat the last.
+  const uint32_t last = (uint32_t)(Q - 1) * ldb;
+  const uint32_t key0 = (uint32_t)col * ldb;
+  auto load_keys = [&](int k0, float (&f)[8 * STEPS]) {
+    if (k0 + 32 <= Q) load_row(keys + (uint32_t)k0 * ldb, key0, f);
+    else load_row(keys, min(key0 + (uint32_t)k0 * ldb, last), f);
+  };
+  // Channels past the head dimension repeat the last (those rows of O^T are not stored).
+  const uint32_t chan = 4u * (uint32_t)min(col, d - 1);
+  const uint32_t val0 = (uint32_t)(4 * hi) * ldb + chan, val_last = last + chan;
+  auto load_vals = [&](int k0, float (&f)[16]) {
+    if (k0 + 32 <= Q) {
+#pragma unroll
+      for (int v = 0; v < 16; v++)
+        f[v] = *reinterpret_cast<const float*>(vals + (uint32_t)(k0 + 8 * (v >> 2)) * ldb + (val0 + (v & 3) * ldb));
+    } else {
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const uint32_t off = val0 + (uint32_t)(k0 + 8 * (v >> 2) + (v & 3)) * ldb;
+        f[v] = *reinterpret_cast<const float*>(vals + min(off, val_last));
+      }
+    }
+  };
+  const int myq = q0 + col, qc = min(myq, Q - 1);
+  const float* kb_row = a.key_bias + b * a.stride;
+  const float* pb_row = BIAS ? a.bias + ((int64_t)h * Q + qc) * a.stride : nullptr;
+  auto load_bias = [&](const float* row, int k0, float (&f)[16]) {
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const float4 w = *reinterpret_cast<const float4*>(row + min(k0 + 8 * g + 4 * hi, a.stride - 4));
+      f[4 * g] = w.x, f[4 * g + 1] = w.y, f[4 * g + 2] = w.z, f[4 * g + 3] = w.w;
+    }
+  };
+
+  float kf[8 * STEPS], vf[16], kb[16], pb[16];
+  half8 qh[STEPS], ql[STEPS];
+  {
+    float qf[8 * STEPS];
+    load_keys(0, kf);
+    load_row(rows, (uint32_t)qc * ldb, qf);
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) split8(qf + 8 * s, qh[s], ql[s]);
+  }
+  load_bias(kb_row, 0, kb);
+  if constexpr (BIAS) load_bias(pb_row, 0, pb);
+  // The loop's order of loads (see the f32 kernel).
+  __builtin_amdgcn_sched_barrier(0);
+  load_vals(0, vf);
+  __builtin_amdgcn_sched_barrier(0);
+
+  floatx16 o = {};
+  float m = -1e30f, offset = 0.0f;
+  float sum = 0.0f;  // over this lane half's keys
+  for (int k0 = 0; k0 < Q; k0 += 32) {
+    floatx16 sc = {};
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+      half8 kh, kl;
+      split8(kf + 8 * s, kh, kl);
+      sc = mfma_f16(kh, qh[s], sc);
+      sc = mfma_f16(kh, ql[s], sc);
+      sc = mfma_f16(kl, qh[s], sc);
+    }
+    load_keys(k0 + 32, kf);
+    float x[16];
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+      const float l = fmaf(sc[v], unit, kb[v]);
+      x[v] = __builtin_amdgcn_fmed3f(BIAS ? l + pb[v] : l, -a.clamp, a.clamp);
+    }
+    load_bias(kb_row, k0 + 32, kb);
+    if constexpr (BIAS) load_bias(pb_row, k0 + 32, pb);
+    if (k0 + 32 > Q) {
+#pragma unroll
+      for (int v = 0; v < 16; v++)
+        if (k0 + 8 * (v >> 2) + 4 * hi + (v & 3) >= Q) x[v] = kDropped;
+    }
+    float mx = x[0];
+#pragma unroll
+    for (int v = 1; v < 16; v++) mx = fmaxf(mx, x[v]);
+    if (__builtin_amdgcn_ballot_w64(mx > m + kF32Slack)) {
+      const float to = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)));
+      const float f = __builtin_amdgcn_exp2f((m - to) * kLog2e);
+      sum *= f;
+#pragma unroll
+      for (int v = 0; v < 16; v++) o[v] *= f;
+      m = to;
+      offset = fmaf(-to, kLog2e, kPairWeight);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; v++) x[v] = __builtin_amdgcn_exp2f(fmaf(x[v], kLog2e, offset));
+    sum += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])) +
+           (((x[8] + x[9]) + (x[10] + x[11])) + ((x[12] + x[13]) + (x[14] + x[15])));
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      half8 ph, pl, vh, vl;
+      split8(x + 8 * s, ph, pl);
+      split8(vf + 8 * s, vh, vl);
+      o = mfma_f16(vh, ph, o);
+      o = mfma_f16(vh, pl, o);
+      o = mfma_f16(vl, ph, o);
+    }
+    load_vals(k0 + 32, vf);
+  }
+  sum += __shfl_xor(sum, 32);
+  if (myq >= Q) return;
+  const float* gr = reinterpret_cast<const float*>(rows + (uint32_t)myq * ldb) + 3 * (int64_t)a.C;
+  const int64_t src = a.transpose ? (int64_t)myq * a.B + b : b * Q + myq;
+  half_t* out = reinterpret_cast<half_t*>(a.weighted) + src * 2 * a.C;
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    const int c = 8 * g + 4 * hi;
+    if constexpr (LOAD) {
+      if (c >= d) break;
+      const float4 gv = *reinterpret_cast<const float4*>(gr + c);
+      half2v h0, l0, h1, l1;
+      pair_split2(o[4 * g] / sum * gv.x, o[4 * g + 1] / sum * gv.y, h0, l0);
+      pair_split2(o[4 * g + 2] / sum * gv.z, o[4 * g + 3] / sum * gv.w, h1, l1);
+      half_t* p = out + pair_index(h * d + c);
+      *reinterpret_cast<half4*>(p) = half4{h0[0], h0[1], h1[0], h1[1]};
+      *reinterpret_cast<half4*>(p + 16) = half4{l0[0], l0[1], l1[0], l1[1]};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (c + i < d) pair_store(out, h * d + c + i, o[4 * g + i] / sum * gr[c + i]);
+    }
+  }
+}
+
+template <int STEPS, int LOAD> int launch_flash_pair_as(const FlashArgs& fa, hipStream_t st) {
+  const int qtiles = (int)ceil_div(fa.Q, 32);
+  const int64_t tiles = (int64_t)fa.B * fa.H * qtiles, per_xcd = ceil_div(tiles, 8 * kF32Waves);
+  AFHIP_REQUIRE(per_xcd < ((int64_t)1 << 28), "attention grid too large");
+  auto k = fa.bias ? attention_flash_pair_kernel<STEPS, LOAD, true> : attention_flash_pair_kernel<STEPS, LOAD, false>;
+  return launch("attention.flash", k, dim3((unsigned)(8 * per_xcd)), dim3(64 * kF32Waves), 0, st, fa, qtiles, tiles,
+                per_xcd);
+}
+
+int launch_flash_pair(const FlashArgs& fa, hipStream_t st) {
+  if (fa.d % 4) return launch_flash_pair_as<2, 0>(fa, st);
+  if (fa.d == 32) return launch_flash_pair_as<2, 2>(fa, st);
+  return fa.d <= 16 ? launch_flash_pair_as<1, 1>(fa, st) : launch_flash_pair_as<2, 1>(fa, st);
 }
 
 // f16 operands, head_dim 32: one wave per 32 queries of one (b, h), keys in
@@ -1264,7 +1646,12 @@ int launch_rows_typed(const RowsArgs& r, const char* label, hipStream_t st) {
   return launch(label, attention_rows_any_kernel<IT, OT>, dim3((unsigned)ceil_div(r.rows, 4)), block, 0, st, r);
 }
 
+// out_dtype kPairRows: pairs (x_scale says how they are scaled).
+constexpr int kPairRows = -1;
 int launch_rows(const RowsArgs& r, int in_dtype, int out_dtype, const char* label, hipStream_t st) {
+  if (out_dtype == kPairRows)
+    return in_dtype == AFHIP_F16 ? launch_rows_typed<half_t, pair_t>(r, label, st)
+                                 : launch_rows_typed<float, pair_t>(r, label, st);
   if (in_dtype == AFHIP_F16)
     return out_dtype == AFHIP_F16 ? launch_rows_typed<half_t, half_t>(r, label, st)
                                   : launch_rows_typed<half_t, float>(r, label, st);
@@ -1301,6 +1688,20 @@ int afhip_attention_prepare_weights(const afhip_attention_desc* desc, const floa
   const int sep = d.pair_bias == AFHIP_PAIR_BIAS_SEPARATE;
   const int pc = sep ? d.pair_channels : d.channels;
   hipStream_t st = (hipStream_t)stream;
+  if (pair_path(d)) {
+    float *sp = (float*)(p + w.s_proj), *bp = (float*)(p + w.b_proj), *bound = (float*)(p + w.bound);
+    if (int s = launch("attention.prepare", attention_pair_project_kernel, dim3(4 * d.channels), dim3(256), 0, st, packed,
+                       d.channels, d.heads, pair_norm_exponent(d.channels), (half_t*)(p + w.w_proj), sp, bp, bound))
+      return s;
+    if (int s = launch("attention.prepare", attention_pair_heads_kernel, dim3(d.heads), dim3(64), 0, st, d.channels,
+                       d.heads, (const float*)bound, sp, bp, (float*)(p + w.logit_scale), (int*)(p + w.v_exp)))
+      return s;
+    const AttentionPairOut o{(half_t*)(p + w.w_out),   (float*)(p + w.s_out),      (float*)(p + w.b_out),
+                             (float*)(p + w.ln_scale), (float*)(p + w.ln_offset),  (float*)(p + w.pair_scale),
+                             (float*)(p + w.pair_offset), (float*)(p + w.w_bias)};
+    return launch("attention.prepare", attention_pair_output_kernel, dim3(d.channels), dim3(256), 0, st, packed,
+                  d.channels, d.heads, pc, sep, (int)(d.pair_bias != 0), (const int*)(p + w.v_exp), o);
+  }
   if (d.precision == AFHIP_PRECISION_F16)
     return launch("attention.prepare", attention_prepare_kernel<half_t>, dim3(1024), dim3(256), 0, st, packed,
                   d.channels, d.heads, pc, sep, d.pair_bias != 0, (float*)(p + w.ln_scale), (float*)(p + w.ln_offset),
@@ -1327,7 +1728,7 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
                 workspace_bytes, ws.total);
   hipStream_t st = (hipStream_t)stream;
   const bool f16 = d.precision == AFHIP_PRECISION_F16;
-  const bool fast = fast_path(d);
+  const bool fast = fast_path(d), pairs = pair_path(d);
   const float unit = fast ? kLog2e : 1.0f;  // logits in base-2 units on the fast path
   const int ct = f16 ? AFHIP_F16 : AFHIP_F32;
   const char* wp = (const char*)prepared;
@@ -1350,6 +1751,7 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
     r.offset = (const float*)(wp + w.ln_offset);
     r.eps = d.epsilon;
     r.out = wsb + ws.normalized;
+    r.x_scale = pairs ? ldexpf(1.0f, pair_norm_exponent(C)) : 1.0f;
     r.mask = mask;
     if (fast) {
       r.key_mask = (half_t*)(wsb + ws.key_mask);
@@ -1365,7 +1767,7 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
     }
     r.stride = ws.stride;
     r.code_stride = ws.code_stride;
-    if ((s = launch_rows(r, d.in_dtype, ct, "attention.norm", st))) return s;
+    if ((s = launch_rows(r, d.in_dtype, pairs ? kPairRows : ct, "attention.norm", st))) return s;
   }
   // 2. A separate pair source: its own LayerNorm, projected to the heads.
   if (d.pair_bias == AFHIP_PAIR_BIAS_SEPARATE) {
@@ -1402,7 +1804,13 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
     g.head_cols = C;
     g.q_scale = unit / sqrtf((float)(C / H));
     GemmTypes t{d.precision, ct, ct, ct};
-    if ((s = run_gemm(g, t, select_variant(t, g.M, g.N, g.K, 1), "attention.project", st))) return s;
+    if (pairs) {  // q's 1 / sqrt(d) is in the weights
+      g.scale = (const float*)(wp + w.s_proj);
+      g.flags |= AFHIP_EPILOGUE_SCALE;
+      if ((s = run_gemm_pairs(g, AFHIP_F32, "attention.project", st))) return s;
+    } else if ((s = run_gemm(g, t, select_variant(t, g.M, g.N, g.K, 1), "attention.project", st))) {
+      return s;
+    }
   }
   // 4. Attention.
   {
@@ -1412,6 +1820,7 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
     fa.key_mask = (const half_t*)(wsb + ws.key_mask);
     fa.bias = bias;
     fa.weighted = wsb + ws.weighted;
+    fa.logit_scale = (const float*)(wp + w.logit_scale);
     fa.B = B;
     fa.Q = Q;
     fa.C = C;
@@ -1441,6 +1850,8 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
                         dim3(kFlashThreads), 0, st, fa)
                : launch("attention.flash", attention_flash_f16_kernel<false>, dim3((unsigned)groups),
                         dim3(kFlashThreads), 0, st, fa);
+    } else if (pairs) {
+      s = launch_flash_pair(fa, st);
     } else {
       s = f16 ? launch_flash_f32<half_t>(fa, st) : launch_flash_f32<float>(fa, st);
     }
@@ -1470,6 +1881,11 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
     GemmArgs gs = g;
     gs.flags &= ~AFHIP_EPILOGUE_RESIDUAL;
     gs.residual = nullptr;
+    if (pairs) {
+      g.scale = (const float*)(wp + w.s_out);
+      g.flags |= AFHIP_EPILOGUE_SCALE;
+      return run_gemm_pairs(g, d.out_dtype, "attention.output", st);
+    }
     const bool fused = C <= 128;
     if (d.residual && !fused) gs.c = wsb + ws.normalized;
     const bool aligned = (reinterpret_cast<uintptr_t>(out) & 15) == 0;

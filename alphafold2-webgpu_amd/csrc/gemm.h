@@ -59,6 +59,15 @@ __device__ __forceinline__ void pair_split(float x, half_t& h, half_t& l) {
   h = (half_t)x;
   l = (half_t)(x - (float)h);
 }
+// Two values at once (v_cvt_pk_f16_f32).
+__device__ __forceinline__ void pair_split2(float x0, float x1, half2v& h, half2v& l) {
+  typedef float float2v __attribute__((ext_vector_type(2)));
+  asm("" : "+v"(x0), "+v"(x1));
+  h = __builtin_convertvector(float2v{x0, x1}, half2v);
+  // v_fma_mix_f32 reads h as it is
+  const float d0 = __builtin_fmaf((float)h[0], -1.0f, x0), d1 = __builtin_fmaf((float)h[1], -1.0f, x1);
+  l = __builtin_convertvector(float2v{d0, d1}, half2v);
+}
 __device__ __forceinline__ void pair_store(half_t* row, int64_t k, float x) {
   half_t h, l;
   pair_split(x, h, l);

@@ -354,3 +354,49 @@ def test_f32_mfma_flash_edges(dev, name, S, L, C, H, precision):
     expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
     got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb, precision=precision)
     assert np.abs(got - expect).max() <= (7e-5 if precision == "f32" else 1e-2) * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("C,H", [(16, 4), (80, 16), (48, 4), (64, 4), (112, 4), (128, 4), (96, 32)])
+@pytest.mark.parametrize("name,S,L,residual,shift", [("msa_column", 33, 2, True, 1), ("triangle_start", 0, 65, False, 0),
+                                                     ("triangle_end", 0, 31, True, 0), ("msa_row", 3, 32, False, 1)])
+def test_f32_pairs_attention(dev, name, S, L, residual, shift, C, H):
+    # f32 precision over pairs of f16: head dimensions 4, 5, 12, 16, 28, 32 and
+    # 3 (chunked and element-wise loads, one and two steps of 16 channels),
+    # ragged query and key blocks, fully masked rows, the residual, and the
+    # weights and the workspace on 4 bytes (shift). The LayerNorm scales and the
+    # projections' columns carry factors of 1e-6 to 1e6 that cancel (queries
+    # against keys, values against the output weights), as any weight may. The
+    # f32 bound of the other tests.
+    import torch
+
+    from afhip import attention
+
+    x, mask, B, Q, tr, w, pb = case(name, S, L, C, H, Cp=12)
+    w = {k: np.array(v, np.float64).reshape(v.shape) for k, v in w.items()}
+    fc, fk = 10.0 ** ref.uniform(91, (C,), -6, 6), 10.0 ** ref.uniform(92, (H,), -6, 6)
+    fv = 10.0 ** ref.uniform(93, (H,), -6, 6)
+    fk, fv = np.repeat(fk, C // H), np.repeat(fv, C // H)
+    if name == "msa_column":  # the normalized-input bias reads the affine too, so the factors stay with the others
+        w["queryNormScale"] *= fc
+        w["queryNormOffset"] *= fc
+        for k in ("queryWeight", "keyWeight", "valueWeight", "gatingWeight"):
+            w[k] = w[k] / fc[:, None]
+    w["queryWeight"] = w["queryWeight"] * fk
+    w["keyWeight"] = w["keyWeight"] / fk
+    w["valueWeight"] = w["valueWeight"] * fv
+    w["outputWeight"] = w["outputWeight"] / fv[:, None]
+    w = {k: v.astype(np.float32) for k, v in w.items()}
+    old = ref.normal(17, (B * Q, C))
+    expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb) + (old.reshape(-1) if residual else 0)
+    separate = pb is not None and pb["source"] == "separate"
+    op = attention.Attention(B, Q, C, H, transpose=tr, pair_bias=None if pb is None else pb["source"],
+                             pair_channels=pb["channels"] if separate else 0, residual=residual)
+    for buffer in ("workspace", "prepared"):
+        size = getattr(op, buffer).numel()
+        setattr(op, buffer, torch.empty(size + 16, dtype=torch.uint8, device=dev)[4 * shift:][:size])
+    op.prepare(attention.pack_weights(w, pb))
+    to = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.float32)).to(dev)  # noqa: E731
+    out = op(to(x.reshape(B * Q, C)), to(mask), to(pb["activations"]) if separate else None,
+             out=to(old) if residual else None)
+    got = out.cpu().numpy().reshape(-1)
+    assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()
