@@ -17,6 +17,9 @@
 //     over the hidden channels in LDS and projected by linearZ; the same pairs
 //     of z are normalised and projected by linearG; out = (p + bz)*sig(g + bg).
 //     The gate is recomputed here from z rather than stored and re-read.
+//
+// At f32 precision 1 and 3 multiply pairs of f16 on the f16 MFMA (gemm.h; the
+// tri_*_pair kernels below); the contraction is the f32 GEMM.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -35,6 +38,7 @@ struct TriWeights {
   // Offsets in bytes into the prepared buffer.
   size_t ln_in_w, ln_in_b, w_proj, b_proj, ln_out_w, ln_out_b, w_z, b_z, w_g, b_g;
   size_t fold_w, fold_b;  // the f16 fast path's folded weights (0 when not eligible)
+  size_t s_proj, s_z, s_g;  // f32 precision: output scales of the pair products
   size_t total;
   int czp, chp, czo;  // padded input width (multiple of 32), padded hidden, padded output rows
 };
@@ -61,6 +65,11 @@ TriWeights tri_layout(const afhip_triangle_desc& d) {
   w.b_z = take(4 * (size_t)w.czo);
   w.w_g = take(es * (size_t)w.czo * w.czp);
   w.b_g = take(4 * (size_t)w.czo);
+  if (d.precision == AFHIP_PRECISION_F32) {
+    w.s_proj = take(4 * 4 * (size_t)w.chp);
+    w.s_z = take(4 * (size_t)w.czo);
+    w.s_g = take(4 * (size_t)w.czo);
+  }
   if (triangle_fast_eligible(d)) {
     w.fold_w = take(2 * (size_t)kFoldMatrices * d.c_z * d.c_z);
     w.fold_b = take(4 * (size_t)kFoldMatrices * d.c_z);
@@ -136,28 +145,30 @@ struct ProjectArgs {
   const float* mask;
   const float* ln_w;
   const float* ln_b;
-  const void* w_proj;  // [4][chp][czp]: ap, ag, bp, bg
+  const void* w_proj;  // [4][chp][czp]: ap, ag, bp, bg (the pair kernels': in fragment order)
   const float* b_proj; // [4][chp]
+  const float* s_proj; // [4][chp] (pair kernels)
   void* out_a;
   void* out_b;
   int64_t cstride;
   int L, P, cz, ch, czp, chp;
   int incoming;
   float eps;
+  float x_scale;  // the pair kernels hold x_hat times this
 };
 
-template <typename ZT, bool F16MATH>
+template <typename ZT>
 __global__ __launch_bounds__(256) void tri_project_kernel(ProjectArgs a) {
-  using CT = typename std::conditional<F16MATH, half_t, float>::type;
+  using CT = half_t;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  // xs: f32 [czp][kRows + 1], channel-major raw z; an: CT [kRows][czp + 8] (f16 only);
+  // xs: f32 [czp][kRows + 1], channel-major raw z; an: CT [kRows][czp + 8];
   // stage: CT [64][kRows + 8] output transpose.
   const int xpitch = kRows + 1;
   float* xs = reinterpret_cast<float*>(smem);
   size_t off = round_up((int64_t)a.czp * xpitch * 4, 16);
   CT* an = reinterpret_cast<CT*>(smem + off);
   const int apitch = a.czp + 8;
-  if (F16MATH) off += round_up((int64_t)kRows * apitch * 2, 16);
+  off += round_up((int64_t)kRows * apitch * 2, 16);
   CT* stage = reinterpret_cast<CT*>(smem + off);
   constexpr int spitch = kRows + 8;
 
@@ -183,8 +194,7 @@ __global__ __launch_bounds__(256) void tri_project_kernel(ProjectArgs a) {
     const int q = tid >> 2, part = tid & 3;
     for (int c = part; c < a.czp; c += 4) {
       float v = c < a.cz ? (xs[c * xpitch + q] - mean) * rstd * a.ln_w[c] + a.ln_b[c] : 0.0f;
-      if (F16MATH) an[q * apitch + c] = (CT)v;
-      else xs[c * xpitch + q] = v;
+      an[q * apitch + c] = (CT)v;
     }
   }
   __syncthreads();
@@ -204,22 +214,13 @@ __global__ __launch_bounds__(256) void tri_project_kernel(ProjectArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; v++) accp[v] = accg[v] = 0.0f;
         const int n = hc + (lane & 31);
-        if constexpr (F16MATH) {
-          for (int k = 0; k < a.czp; k += 16) {
-            const int kk = k + 8 * (lane >> 5);
-            half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
-            half8 bpf = *reinterpret_cast<const half8*>(wp + (size_t)n * a.czp + kk);
-            half8 bgf = *reinterpret_cast<const half8*>(wg + (size_t)n * a.czp + kk);
-            accp = mfma_f16(af, bpf, accp);
-            accg = mfma_f16(af, bgf, accg);
-          }
-        } else {
-          for (int k = 0; k < a.czp; k += 2) {
-            const int kk = k + (lane >> 5);
-            float af = xs[kk * xpitch + rw + (lane & 31)];
-            accp = mfma_f32(af, wp[(size_t)n * a.czp + kk], accp);
-            accg = mfma_f32(af, wg[(size_t)n * a.czp + kk], accg);
-          }
+        for (int k = 0; k < a.czp; k += 16) {
+          const int kk = k + 8 * (lane >> 5);
+          half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
+          half8 bpf = *reinterpret_cast<const half8*>(wp + (size_t)n * a.czp + kk);
+          half8 bgf = *reinterpret_cast<const half8*>(wg + (size_t)n * a.czp + kk);
+          accp = mfma_f16(af, bpf, accp);
+          accg = mfma_f16(af, bgf, accg);
         }
         const float bpv = bp[n], bgv = bg[n];
 #pragma unroll
@@ -262,18 +263,20 @@ struct OutputArgs {
   const float* b_z;
   const void* w_g;  // [czo][czp]
   const float* b_g;
+  const float* s_z;  // pair kernels
+  const float* s_g;
   void* out;
   int pair0;        // first pair of this block
   int pairs;        // pairs in this block
   int cz, ch, czp, chp;
   int residual;
   float eps;
+  float x_scale, h_scale;  // the pair kernels' x_hat of z and of the contracted values
 };
 
-// Loads 64 columns of a channel-major tile (xs[c][q]) and normalises them in
-// place (f32) or into an[q][c] (f16). Returns after a barrier.
-template <typename CT, bool F16MATH>
-__device__ __forceinline__ void normalize_tile(float* xs, int xpitch, CT* an, int apitch, int channels, int padded,
+// Normalises 64 columns of a channel-major tile (xs[c][q]) into an[q][c].
+// Returns after a barrier.
+__device__ __forceinline__ void normalize_tile(float* xs, int xpitch, half_t* an, int apitch, int channels, int padded,
                                                const float* w, const float* b, float eps, int tid) {
   float mean, rstd;
   column_stats(xs, xpitch, channels, eps, tid, mean, rstd);
@@ -281,41 +284,32 @@ __device__ __forceinline__ void normalize_tile(float* xs, int xpitch, CT* an, in
   __syncthreads();
   for (int c = part; c < padded; c += 4) {
     float v = c < channels ? (xs[c * xpitch + q] - mean) * rstd * w[c] + b[c] : 0.0f;
-    if (F16MATH) an[q * apitch + c] = (CT)v;
-    else xs[c * xpitch + q] = v;
+    an[q * apitch + c] = (half_t)v;
   }
   __syncthreads();
 }
 
 // acc[t] += A (64 x K from LDS) * W^T for the wave's column tiles.
-template <typename CT, bool F16MATH>
-__device__ __forceinline__ void tile_gemm(floatx16 (&acc)[2], const float* xs, int xpitch, const CT* an, int apitch,
-                                          const CT* W, int K, int czo, int lane, int wave) {
+__device__ __forceinline__ void tile_gemm(floatx16 (&acc)[2], const half_t* an, int apitch, const half_t* W, int K,
+                                          int czo, int lane, int wave) {
   const int rw = 32 * (wave & 1);
 #pragma unroll
   for (int t = 0; t < 2; t++) {
     const int j = (wave >> 1) + 2 * t;
     if (32 * j >= czo) continue;
     const int n = 32 * j + (lane & 31);
-    if constexpr (F16MATH) {
-      for (int k = 0; k < K; k += 16) {
-        const int kk = k + 8 * (lane >> 5);
-        half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
-        half8 bf = *reinterpret_cast<const half8*>(W + (size_t)n * K + kk);
-        acc[t] = mfma_f16(af, bf, acc[t]);
-      }
-    } else {
-      for (int k = 0; k < K; k += 2) {
-        const int kk = k + (lane >> 5);
-        acc[t] = mfma_f32(xs[kk * xpitch + rw + (lane & 31)], W[(size_t)n * K + kk], acc[t]);
-      }
+    for (int k = 0; k < K; k += 16) {
+      const int kk = k + 8 * (lane >> 5);
+      half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
+      half8 bf = *reinterpret_cast<const half8*>(W + (size_t)n * K + kk);
+      acc[t] = mfma_f16(af, bf, acc[t]);
     }
   }
 }
 
-template <typename ZT, typename OT, bool F16MATH>
+template <typename ZT, typename OT>
 __global__ __launch_bounds__(256) void tri_output_kernel(OutputArgs a) {
-  using CT = typename std::conditional<F16MATH, half_t, float>::type;
+  using CT = half_t;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int xpitch = kRows + 1;
   const int kmax = a.chp > a.czp ? a.chp : a.czp;
@@ -336,14 +330,13 @@ __global__ __launch_bounds__(256) void tri_output_kernel(OutputArgs a) {
     xs[c * xpitch + q] = v;
   }
   __syncthreads();
-  normalize_tile<CT, F16MATH>(xs, xpitch, an, apitch, a.ch, a.chp, a.ln_out_w, a.ln_out_b, a.eps, tid);
+  normalize_tile(xs, xpitch, an, apitch, a.ch, a.chp, a.ln_out_w, a.ln_out_b, a.eps, tid);
   floatx16 accz[2], accg[2];
 #pragma unroll
   for (int t = 0; t < 2; t++)
 #pragma unroll
     for (int v = 0; v < 16; v++) accz[t][v] = accg[t][v] = 0.0f;
-  tile_gemm<CT, F16MATH>(accz, xs, xpitch, an, apitch, reinterpret_cast<const CT*>(a.w_z), a.chp,
-                         (int)round_up(a.cz, 32), lane, wave);
+  tile_gemm(accz, an, apitch, reinterpret_cast<const CT*>(a.w_z), a.chp, (int)round_up(a.cz, 32), lane, wave);
   __syncthreads();
 
   // Phase 2: the same pairs of z, transposed to channel-major.
@@ -354,9 +347,8 @@ __global__ __launch_bounds__(256) void tri_output_kernel(OutputArgs a) {
     xs[c * xpitch + q] = v;
   }
   __syncthreads();
-  normalize_tile<CT, F16MATH>(xs, xpitch, an, apitch, a.cz, a.czp, a.ln_in_w, a.ln_in_b, a.eps, tid);
-  tile_gemm<CT, F16MATH>(accg, xs, xpitch, an, apitch, reinterpret_cast<const CT*>(a.w_g), a.czp,
-                         (int)round_up(a.cz, 32), lane, wave);
+  normalize_tile(xs, xpitch, an, apitch, a.cz, a.czp, a.ln_in_w, a.ln_in_b, a.eps, tid);
+  tile_gemm(accg, an, apitch, reinterpret_cast<const CT*>(a.w_g), a.czp, (int)round_up(a.cz, 32), lane, wave);
 
   OT* out = reinterpret_cast<OT*>(a.out);
   const int rw = 32 * (wave & 1);
@@ -375,6 +367,343 @@ __global__ __launch_bounds__(256) void tri_output_kernel(OutputArgs a) {
       if (a.residual) y += (float)out[at];
       out[at] = (OT)y;
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// f32 precision: both projections over pairs of f16
+// ---------------------------------------------------------------------------
+//
+// The f32 kernels before these ran the f32 MFMA, one 64-pair tile a workgroup
+// through all four (two) matrices, with the weights read element by element in
+// the middle of the MFMA chain: at L = 59, 55 of 256 CUs worked through 32k
+// cycles of MFMA each. Here a tile's columns are split over as many workgroups
+// as it takes to fill the chip (every one normalises the tile for itself), the
+// products are three f16 MFMAs of 32 cycles where eight f32 ones took 512, and
+// the weights come in fragment order, 1 KiB a load, one group of steps ahead.
+// Measured at c_z = c_h = 128, project / output: L = 59 83 / 63 us before,
+// 10.7 / 12.2 after; L = 256 365 / 157 before, 58 / 64 after.
+
+constexpr int kPairRows = 64;   // pairs a workgroup
+constexpr int kMaxSteps = 8;    // c_z <= 128 in steps of 16
+
+// Element (n, k) of a weight matrix of `steps` 16-wide steps, in the order the
+// lanes load fragments: [n / 32][step][plane][lane][8], lane = n % 32 +
+// 32 (k % 16 / 8). h is plane 0; l lies 512 halves on.
+__device__ __forceinline__ int64_t pair_fragment(int n, int k, int steps) {
+  return (((int64_t)(n >> 5) * steps + (k >> 4)) * 2 * 64 + (n & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
+}
+
+struct PairSources {
+  struct Matrix {
+    const float *w, *b, *gamma, *beta;  // w [rows][cols], the LayerNorm that feeds it
+    int rows, cols, padded, steps, x_exp;
+    half_t* out;
+    float *scale, *bias;
+  } m[6];
+};
+
+// One workgroup a (row, matrix): W' = W diag(gamma) in double times 2^e (the
+// largest element in [2^14, 2^15)), scale 2^-(x_exp + e), bias b + W beta;
+// padding rows and columns are zeros.
+__global__ __launch_bounds__(64) void tri_pair_prepare_kernel(PairSources src) {
+  const PairSources::Matrix& m = src.m[blockIdx.y];
+  const int n = blockIdx.x, lane = threadIdx.x;
+  if (n >= m.padded) return;
+  const bool in = n < m.rows;
+  const float* w = m.w + (int64_t)n * m.cols;
+  float most = 0.0f;
+  double offset = 0.0;
+  if (in)
+    for (int c = lane; c < m.cols; c += 64) {
+      most = fmaxf(most, fabsf((float)((double)w[c] * m.gamma[c])));
+      offset += (double)w[c] * m.beta[c];
+    }
+  for (int o = 32; o > 0; o >>= 1) {
+    most = fmaxf(most, __shfl_xor(most, o));
+    offset += __shfl_xor(offset, o);
+  }
+  const int e = pair_exponent(most);
+  for (int c = lane; c < 16 * m.steps; c += 64) {
+    half_t h, l;
+    pair_split(in && c < m.cols ? (float)ldexp((double)w[c] * m.gamma[c], e) : 0.0f, h, l);
+    const int64_t at = pair_fragment(n, c, m.steps);
+    m.out[at] = h;
+    m.out[at + 512] = l;
+  }
+  if (lane == 0) {
+    m.scale[n] = in ? ldexpf(1.0f, -(m.x_exp + e)) : 1.0f;
+    m.bias[n] = in ? (float)(m.b[n] + offset) : 0.0f;
+  }
+}
+
+// Four lanes normalise one row of z (row pointer, or null for zeros) and write
+// x_hat x_scale as pairs to `dst` (a pair row in LDS): lane `part` takes
+// channels 16 i + 4 part + [0, 4) of each block i.
+template <typename ZT>
+__device__ __forceinline__ void pair_normalize_row(const ZT* row, int cz, int steps, float eps, float x_scale, int part,
+                                                   bool vec, half_t* dst) {
+  float v[kMaxSteps][4];
+#pragma unroll
+  for (int i = 0; i < kMaxSteps; i++) {
+    const int c = 16 * i + 4 * part;
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[i][e] = 0.0f;
+    if (i >= steps || !row) continue;
+    if (vec) {
+      if (c < cz) {
+        typedef ZT zt4 __attribute__((ext_vector_type(4)));
+        const zt4 w = *reinterpret_cast<const zt4*>(row + c);
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[i][e] = (float)w[e];
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (c + e < cz) v[i][e] = (float)row[c + e];
+    }
+  }
+  float s = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kMaxSteps; i++) s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+  s += __shfl_xor(s, 1);
+  s += __shfl_xor(s, 2);
+  const float mean = s / (float)cz;
+  float d2 = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kMaxSteps; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      v[i][e] = 16 * i + 4 * part + e < cz ? v[i][e] - mean : 0.0f;
+      d2 += v[i][e] * v[i][e];
+    }
+  d2 += __shfl_xor(d2, 1);
+  d2 += __shfl_xor(d2, 2);
+  const float rstd = fast_rsqrt(d2 / (float)cz + eps) * x_scale;
+#pragma unroll
+  for (int i = 0; i < kMaxSteps; i++) {
+    if (i >= steps) continue;
+    half2v h0, l0, h1, l1;
+    pair_split2(v[i][0] * rstd, v[i][1] * rstd, h0, l0);
+    pair_split2(v[i][2] * rstd, v[i][3] * rstd, h1, l1);
+    half_t* p = dst + 32 * i + 4 * part;
+    *reinterpret_cast<half4*>(p) = half4{h0[0], h0[1], h1[0], h1[1]};
+    *reinterpret_cast<half4*>(p + 16) = half4{l0[0], l0[1], l1[0], l1[1]};
+  }
+}
+
+// Two steps' fragments (h, l of each) of one matrix block; `w` at the block's
+// first fragment, this lane's 16 bytes.
+struct PairFragments {
+  half8 h[2], l[2];
+  __device__ __forceinline__ void load(const half_t* w, int s) {
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      h[u] = *reinterpret_cast<const half8*>(w + (int64_t)(s + u) * 1024);
+      l[u] = *reinterpret_cast<const half8*>(w + (int64_t)(s + u) * 1024 + 512);
+    }
+  }
+};
+
+// LDS pair rows of 16 `steps` channels, padded by 16 bytes: 16 rows' fragments
+// then start on 16 different groups of four banks.
+__host__ __device__ constexpr int pair_pitch(int steps) { return 32 * steps + 8; }  // halves
+
+// Wave (rows 32 (w % 2).., operand w / 2) of a tile computes W x_hat^T for the
+// projection and the gate of 32 hidden channels: a lane ends with one pair and
+// 16 channels, so each store of a channel is 32 consecutive pairs.
+template <typename ZT> __global__ __launch_bounds__(256) void tri_project_pair_kernel(ProjectArgs a, int vec) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  half_t* an = reinterpret_cast<half_t*>(smem);
+  const int steps = a.czp / 16, pitch = pair_pitch(steps);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r0 = blockIdx.x * kPairRows;
+  const ZT* z = reinterpret_cast<const ZT*>(a.z);
+  auto pair_of = [&](int r) { return a.incoming ? (r % a.L) * a.L + r / a.L : r; };
+  const int o = wave >> 1, hi = lane >> 5;
+  const int r = r0 + 32 * (wave & 1) + (lane & 31);
+  const float keep = r < a.P ? a.mask[pair_of(r)] : 0.0f;
+  const int blocks = a.chp / 32;
+  const half_t* W = reinterpret_cast<const half_t*>(a.w_proj) + (int64_t)2 * o * a.chp * 2 * a.czp + 8 * lane;
+  const int64_t matrix = (int64_t)a.chp * 2 * a.czp, block = (int64_t)steps * 1024;
+  PairFragments fp, fg;
+  fp.load(W + blockIdx.y * block, 0);
+  fg.load(W + matrix + blockIdx.y * block, 0);
+  {
+    const int q = tid >> 2, rq = r0 + q;
+    pair_normalize_row<ZT>(rq < a.P ? z + (int64_t)pair_of(rq) * a.cz : nullptr, a.cz, steps, a.eps, a.x_scale, tid & 3,
+                           vec, an + q * pitch);
+  }
+  __syncthreads();
+  const half_t* xr = an + (32 * (wave & 1) + (lane & 31)) * pitch + 8 * hi;
+  for (int nb = blockIdx.y; nb < blocks; nb += gridDim.y) {
+    floatx16 p = {}, g = {};
+    for (int s = 0; s < steps; s += 2) {
+      const PairFragments cp = fp, cg = fg;
+      // The next two steps, or the next block's first.
+      const int ns = s + 2 < steps ? s + 2 : 0, nn = min(s + 2 < steps ? nb : nb + (int)gridDim.y, blocks - 1);
+      fp.load(W + nn * block, ns);
+      fg.load(W + matrix + nn * block, ns);
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const half8 xh = *reinterpret_cast<const half8*>(xr + 32 * (s + u));
+        const half8 xl = *reinterpret_cast<const half8*>(xr + 32 * (s + u) + 16);
+        p = mfma_f16(cp.h[u], xh, p);
+        g = mfma_f16(cg.h[u], xh, g);
+        p = mfma_f16(cp.h[u], xl, p);
+        g = mfma_f16(cg.h[u], xl, g);
+        p = mfma_f16(cp.l[u], xh, p);
+        g = mfma_f16(cg.l[u], xh, g);
+      }
+    }
+    const int c0 = 32 * nb + 4 * hi;
+    const float *sp = a.s_proj + 2 * o * a.chp, *bp = a.b_proj + 2 * o * a.chp;
+    float* out = reinterpret_cast<float*>(o == 0 ? a.out_a : a.out_b) + r;
+#pragma unroll
+    for (int v4 = 0; v4 < 4; v4++) {
+      const int c = c0 + 8 * v4;
+      const float4 s1 = *reinterpret_cast<const float4*>(sp + c), b1 = *reinterpret_cast<const float4*>(bp + c);
+      const float4 s2 = *reinterpret_cast<const float4*>(sp + a.chp + c), b2 = *reinterpret_cast<const float4*>(bp + a.chp + c);
+      const float S1[4] = {s1.x, s1.y, s1.z, s1.w}, B1[4] = {b1.x, b1.y, b1.z, b1.w};
+      const float S2[4] = {s2.x, s2.y, s2.z, s2.w}, B2[4] = {b2.x, b2.y, b2.z, b2.w};
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float y = keep * fmaf(p[4 * v4 + e], S1[e], B1[e]) * sigmoidf_(fmaf(g[4 * v4 + e], S2[e], B2[e]));
+        if (c + e < a.ch && r < a.P) out[(int64_t)(c + e) * a.cstride] = y;
+      }
+    }
+  }
+}
+
+// A tile of 64 pairs of the output: waves 0 and 1 (rows 32 w..) multiply the
+// normalised contraction by linearZ, waves 2 and 3 the normalised z by linearG;
+// the gates cross through LDS. A lane ends with one channel and 16 pairs, so
+// each store of a pair is 32 consecutive channels.
+template <typename ZT, typename OT> __global__ __launch_bounds__(256) void tri_output_pair_kernel(OutputArgs a, int vec) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int zsteps = a.czp / 16, hsteps = a.chp / 16, zpitch = pair_pitch(zsteps), hpitch = pair_pitch(hsteps);
+  half_t* hn = reinterpret_cast<half_t*>(smem);
+  half_t* zn = hn + kPairRows * hpitch;
+  float* red = reinterpret_cast<float*>(zn + kPairRows * zpitch);  // [2][4][64], then the gates [2][32][32]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q0 = blockIdx.x * kPairRows;
+  const ZT* z = reinterpret_cast<const ZT*>(a.z);
+  const float* X = reinterpret_cast<const float*>(a.contracted);
+  const bool gate = wave >= 2;
+  const int rw = 32 * (wave & 1), blocks = (a.cz + 31) / 32;
+  const int steps = gate ? zsteps : hsteps;
+  const half_t* W = reinterpret_cast<const half_t*>(gate ? a.w_g : a.w_z) + 8 * lane;
+  const int64_t block = (int64_t)steps * 1024;
+  PairFragments f;
+  f.load(W + blockIdx.y * block, 0);
+
+  // The contraction's LayerNorm: lane = pair, wave w the channels
+  // [w chp / 4, (w + 1) chp / 4), in groups of eight (chp <= 256).
+  // Channels past ch and pairs past the last repeat one that is there (the
+  // pairs are not stored, the channels are zeroed against `live`). The empty
+  // asm keeps one pointer and one bound in vector registers: 64 of either would
+  // not fit the scalar ones.
+  const int groups = a.chp / 32, cw = wave * (a.chp / 4);
+  float x[8][8];
+  const float* xp = X + (int64_t)min(cw, a.ch - 1) * a.bstride + min(q0 + lane, a.pairs - 1);
+  int live = a.ch - cw;
+  asm("" : "+v"(live));
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    if (i < groups) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float w = *xp;
+        xp += cw + 8 * i + e + 1 < a.ch ? a.bstride : 0;
+        asm("" : "+v"(xp));
+        x[i][e] = 8 * i + e < live ? w : 0.0f;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; e++) x[i][e] = 0.0f;
+    }
+  }
+  {
+    const int q = tid >> 2;
+    pair_normalize_row<ZT>(q0 + q < a.pairs ? z + (int64_t)(a.pair0 + q0 + q) * a.cz : nullptr, a.cz, zsteps, a.eps,
+                           a.x_scale, tid & 3, vec, zn + q * zpitch);
+  }
+  float s = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) s += x[i][e];
+  red[wave * 64 + lane] = s;
+  __syncthreads();
+  const float mean = ((red[lane] + red[64 + lane]) + (red[128 + lane] + red[192 + lane])) / (float)a.ch;
+  float d2 = 0.0f;
+  const int lives = min(live, 8 * groups);
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      x[i][e] = 8 * i + e < lives ? x[i][e] - mean : 0.0f;
+      d2 += x[i][e] * x[i][e];
+    }
+  red[256 + wave * 64 + lane] = d2;
+  __syncthreads();
+  d2 = (red[256 + lane] + red[320 + lane]) + (red[384 + lane] + red[448 + lane]);
+  const float rstd = fast_rsqrt(d2 / (float)a.ch + a.eps) * a.h_scale;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    if (i >= groups) continue;
+    half8 h, l;
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      half2v h2, l2;
+      pair_split2(x[i][e] * rstd, x[i][e + 1] * rstd, h2, l2);
+      h[e] = h2[0], h[e + 1] = h2[1], l[e] = l2[0], l[e + 1] = l2[1];
+    }
+    half_t* p = hn + lane * hpitch + pair_index(cw + 8 * i);
+    *reinterpret_cast<half8*>(p) = h;
+    *reinterpret_cast<half8*>(p + 16) = l;
+  }
+  __syncthreads();
+
+  const half_t* xr = (gate ? zn + (rw + (lane & 31)) * zpitch : hn + (rw + (lane & 31)) * hpitch) + 8 * (lane >> 5);
+  float* gates = red + (wave & 1) * 1024;
+  OT* out = reinterpret_cast<OT*>(a.out);
+  for (int nb = blockIdx.y; nb < blocks; nb += gridDim.y) {
+    floatx16 acc = {};
+    for (int k = 0; k < steps; k += 2) {
+      const PairFragments c = f;
+      const int nk = k + 2 < steps ? k + 2 : 0, nn = min(k + 2 < steps ? nb : nb + (int)gridDim.y, blocks - 1);
+      f.load(W + nn * block, nk);
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const half8 xh = *reinterpret_cast<const half8*>(xr + 32 * (k + u));
+        const half8 xl = *reinterpret_cast<const half8*>(xr + 32 * (k + u) + 16);
+        acc = mfma_f16(xh, c.h[u], acc);
+        acc = mfma_f16(xh, c.l[u], acc);
+        acc = mfma_f16(xl, c.h[u], acc);
+      }
+    }
+    const int n = 32 * nb + (lane & 31);
+    const float sc = (gate ? a.s_g : a.s_z)[n], bi = (gate ? a.b_g : a.b_z)[n];
+    if (gate) {
+#pragma unroll
+      for (int v = 0; v < 16; v++) gates[v * 64 + lane] = sigmoidf_(fmaf(acc[v], sc, bi));
+    }
+    __syncthreads();
+    if (!gate) {
+      float y[16];
+#pragma unroll
+      for (int v = 0; v < 16; v++) y[v] = fmaf(acc[v], sc, bi) * gates[v * 64 + lane];
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const int q = q0 + rw + mfma_row(v, lane);
+        if (n < a.cz && q < a.pairs) {
+          const int64_t at = (int64_t)(a.pair0 + q) * a.cz + n;
+          out[at] = (OT)(a.residual ? y[v] + (float)out[at] : y[v]);
+        }
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -456,34 +785,61 @@ int validate(const afhip_triangle_desc* d) {
   return AFHIP_OK;
 }
 
-template <typename ZT, bool F16MATH>
-int launch_project(const ProjectArgs& pa, size_t shared, hipStream_t s) {
-  if (int st = allow_lds((const void*)tri_project_kernel<ZT, F16MATH>, shared)) return st;
-  return launch("triangle.project", tri_project_kernel<ZT, F16MATH>, dim3((unsigned)ceil_div(pa.P, kRows)),
-                dim3(256), shared, s, pa);
+template <typename ZT> int launch_project(const ProjectArgs& pa, size_t shared, hipStream_t s) {
+  if (int st = allow_lds((const void*)tri_project_kernel<ZT>, shared)) return st;
+  return launch("triangle.project", tri_project_kernel<ZT>, dim3((unsigned)ceil_div(pa.P, kRows)), dim3(256), shared, s,
+                pa);
 }
 
-template <typename ZT, typename OT, bool F16MATH>
-int launch_output(const OutputArgs& oa, size_t shared, hipStream_t s) {
-  if (int st = allow_lds((const void*)tri_output_kernel<ZT, OT, F16MATH>, shared)) return st;
-  return launch("triangle.output", tri_output_kernel<ZT, OT, F16MATH>, dim3((unsigned)ceil_div(oa.pairs, kRows)),
-                dim3(256), shared, s, oa);
+template <typename ZT, typename OT> int launch_output(const OutputArgs& oa, size_t shared, hipStream_t s) {
+  if (int st = allow_lds((const void*)tri_output_kernel<ZT, OT>, shared)) return st;
+  return launch("triangle.output", tri_output_kernel<ZT, OT>, dim3((unsigned)ceil_div(oa.pairs, kRows)), dim3(256),
+                shared, s, oa);
 }
 
-template <bool F16MATH>
-int dispatch_project(int zd, const ProjectArgs& pa, size_t shared, hipStream_t s) {
-  if (zd == AFHIP_F32) return launch_project<float, F16MATH>(pa, shared, s);
-  return launch_project<half_t, F16MATH>(pa, shared, s);
+// How many workgroups share a tile's column blocks: enough for two a CU, as
+// each of them normalises the tile for itself.
+unsigned column_splits(int64_t tiles, int blocks) {
+  const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  return (unsigned)std::max<int64_t>(1, std::min<int64_t>(blocks, 2 * cus / tiles));
 }
 
-template <bool F16MATH>
-int dispatch_output(int zd, int od, const OutputArgs& oa, size_t shared, hipStream_t s) {
-  if (zd == AFHIP_F32) {
-    if (od == AFHIP_F32) return launch_output<float, float, F16MATH>(oa, shared, s);
-    return launch_output<float, half_t, F16MATH>(oa, shared, s);
-  }
-  if (od == AFHIP_F32) return launch_output<half_t, float, F16MATH>(oa, shared, s);
-  return launch_output<half_t, half_t, F16MATH>(oa, shared, s);
+bool rows_on_four(const void* z, int cz, size_t es) {
+  return cz % 4 == 0 && (reinterpret_cast<uintptr_t>(z) & (4 * es - 1)) == 0;
+}
+
+template <typename ZT> int launch_project_pair(const ProjectArgs& pa, hipStream_t s) {
+  const int64_t tiles = ceil_div(pa.P, kPairRows);
+  const size_t shared = (size_t)kPairRows * pair_pitch(pa.czp / 16) * 2;
+  auto k = tri_project_pair_kernel<ZT>;
+  if (int st = allow_lds((const void*)k, shared)) return st;
+  return launch("triangle.project", k, dim3((unsigned)tiles, column_splits(tiles, pa.chp / 32)), dim3(256), shared, s, pa,
+                (int)rows_on_four(pa.z, pa.cz, sizeof(ZT)));
+}
+
+template <typename ZT, typename OT> int launch_output_pair(const OutputArgs& oa, hipStream_t s) {
+  const int64_t tiles = ceil_div(oa.pairs, kPairRows);
+  const size_t shared =
+      (size_t)kPairRows * (pair_pitch(oa.czp / 16) + pair_pitch(oa.chp / 16)) * 2 + 2 * 32 * 32 * 4;
+  auto k = tri_output_pair_kernel<ZT, OT>;
+  if (int st = allow_lds((const void*)k, shared)) return st;
+  return launch("triangle.output", k, dim3((unsigned)tiles, column_splits(tiles, (oa.cz + 31) / 32)), dim3(256), shared,
+                s, oa, (int)rows_on_four(oa.z, oa.cz, sizeof(ZT)));
+}
+
+int dispatch_project(bool f16, int zd, const ProjectArgs& pa, size_t shared, hipStream_t s) {
+  if (!f16) return zd == AFHIP_F32 ? launch_project_pair<float>(pa, s) : launch_project_pair<half_t>(pa, s);
+  return zd == AFHIP_F32 ? launch_project<float>(pa, shared, s) : launch_project<half_t>(pa, shared, s);
+}
+
+template <typename ZT> int dispatch_output_to(bool f16, int od, const OutputArgs& oa, size_t shared, hipStream_t s) {
+  if (!f16) return od == AFHIP_F32 ? launch_output_pair<ZT, float>(oa, s) : launch_output_pair<ZT, half_t>(oa, s);
+  return od == AFHIP_F32 ? launch_output<ZT, float>(oa, shared, s) : launch_output<ZT, half_t>(oa, shared, s);
+}
+
+int dispatch_output(bool f16, int zd, int od, const OutputArgs& oa, size_t shared, hipStream_t s) {
+  return zd == AFHIP_F32 ? dispatch_output_to<float>(f16, od, oa, shared, s)
+                         : dispatch_output_to<half_t>(f16, od, oa, shared, s);
 }
 
 }  // namespace
@@ -531,11 +887,25 @@ int afhip_triangle_prepare_weights(const afhip_triangle_desc* desc, const float*
   o[0] = 0;
   for (int i = 0; i < 16; i++) o[i + 1] = o[i] + sizes[i];
   char* base = (char*)prepared;
-  const bool f16 = d.precision == AFHIP_PRECISION_F16;
-  size_t es = f16 ? 2 : 4;
+  if (d.precision == AFHIP_PRECISION_F32) {
+    // ORDER indices as below; the pair kernels need nothing else.
+    PairSources src{};
+    auto matrix = [&](int at, int index, int norm, int rows, int cols, int padded, int steps, size_t out, size_t scale,
+                      size_t bias) {
+      src.m[at] = {packed + o[index], packed + o[index + 1], packed + o[norm], packed + o[norm + 1], rows, cols,
+                   padded, steps, pair_norm_exponent(cols), (half_t*)(base + out), (float*)(base + scale),
+                   (float*)(base + bias)};
+    };
+    for (int k = 0; k < 4; k++)
+      matrix(k, 2 + 2 * k, 0, ch, cz, w.chp, w.czp / 16, w.w_proj + 4 * (size_t)k * w.chp * w.czp,
+             w.s_proj + 4 * (size_t)k * w.chp, w.b_proj + 4 * (size_t)k * w.chp);
+    matrix(4, 12, 10, cz, ch, w.czo, w.chp / 16, w.w_z, w.s_z, w.b_z);
+    matrix(5, 14, 0, cz, cz, w.czo, w.czp / 16, w.w_g, w.s_g, w.b_g);
+    return launch("tri_prepare", tri_pair_prepare_kernel, dim3((unsigned)std::max(w.chp, w.czo), 6), dim3(64), 0, st, src);
+  }
+  const size_t es = 2;
   auto mat = [&](int index, int rows, int cols, size_t dst, int prow, int pcol) {
-    return f16 ? pad_matrix<half_t>(packed + o[index], rows, cols, base + dst, prow, pcol, st)
-               : pad_matrix<float>(packed + o[index], rows, cols, base + dst, prow, pcol, st);
+    return pad_matrix<half_t>(packed + o[index], rows, cols, base + dst, prow, pcol, st);
   };
   int s;
   if ((s = pad_vector(packed + o[0], cz, base + w.ln_in_w, cz, st))) return s;
@@ -595,6 +965,8 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
   pa.ln_b = (const float*)(wb + w.ln_in_b);
   pa.w_proj = wb + w.w_proj;
   pa.b_proj = (const float*)(wb + w.b_proj);
+  pa.s_proj = (const float*)(wb + w.s_proj);
+  pa.x_scale = ldexpf(1.0f, pair_norm_exponent(d.c_z));
   pa.out_a = wsb + ws.op_a;
   pa.out_b = wsb + ws.op_b;
   pa.cstride = ws.cstride;
@@ -625,9 +997,9 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
     fa.eps = d.epsilon;
     s = launch_triangle_project_f16(fa, d.pair_dtype, st);
   } else {
-    size_t psh = round_up((int64_t)w.czp * (kRows + 1) * 4, 16) +
-                 (f16 ? round_up((int64_t)kRows * (w.czp + 8) * 2, 16) : 0) + (size_t)64 * (kRows + 8) * (f16 ? 2 : 4);
-    s = f16 ? dispatch_project<true>(d.pair_dtype, pa, psh, st) : dispatch_project<false>(d.pair_dtype, pa, psh, st);
+    const size_t psh = round_up((int64_t)w.czp * (kRows + 1) * 4, 16) +
+                       round_up((int64_t)kRows * (w.czp + 8) * 2, 16) + (size_t)64 * (kRows + 8) * 2;
+    s = dispatch_project(f16, d.pair_dtype, pa, psh, st);
   }
   if (s) return s;
 
@@ -637,7 +1009,7 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
   const size_t es = f16 ? 2 : 4;
   GemmTypes types{d.precision, f16 ? AFHIP_F16 : AFHIP_F32, f16 ? AFHIP_F16 : AFHIP_F32, f16 ? AFHIP_F16 : AFHIP_F32};
   const int kmax = std::max(w.chp, w.czp);
-  size_t osh = round_up((int64_t)kmax * (kRows + 1) * 4, 16) + (f16 ? (size_t)kRows * (kmax + 8) * 2 : 0);
+  const size_t osh = round_up((int64_t)kmax * (kRows + 1) * 4, 16) + (size_t)kRows * (kmax + 8) * 2;
   for (int i0 = 0; i0 < L; i0 += ws.block_rows) {
     const int count = std::min(ws.block_rows, L - i0);
     GemmArgs g;
@@ -669,6 +1041,10 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
     oa.b_z = (const float*)(wb + w.b_z);
     oa.w_g = wb + w.w_g;
     oa.b_g = (const float*)(wb + w.b_g);
+    oa.s_z = (const float*)(wb + w.s_z);
+    oa.s_g = (const float*)(wb + w.s_g);
+    oa.x_scale = pa.x_scale;
+    oa.h_scale = ldexpf(1.0f, pair_norm_exponent(d.c_hidden));
     oa.out = out;
     oa.pair0 = i0 * L;
     oa.pairs = count * L;
@@ -694,8 +1070,7 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
       fo.eps = d.epsilon;
       s = launch_triangle_output_f16(fo, d.pair_dtype, d.out_dtype, st);
     } else {
-      s = f16 ? dispatch_output<true>(d.pair_dtype, d.out_dtype, oa, osh, st)
-              : dispatch_output<false>(d.pair_dtype, d.out_dtype, oa, osh, st);
+      s = dispatch_output(f16, d.pair_dtype, d.out_dtype, oa, osh, st);
     }
     if (s) return s;
   }

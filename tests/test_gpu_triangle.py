@@ -175,3 +175,46 @@ def test_invalid_input_raises_range_error(dev):
     inp["z"] = inp["z"].reshape(-1)[1:]
     with pytest.raises(_lib.RangeError, match="z has"):
         gpu_class("outgoing")().run(inp)
+
+
+@pytest.mark.parametrize("direction", ["outgoing", "incoming"])
+@pytest.mark.parametrize("length,cz,ch,pair_dtype,out_dtype,residual,shift", [
+    (1, 4, 8, "f32", "f32", False, 0), (8, 31, 33, "f32", "f32", True, 1), (9, 128, 256, "f16", "f32", False, 0),
+    (33, 100, 72, "f32", "f16", True, 1), (23, 64, 224, "f16", "f32", True, 3), (90, 128, 128, "f32", "f32", False, 0)])
+def test_f32_pair_kernels(dev, direction, length, cz, ch, pair_dtype, out_dtype, residual, shift):
+    # f32 precision's projection and output kernels over pairs of f16: ragged
+    # tiles of 64 pairs, channels short of their 32-wide padding, one to four
+    # column splits, z and the output off 16-byte alignment (shift elements),
+    # f16 storage, the residual. The input LayerNorm's scales and the columns of
+    # the weights it feeds carry factors of 1e-6 to 1e6 that cancel, as any
+    # weight may. f32 out: the f32 bound; f16 out: half an ulp besides.
+    import torch
+
+    from afhip import triangle
+
+    inp = ref.deterministic_triangle_input(length, cz, ch, seed=length + ch)
+    w = {k: np.array(v, np.float64) for k, v in inp["weights"].items()}
+    fc, fh = 10.0 ** ref.uniform(61, (cz,), -6, 6), 10.0 ** ref.uniform(62, (ch,), -6, 6)
+    for name, factor in (("layerNormIn", fc), ("layerNormOut", fh)):
+        w[name + "Weight"] *= factor
+        w[name + "Bias"] *= factor
+    for name in ("AP", "AG", "BP", "BG", "G"):
+        w[f"linear{name}Weight"] /= fc
+    w["linearZWeight"] /= fh
+    w = {k: v.astype(np.float32) for k, v in w.items()}
+    z = ref.round_f16(inp["z"])
+    old = ref.round_f16(ref.normal(63, z.shape))
+    expect = ref.triangle(direction, z, inp["mask"], w) + (old if residual else 0)
+    op = triangle.TriangleMultiplication(length, cz, ch, direction=direction, pair_dtype=pair_dtype,
+                                         out_dtype=out_dtype, residual=residual)
+    op.prepare(w)
+    tdt = {"f32": torch.float32, "f16": torch.float16}
+
+    def place(a, dtype):
+        flat = torch.zeros(a.size + shift, dtype=tdt[dtype], device=dev)
+        flat[shift:] = torch.from_numpy(np.ascontiguousarray(a)).to(dev).reshape(-1)
+        return flat[shift:].reshape(a.shape)
+
+    mask = torch.from_numpy(np.ascontiguousarray(inp["mask"], np.float32)).to(dev)
+    out = op(place(z, pair_dtype), mask, out=place(old, out_dtype)).float().cpu().numpy()
+    assert np.abs(out - expect).max() <= (1e-5 if out_dtype == "f32" else 1e-5 + 2.0 ** -11) * np.abs(expect).max()
