@@ -1292,6 +1292,193 @@ __global__ __launch_bounds__(kFlashThreads) void attention_flash_f16_kernel(Flas
   }
 }
 
+// f16 at head dimension 8 with heads in fours (the extra-MSA stack's 8 heads of
+// 8): a wave takes 32 queries of four heads of one batch entry, whose 32
+// channels are one 64-byte piece of a row, and needs no other wave. The heads'
+// S^T = K_h Q_h^T are one 32x32x8 MFMA each, their softmax the kernel above's,
+// step for step; in O^T += V^T P_h^T the V^T fragment keeps head h's eight
+// channels and is zero in the others, so one accumulator holds the four heads
+// (head h in registers 4 h .. 4 h + 3). K comes from global memory in the
+// MFMA's layout, V by DMA into two LDS buffers of the wave's own for the
+// transposing reads, both one block ahead; keys past the end read as zeros.
+//
+// The kernel above pads each head to 32 channels and shares tiles between eight
+// waves behind a barrier a block: over few keys it is one long chain of load,
+// barrier, compute, barrier. Measured, 8 heads of 8 with a pair bias: 1,024
+// sequences x 59 residues 47 -> 22 us, x 150 152 -> 86.
+constexpr int kH8Waves = 4;
+constexpr int kH8Buffer = 32 * 64;  // bytes of a block's V
+
+template <bool BIAS>
+__global__ __launch_bounds__(64 * kH8Waves, 4) void attention_flash_heads8_kernel(FlashArgs a, int qtiles,
+                                                                                  int64_t tiles, int64_t per_xcd) {
+  __shared__ __attribute__((aligned(1024))) unsigned char vbuf[kH8Waves][2][kH8Buffer];
+  const int lane = threadIdx.x & 63, col = lane & 31, hi = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t group = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const int64_t t = group * kH8Waves + wave;
+  if (t >= tiles) return;  // the whole wave; there is no barrier
+  const int hgroups = a.H / 4;
+  const int q0 = 32 * (int)(t % qtiles);
+  const int hg = (int)(t / qtiles % hgroups);
+  const int64_t b = t / qtiles / hgroups;
+  const int Q = a.Q;
+  const int64_t ld4 = 4 * (int64_t)a.C;
+  const half_t* rows = reinterpret_cast<const half_t*>(a.qkvg) + b * Q * ld4 + 32 * hg;
+  const half_t* keys = rows + a.C;
+  // V from the entry's first row to the end of its last one's 64 bytes.
+  const int32x4_t rv = make_rsrc(rows + 2 * a.C, (uint32_t)(((int64_t)(Q - 1) * ld4 + 32) * 2));
+  const uint32_t row_bytes = (uint32_t)ld4 * 2;
+  const uint32_t voff = (uint32_t)(lane >> 2) * row_bytes + 16 * (lane & 3);  // key lane / 4, chunk lane % 4
+  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(&vbuf[wave][0][0]);
+  auto fetch_v = [&](int k0, int buf) {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      dma16(rv, lds0 + buf * kH8Buffer + 1024 * i, voff + (uint32_t)(k0 + 16 * i) * row_bytes);
+  };
+  half4 qf[4], kf[4];
+  half_t code;
+  auto load_keys = [&](int k0) {  // keys past the end repeat the last (their codes are -inf)
+    const half_t* p = keys + (int64_t)min(k0 + col, Q - 1) * ld4 + 4 * hi;
+#pragma unroll
+    for (int h = 0; h < 4; h++) kf[h] = *reinterpret_cast<const half4*>(p + 8 * h);
+    code = a.key_mask[b * a.code_stride + min(k0, a.code_stride - 32) + col];
+  };
+  const int myq = q0 + col, qc = min(myq, Q - 1);
+  {
+    const half_t* p = rows + (int64_t)qc * ld4 + 4 * hi;
+#pragma unroll
+    for (int h = 0; h < 4; h++) qf[h] = *reinterpret_cast<const half4*>(p + 8 * h);
+  }
+  load_keys(0);
+  fetch_v(0, 0);
+
+  floatx16 o = {};
+  float run_sum[4] = {}, m[4] = {}, lo[4], up[4];
+#pragma unroll
+  for (int h = 0; h < 4; h++) lo[h] = -kLogitBound, up[h] = kLogitBound;
+  const half_t one = (half_t)1.0f;
+  // The transposing reads' addresses, as in the kernel above.
+  const int tr_key = 4 * hi + ((lane & 15) >> 2), tr_ch = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+
+  for (int k0 = 0, buf = 0; k0 < Q; k0 += 32, buf ^= 1) {
+    // This block's V and K (and every read before them) have landed, and the
+    // other buffer's reads are done: it takes the next block's V.
+    wait_vmcnt<0>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    fetch_v(k0 + 32, buf ^ 1);
+    half4 kc[4];
+#pragma unroll
+    for (int h = 0; h < 4; h++) kc[h] = kf[h];
+    const half4 am = hi ? half4{} : half4{code, one, (half_t)0.0f, (half_t)0.0f};
+    load_keys(k0 + 32);
+    half8 vt[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const unsigned char* vp = &vbuf[wave][buf][(16 * s + tr_key) * 64 + 2 * tr_ch];
+      const short4v x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)vp);
+      const short4v y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)(vp + 8 * 64));
+      vt[s] = __builtin_bit_cast(half8, short8v{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]});
+    }
+    const bool first = k0 == 0, last = k0 + 32 > Q;
+#pragma unroll
+    for (int h = 0; h < 4; h++) {
+      floatx16 sc = {};
+      if constexpr (BIAS) {
+        const float* row = a.bias + ((int64_t)(4 * hg + h) * Q + qc) * a.stride;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const float4 w = *reinterpret_cast<const float4*>(row + min(k0 + 8 * g + 4 * hi, a.stride - 4));
+          sc[4 * g] = w.x, sc[4 * g + 1] = w.y, sc[4 * g + 2] = w.z, sc[4 * g + 3] = w.w;
+        }
+      }
+      sc = __builtin_amdgcn_mfma_f32_32x32x8f16(kc[h], qf[h], sc, 0, 0, 0);
+      const half4 bm_frag = hi ? half4{} : half4{(half_t)kMaskScale, (half_t)(-m[h]), (half_t)0.0f, (half_t)0.0f};
+      sc = __builtin_amdgcn_mfma_f32_32x32x8f16(am, bm_frag, sc, 0, 0, 0);
+      float x[16];
+#pragma unroll
+      for (int v = 0; v < 16; v++) x[v] = sc[v];
+      auto drop_past_end = [&]() {
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+          if (k0 + 8 * (v >> 2) + 4 * hi + (v & 3) >= Q) x[v] = -INFINITY;
+      };
+      if (last) drop_past_end();
+      float bm = x[0];
+#pragma unroll
+      for (int v = 1; v < 16; v++) bm = fmaxf(bm, x[v]);
+      if (__builtin_amdgcn_ballot_w64(bm > up[h] || bm < lo[h] + kClampReach)) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) x[v] = __builtin_amdgcn_fmed3f(x[v], lo[h], up[h]);
+        if (last) drop_past_end();
+        bm = __builtin_amdgcn_fmed3f(bm, lo[h], up[h]);
+      }
+      if (first || __builtin_amdgcn_ballot_w64(bm > kSlack)) {
+        const float pm = fmaxf(bm, __shfl_xor(bm, 32));
+        const float want = first ? pm : m[h] + fmaxf(pm, 0.0f);
+        const float mn = (float)(half_t)want;
+        const float delta = mn - m[h];
+#pragma unroll
+        for (int v = 0; v < 16; v++) x[v] -= delta;
+        lo[h] -= delta;
+        up[h] -= delta;
+        if (!first) {
+          const float f = __builtin_amdgcn_exp2f(-delta);
+          run_sum[h] *= f;
+#pragma unroll
+          for (int i = 0; i < 4; i++) o[4 * h + i] *= f;
+        }
+        m[h] = mn;
+      }
+      half8 pf[2];
+#pragma unroll
+      for (int v = 0; v < 16; v += 2) {
+        const half2v pp = half2v{(half_t)__builtin_amdgcn_exp2f(x[v]), (half_t)__builtin_amdgcn_exp2f(x[v + 1])};
+        run_sum[h] = __builtin_amdgcn_fdot2(pp, half2v{one, one}, run_sum[h], false);
+        pf[v >> 3][v & 7] = pp[0];
+        pf[v >> 3][(v & 7) + 1] = pp[1];
+      }
+      // Head h's channels of V^T; the other heads' rows add zeros.
+      const bool mine = (col >> 3) == h;
+#pragma unroll
+      for (int s = 0; s < 2; s++) o = mfma_f16(mine ? vt[s] : half8{}, pf[s], o);
+    }
+  }
+  wait_vmcnt<0>();  // the fetch past the last block lands before the wave ends
+#pragma unroll
+  for (int h = 0; h < 4; h++) run_sum[h] += __shfl_xor(run_sum[h], 32);
+  if (myq >= Q) return;
+  const half_t* gr = rows + (int64_t)myq * ld4 + 3 * a.C + 4 * hi;
+  const int64_t src = a.transpose ? (int64_t)myq * a.B + b : b * Q + myq;
+  half_t* out = reinterpret_cast<half_t*>(a.weighted) + src * a.C + 32 * hg + 4 * hi;
+  half4 gv[4];
+#pragma unroll
+  for (int h = 0; h < 4; h++) gv[h] = *reinterpret_cast<const half4*>(gr + 8 * h);
+#pragma unroll
+  for (int h = 0; h < 4; h++) {
+    const float inv = 1.0f / run_sum[h];
+    half4 r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) r[i] = (half_t)(o[4 * h + i] * inv * (float)gv[h][i]);
+    *reinterpret_cast<half4*>(out + 8 * h) = r;
+  }
+}
+
+// V's resource spans the entry's rows and the fetch ahead 63 more: 32-bit offsets.
+bool heads8_eligible(const afhip_attention_desc& d) {
+  return fast_path(d) && d.channels / d.heads == 8 && d.heads % 4 == 0 &&
+         ((int64_t)d.queries + 64) * 8 * d.channels < (int64_t)kOutOfRange;
+}
+
+int launch_flash_heads8(const FlashArgs& fa, hipStream_t st) {
+  const int qtiles = (int)ceil_div(fa.Q, 32);
+  const int64_t tiles = (int64_t)fa.B * (fa.H / 4) * qtiles, per_xcd = ceil_div(tiles, 8 * kH8Waves);
+  AFHIP_REQUIRE(per_xcd < ((int64_t)1 << 28), "attention grid too large");
+  auto k = fa.bias ? attention_flash_heads8_kernel<true> : attention_flash_heads8_kernel<false>;
+  return launch("attention.flash", k, dim3((unsigned)(8 * per_xcd)), dim3(64 * kH8Waves), 0, st, fa, qtiles, tiles,
+                per_xcd);
+}
+
 // The same attention at head dimension 32 (every Evoformer attention), with
 // more independent work a wave and no staging registers:
 //  - a wave takes 64 queries of one (b, h), as two 32-query tiles against
@@ -1808,7 +1995,13 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
       g.scale = (const float*)(wp + w.s_proj);
       g.flags |= AFHIP_EPILOGUE_SCALE;
       if ((s = run_gemm_pairs(g, AFHIP_F32, "attention.project", st))) return s;
-    } else if ((s = run_gemm(g, t, select_variant(t, g.M, g.N, g.K, 1), "attention.project", st))) {
+    } else if (const afhip_variant v = select_variant(t, g.M, g.N, g.K, 1);
+               v.source == 0 && C == 64 && g.M >= 16384 && stream_eligible(g, t)) {
+      // 256 columns are few for STREAM's rule (heuristic_variant), but a K of 64 is all
+      // output: 60416 x 64 x 256 on MI355X 14.5 us against 26 on LDS_DMA tiles,
+      // 153600 rows 20 against 56.
+      if ((s = run_gemm_stream(g, t, "attention.project", st))) return s;
+    } else if ((s = run_gemm(g, t, v, "attention.project", st))) {
       return s;
     }
   }
@@ -1843,6 +2036,8 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
         s = launch("attention.flash", k, dim3((unsigned)groups), dim3(kF2Threads), kF2Buffers * kF2BufNoBias, st,
                    fa);
       }
+    } else if (heads8_eligible(d)) {
+      s = launch_flash_heads8(fa, st);
     } else if (fast) {
       const int64_t groups = ceil_div(B, kFlashBatch) * H * ceil_div(Q, 32 * kFlashQueryWaves);
       AFHIP_REQUIRE(groups < ((int64_t)1 << 31), "attention grid too large");

@@ -400,3 +400,26 @@ def test_f32_pairs_attention(dev, name, S, L, residual, shift, C, H):
              out=to(old) if residual else None)
     got = out.cpu().numpy().reshape(-1)
     assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("C,H", [(32, 4), (64, 8), (96, 12)])
+@pytest.mark.parametrize("name,S,L,scale", [("msa_row", 3, 1, 1), ("msa_row", 2, 33, 12), ("msa_column", 31, 3, 4),
+                                            ("msa_column", 97, 2, 4), ("triangle_end", 0, 64, 1),
+                                            ("triangle_start", 0, 65, 12)])
+def test_f16_four_heads_of_eight(dev, name, S, L, scale, C, H):
+    # Head dimension 8 with heads in fours: ragged blocks of 32 queries and
+    # keys, fully masked rows, and logits that spread (the pair bias, or the
+    # queries, scaled up) so that the softmax offset moves in later blocks. Above
+    # 64 queries a masked tail too. The general f16 bound of 1e-2.
+    x, mask, B, Q, tr, w, pb = case(name, S, L, C, H, Cp=16)
+    if Q > 64:
+        mask[-5:] = 0.0
+    if pb is None:
+        w["queryWeight"] = w["queryWeight"] * scale
+    else:
+        pb["projectionWeight"] = pb["projectionWeight"] * scale
+    expect = ref.attention(ref.round_f16(x), mask, w, B, Q, C, H, transpose=tr,
+                           pair_bias=None if pb is None else {k: ref.round_f16(v) if k == "activations" else v
+                                                              for k, v in pb.items()})
+    got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb, precision="f16", in_dtype="f16", out_dtype="f16")
+    assert np.abs(got - expect).max() <= 1e-2 * np.abs(expect).max()
