@@ -34,6 +34,7 @@
 #include <cmath>
 
 #include "gemm.h"
+#include "pairs.h"
 
 namespace afhip {
 
@@ -48,6 +49,7 @@ bool fused_ok(const afhip_opm_desc& d) {
 
 struct OpmWeights {
   size_t ln_scale, ln_offset, w_lr, b_lr, w_out, b_out, total;
+  size_t s_lr;  // f32 precision: the pair projection's output scales
   int cmp;  // c_m padded to 32
   int cop;  // 2 * c_outer padded to 64 (projection columns)
   int czp;  // c_z padded to 32 (output rows of W_out^T)
@@ -71,6 +73,7 @@ OpmWeights opm_layout(const afhip_opm_desc& d) {
   w.b_lr = take(4 * (size_t)w.cop);
   w.w_out = take(es * (size_t)w.czp * d.c_outer * d.c_outer);
   w.b_out = take(4 * (size_t)w.czp);
+  if (d.precision == AFHIP_PRECISION_F32) w.s_lr = take(4 * (size_t)w.cop);
   w.total = at;
   return w;
 }
@@ -106,8 +109,10 @@ struct ProjectArgs {
   const float* mask;
   const float* ln_scale;
   const float* ln_offset;
-  const void* w_lr;  // [cop][cmp]: rows [0, co) left, [co, 2co) right
+  const void* w_lr;  // [cop][cmp]: rows [0, co) left, [co, 2co) right (pairs: in fragment order)
   const float* b_lr;
+  const float* s_lr;  // pair kernel: output scales, and what x_hat is held times
+  float x_scale;
   void* left;
   void* right;
   int64_t sp;
@@ -115,16 +120,16 @@ struct ProjectArgs {
   float eps;
 };
 
-template <typename MT, bool F16MATH>
+template <typename MT>
 __global__ __launch_bounds__(256) void opm_project_kernel(ProjectArgs a) {
-  using CT = typename std::conditional<F16MATH, half_t, float>::type;
+  using CT = half_t;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int xpitch = kRows + 1;
   float* xs = reinterpret_cast<float*>(smem);
   size_t off = round_up((int64_t)a.cmp * xpitch * 4, 16);
   CT* an = reinterpret_cast<CT*>(smem + off);
   const int apitch = a.cmp + 8;
-  if (F16MATH) off += round_up((int64_t)kRows * apitch * 2, 16);
+  off += round_up((int64_t)kRows * apitch * 2, 16);
   CT* stage = reinterpret_cast<CT*>(smem + off);
   constexpr int spitch = kRows + 8;
 
@@ -161,8 +166,7 @@ __global__ __launch_bounds__(256) void opm_project_kernel(ProjectArgs a) {
     const float rstd = fast_rsqrt(var / (float)a.cm + a.eps);
     for (int c = part; c < a.cmp; c += 4) {
       float v = c < a.cm ? (xs[c * xpitch + q] - mean) * rstd * a.ln_scale[c] + a.ln_offset[c] : 0.0f;
-      if (F16MATH) an[q * apitch + c] = (CT)v;
-      else xs[c * xpitch + q] = v;
+      an[q * apitch + c] = (CT)v;
     }
   }
   __syncthreads();
@@ -175,18 +179,11 @@ __global__ __launch_bounds__(256) void opm_project_kernel(ProjectArgs a) {
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[v] = 0.0f;
     const int n = nc + (lane & 31);
-    if constexpr (F16MATH) {
-      for (int k = 0; k < a.cmp; k += 16) {
-        const int kk = k + 8 * (lane >> 5);
-        half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
-        half8 bf = *reinterpret_cast<const half8*>(W + (size_t)n * a.cmp + kk);
-        acc = mfma_f16(af, bf, acc);
-      }
-    } else {
-      for (int k = 0; k < a.cmp; k += 2) {
-        const int kk = k + (lane >> 5);
-        acc = mfma_f32(xs[kk * xpitch + rw + (lane & 31)], W[(size_t)n * a.cmp + kk], acc);
-      }
+    for (int k = 0; k < a.cmp; k += 16) {
+      const int kk = k + 8 * (lane >> 5);
+      half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
+      half8 bf = *reinterpret_cast<const half8*>(W + (size_t)n * a.cmp + kk);
+      acc = mfma_f16(af, bf, acc);
     }
     const float bias = a.b_lr[n];
 #pragma unroll
@@ -213,6 +210,101 @@ __global__ __launch_bounds__(256) void opm_project_kernel(ProjectArgs a) {
       dst[((int64_t)res * a.co + o) * a.sp + s] = stage[nl * spitch + i];
     }
     __syncthreads();
+  }
+}
+
+// f32 precision: the projection over pairs of f16 (pairs.h), any c_m <= 512.
+// Wave (rows 32 (w % 2).., column block w / 2 of each two) computes W x_hat^T, so
+// a lane ends with one (residue, sequence) row and 16 channels and each store
+// of a channel is up to 32 consecutive sequences. Before, 64-row tiles on the
+// f32 MFMA read the weights element by element inside the chain: at N_seq = 512,
+// N_res = 100, c_m = 256 224 us, now 24.
+template <typename MT, int MAXSTEPS>
+__global__ __launch_bounds__(256) void opm_project_pair_kernel(ProjectArgs a, int vec) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  half_t* an = reinterpret_cast<half_t*>(smem);
+  const int steps = a.cmp / 16, pitch = pair_pitch(steps);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rows = a.S * a.L, r0 = blockIdx.x * kPairRows;
+  const MT* msa = reinterpret_cast<const MT*>(a.msa);
+  const int hi = lane >> 5, r = r0 + 32 * (wave & 1) + (lane & 31);
+  const int res = r / a.S, seq = r - res * a.S;
+  const float keep = r < rows ? a.mask[(int64_t)seq * a.L + res] : 0.0f;
+  const int64_t block = (int64_t)steps * 1024;
+  const half_t* W = reinterpret_cast<const half_t*>(a.w_lr) + 8 * lane;
+  PairFragments f;
+  f.load(W + (2 * blockIdx.y + (wave >> 1)) * block, 0);
+  {
+    const int rq = r0 + (tid >> 2), rres = rq / a.S, rseq = rq - rres * a.S;
+    pair_normalize_row<MT, MAXSTEPS>(rq < rows ? msa + ((int64_t)rseq * a.L + rres) * a.cm : nullptr, a.cm, steps, a.eps,
+                                     a.x_scale, tid & 3, vec, an + (tid >> 2) * pitch);
+  }
+  __syncthreads();
+  const half_t* xr = an + (32 * (wave & 1) + (lane & 31)) * pitch + 8 * hi;
+  const int twos = a.cop / 64;
+  for (int p = blockIdx.y; p < twos; p += gridDim.y) {
+    const int nb = 2 * p + (wave >> 1);
+    floatx16 acc = {};
+    for (int s = 0; s < steps; s += 2) {
+      const PairFragments c = f;
+      // The next two steps, or the next block's first.
+      const int ns = s + 2 < steps ? s + 2 : 0;
+      const int np = min(s + 2 < steps ? p : p + (int)gridDim.y, twos - 1);
+      f.load(W + (2 * np + (wave >> 1)) * block, ns);
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const half8 xh = *reinterpret_cast<const half8*>(xr + 32 * (s + u));
+        const half8 xl = *reinterpret_cast<const half8*>(xr + 32 * (s + u) + 16);
+        acc = mfma_f16(c.h[u], xh, acc);
+        acc = mfma_f16(c.h[u], xl, acc);
+        acc = mfma_f16(c.l[u], xh, acc);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+      const int c = 32 * nb + 8 * (v >> 2) + 4 * hi + (v & 3);
+      const float y = keep * fmaf(acc[v], a.s_lr[c], a.b_lr[c]);
+      const bool left = c < a.co;
+      float* dst = reinterpret_cast<float*>(left ? a.left : a.right);
+      if (c < 2 * a.co && r < rows) dst[((int64_t)res * a.co + (left ? c : c - a.co)) * a.sp + seq] = y;
+    }
+  }
+}
+
+// The pair projection's weights, one wave a row n of [cop]: W' = W diag(gamma) in
+// double times 2^e (largest element in [2^14, 2^15)), scale 2^-(x_exp + e), bias
+// b + W beta; padding rows and columns are zeros.
+__global__ __launch_bounds__(64) void opm_pair_prepare_kernel(const float* __restrict__ packed, int cm, int co, int cmp,
+                                                              int x_exp, half_t* __restrict__ w_lr,
+                                                              float* __restrict__ s_lr, float* __restrict__ b_lr) {
+  const int n = blockIdx.x, lane = threadIdx.x;
+  const float *gamma = packed, *beta = packed + cm;
+  const bool in = n < 2 * co, left = n < co;
+  const float* w = beta + cm + (left ? 0 : (int64_t)cm * co + co);  // [cm][co], then its bias
+  const int col = left ? n : n - co;
+  float most = 0.0f;
+  double offset = 0.0;
+  if (in)
+    for (int k = lane; k < cm; k += 64) {
+      const double v = w[(int64_t)k * co + col];
+      most = fmaxf(most, fabsf((float)(v * gamma[k])));
+      offset += v * beta[k];
+    }
+  for (int o = 32; o > 0; o >>= 1) {
+    most = fmaxf(most, __shfl_xor(most, o));
+    offset += __shfl_xor(offset, o);
+  }
+  const int e = pair_exponent(most);
+  for (int k = lane; k < cmp; k += 64) {
+    half_t h, l;
+    pair_split(in && k < cm ? (float)ldexp((double)w[(int64_t)k * co + col] * gamma[k], e) : 0.0f, h, l);
+    const int64_t at = pair_fragment(n, k, cmp / 16);
+    w_lr[at] = h;
+    w_lr[at + 512] = l;
+  }
+  if (lane == 0) {
+    s_lr[n] = in ? ldexpf(1.0f, -(x_exp + e)) : 1.0f;
+    b_lr[n] = in ? (float)(w[(int64_t)cm * co + col] + offset) : 0.0f;
   }
 }
 
@@ -528,10 +620,24 @@ int validate(const afhip_opm_desc* d) {
   return AFHIP_OK;
 }
 
-template <typename MT, bool F16MATH>
-int launch_project(const ProjectArgs& pa, size_t shared, hipStream_t s) {
-  if (int st = allow_lds((const void*)opm_project_kernel<MT, F16MATH>, shared)) return st;
-  return launch("opm.project", opm_project_kernel<MT, F16MATH>, dim3((unsigned)ceil_div((int64_t)pa.S * pa.L, kRows)),
+template <typename MT, int MAXSTEPS> int launch_project_pair_steps(const ProjectArgs& pa, hipStream_t s) {
+  const int64_t tiles = ceil_div((int64_t)pa.S * pa.L, kPairRows);
+  const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const unsigned splits = (unsigned)std::max<int64_t>(1, std::min<int64_t>(pa.cop / 64, 2 * cus / tiles));
+  const size_t shared = (size_t)kPairRows * pair_pitch(pa.cmp / 16) * 2;
+  auto k = opm_project_pair_kernel<MT, MAXSTEPS>;
+  if (int st = allow_lds((const void*)k, shared)) return st;
+  return launch("opm.project", k, dim3((unsigned)tiles, splits), dim3(256), shared, s, pa,
+                (int)rows_on_four(pa.msa, pa.cm, sizeof(MT)));
+}
+
+template <typename MT> int launch_project_pair(const ProjectArgs& pa, hipStream_t s) {
+  return pa.cmp <= 256 ? launch_project_pair_steps<MT, 16>(pa, s) : launch_project_pair_steps<MT, 32>(pa, s);
+}
+
+template <typename MT> int launch_project(const ProjectArgs& pa, size_t shared, hipStream_t s) {
+  if (int st = allow_lds((const void*)opm_project_kernel<MT>, shared)) return st;
+  return launch("opm.project", opm_project_kernel<MT>, dim3((unsigned)ceil_div((int64_t)pa.S * pa.L, kRows)),
                 dim3(256), shared, s, pa);
 }
 
@@ -578,6 +684,11 @@ int afhip_opm_prepare_weights(const afhip_opm_desc* desc, const float* packed, v
                        w.cmp, w.cop, w.czp, (float*)(base + w.w_lr), (float*)(base + w.b_lr),
                        (float*)(base + w.w_out), (float*)(base + w.b_out), ln_s, ln_o, false))
       return s;
+    // The projection's weights again, as pairs over the f32 ones.
+    if (int s = launch("opm.prepare", opm_pair_prepare_kernel, dim3(w.cop), dim3(64), 0, st, packed, d.c_m, d.c_outer,
+                       w.cmp, pair_norm_exponent(d.c_m), (half_t*)(base + w.w_lr), (float*)(base + w.s_lr),
+                       (float*)(base + w.b_lr)))
+      return s;
   }
   return AFHIP_OK;
 }
@@ -615,8 +726,10 @@ int afhip_opm_run(const afhip_opm_desc* desc, const void* activations, const flo
   pa.cmp = w.cmp;
   pa.cop = w.cop;
   pa.eps = d.layer_norm_epsilon;
-  size_t psh = round_up((int64_t)w.cmp * (kRows + 1) * 4, 16) +
-               (f16 ? round_up((int64_t)kRows * (w.cmp + 8) * 2, 16) : 0) + (size_t)64 * (kRows + 8) * (f16 ? 2 : 4);
+  pa.s_lr = (const float*)(wb + w.s_lr);
+  pa.x_scale = ldexpf(1.0f, pair_norm_exponent(d.c_m));
+  const size_t psh = round_up((int64_t)w.cmp * (kRows + 1) * 4, 16) + round_up((int64_t)kRows * (w.cmp + 8) * 2, 16) +
+                     (size_t)64 * (kRows + 8) * 2;
   int s;
   float* count = (float*)(wsb + ws.count);
   // The fast projection computes the pair counts in the same launch.
@@ -624,9 +737,9 @@ int afhip_opm_run(const afhip_opm_desc* desc, const void* activations, const flo
   if (fast)
     s = d.msa_dtype == AFHIP_F32 ? launch_fast_cm<float>(pa, count, st) : launch_fast_cm<half_t>(pa, count, st);
   else if (f16)
-    s = d.msa_dtype == AFHIP_F32 ? launch_project<float, true>(pa, psh, st) : launch_project<half_t, true>(pa, psh, st);
+    s = d.msa_dtype == AFHIP_F32 ? launch_project<float>(pa, psh, st) : launch_project<half_t>(pa, psh, st);
   else
-    s = d.msa_dtype == AFHIP_F32 ? launch_project<float, false>(pa, psh, st) : launch_project<half_t, false>(pa, psh, st);
+    s = d.msa_dtype == AFHIP_F32 ? launch_project_pair<float>(pa, st) : launch_project_pair<half_t>(pa, st);
   if (s) return s;
 
   if (!fast) {

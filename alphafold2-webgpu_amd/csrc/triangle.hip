@@ -25,6 +25,7 @@
 #include <cstring>
 
 #include "gemm.h"
+#include "pairs.h"
 #include "triangle_fast.h"
 
 namespace afhip {
@@ -384,15 +385,7 @@ __global__ __launch_bounds__(256) void tri_output_kernel(OutputArgs a) {
 // Measured at c_z = c_h = 128, project / output: L = 59 83 / 63 us before,
 // 10.7 / 12.2 after; L = 256 365 / 157 before, 58 / 64 after.
 
-constexpr int kPairRows = 64;   // pairs a workgroup
-constexpr int kMaxSteps = 8;    // c_z <= 128 in steps of 16
-
-// Element (n, k) of a weight matrix of `steps` 16-wide steps, in the order the
-// lanes load fragments: [n / 32][step][plane][lane][8], lane = n % 32 +
-// 32 (k % 16 / 8). h is plane 0; l lies 512 halves on.
-__device__ __forceinline__ int64_t pair_fragment(int n, int k, int steps) {
-  return (((int64_t)(n >> 5) * steps + (k >> 4)) * 2 * 64 + (n & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
-}
+constexpr int kMaxSteps = 8;  // c_z <= 128 in steps of 16
 
 struct PairSources {
   struct Matrix {
@@ -437,78 +430,6 @@ __global__ __launch_bounds__(64) void tri_pair_prepare_kernel(PairSources src) {
   }
 }
 
-// Four lanes normalise one row of z (row pointer, or null for zeros) and write
-// x_hat x_scale as pairs to `dst` (a pair row in LDS): lane `part` takes
-// channels 16 i + 4 part + [0, 4) of each block i.
-template <typename ZT>
-__device__ __forceinline__ void pair_normalize_row(const ZT* row, int cz, int steps, float eps, float x_scale, int part,
-                                                   bool vec, half_t* dst) {
-  float v[kMaxSteps][4];
-#pragma unroll
-  for (int i = 0; i < kMaxSteps; i++) {
-    const int c = 16 * i + 4 * part;
-#pragma unroll
-    for (int e = 0; e < 4; e++) v[i][e] = 0.0f;
-    if (i >= steps || !row) continue;
-    if (vec) {
-      if (c < cz) {
-        typedef ZT zt4 __attribute__((ext_vector_type(4)));
-        const zt4 w = *reinterpret_cast<const zt4*>(row + c);
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[i][e] = (float)w[e];
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-        if (c + e < cz) v[i][e] = (float)row[c + e];
-    }
-  }
-  float s = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kMaxSteps; i++) s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
-  s += __shfl_xor(s, 1);
-  s += __shfl_xor(s, 2);
-  const float mean = s / (float)cz;
-  float d2 = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kMaxSteps; i++)
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      v[i][e] = 16 * i + 4 * part + e < cz ? v[i][e] - mean : 0.0f;
-      d2 += v[i][e] * v[i][e];
-    }
-  d2 += __shfl_xor(d2, 1);
-  d2 += __shfl_xor(d2, 2);
-  const float rstd = fast_rsqrt(d2 / (float)cz + eps) * x_scale;
-#pragma unroll
-  for (int i = 0; i < kMaxSteps; i++) {
-    if (i >= steps) continue;
-    half2v h0, l0, h1, l1;
-    pair_split2(v[i][0] * rstd, v[i][1] * rstd, h0, l0);
-    pair_split2(v[i][2] * rstd, v[i][3] * rstd, h1, l1);
-    half_t* p = dst + 32 * i + 4 * part;
-    *reinterpret_cast<half4*>(p) = half4{h0[0], h0[1], h1[0], h1[1]};
-    *reinterpret_cast<half4*>(p + 16) = half4{l0[0], l0[1], l1[0], l1[1]};
-  }
-}
-
-// Two steps' fragments (h, l of each) of one matrix block; `w` at the block's
-// first fragment, this lane's 16 bytes.
-struct PairFragments {
-  half8 h[2], l[2];
-  __device__ __forceinline__ void load(const half_t* w, int s) {
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      h[u] = *reinterpret_cast<const half8*>(w + (int64_t)(s + u) * 1024);
-      l[u] = *reinterpret_cast<const half8*>(w + (int64_t)(s + u) * 1024 + 512);
-    }
-  }
-};
-
-// LDS pair rows of 16 `steps` channels, padded by 16 bytes: 16 rows' fragments
-// then start on 16 different groups of four banks.
-__host__ __device__ constexpr int pair_pitch(int steps) { return 32 * steps + 8; }  // halves
-
 // Wave (rows 32 (w % 2).., operand w / 2) of a tile computes W x_hat^T for the
 // projection and the gate of 32 hidden channels: a lane ends with one pair and
 // 16 channels, so each store of a channel is 32 consecutive pairs.
@@ -531,7 +452,7 @@ template <typename ZT> __global__ __launch_bounds__(256) void tri_project_pair_k
   fg.load(W + matrix + blockIdx.y * block, 0);
   {
     const int q = tid >> 2, rq = r0 + q;
-    pair_normalize_row<ZT>(rq < a.P ? z + (int64_t)pair_of(rq) * a.cz : nullptr, a.cz, steps, a.eps, a.x_scale, tid & 3,
+    pair_normalize_row<ZT, kMaxSteps>(rq < a.P ? z + (int64_t)pair_of(rq) * a.cz : nullptr, a.cz, steps, a.eps, a.x_scale, tid & 3,
                            vec, an + q * pitch);
   }
   __syncthreads();
@@ -625,7 +546,7 @@ template <typename ZT, typename OT> __global__ __launch_bounds__(256) void tri_o
   }
   {
     const int q = tid >> 2;
-    pair_normalize_row<ZT>(q0 + q < a.pairs ? z + (int64_t)(a.pair0 + q0 + q) * a.cz : nullptr, a.cz, zsteps, a.eps,
+    pair_normalize_row<ZT, kMaxSteps>(q0 + q < a.pairs ? z + (int64_t)(a.pair0 + q0 + q) * a.cz : nullptr, a.cz, zsteps, a.eps,
                            a.x_scale, tid & 3, vec, zn + q * zpitch);
   }
   float s = 0.0f;
@@ -802,10 +723,6 @@ template <typename ZT, typename OT> int launch_output(const OutputArgs& oa, size
 unsigned column_splits(int64_t tiles, int blocks) {
   const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>(blocks, 2 * cus / tiles));
-}
-
-bool rows_on_four(const void* z, int cz, size_t es) {
-  return cz % 4 == 0 && (reinterpret_cast<uintptr_t>(z) & (4 * es - 1)) == 0;
 }
 
 template <typename ZT> int launch_project_pair(const ProjectArgs& pa, hipStream_t s) {

@@ -384,3 +384,32 @@ def test_transition_f32_pairs(dev, rows, c, h, in_dt, out_dt, residual, shift):
 
     out = op(place(x, in_dt), out=place(old, out_dt)).float().cpu().numpy()
     assert np.abs(out - expect).max() <= (1e-5 if out_dt == "f32" else 1e-5 + 2.0 ** -11) * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("S,L,cm,co,cz,msa_dtype,shift", [(1, 3, 512, 32, 16, "f32", 0), (65, 2, 300, 20, 8, "f16", 1),
+                                                          (31, 9, 17, 40, 12, "f32", 3), (64, 70, 64, 32, 128, "f32", 0)])
+def test_opm_f32_pair_projection(dev, S, L, cm, co, cz, msa_dtype, shift):
+    # f32 precision's projection over pairs of f16: one to two column blocks of
+    # 64, ragged tiles whose rows cross residues, channels short of their padding
+    # and up to 512, the MSA off 16-byte alignment (shift elements). The
+    # LayerNorm's scales and the columns of the weights it feeds carry factors of
+    # 1e-6 to 1e6 that cancel. The f32 bound of the other tests.
+    import torch
+
+    from afhip import opm
+
+    act = ref.round_f16(ref.normal(41 + cm, (S, L, cm)))
+    mask = (ref.uniform(42, (S, L), 0, 1) > 0.2).astype(np.float32)
+    fc = 10.0 ** ref.uniform(43, (cm,), -6, 6)
+    w = {"layerNormScale": ref.normal(44, (cm,), 0.01, 1.0) * fc, "layerNormOffset": ref.normal(45, (cm,), 0.01) * fc,
+         "leftWeight": ref.normal(46, (cm, co), 1 / cm) / fc[:, None], "leftBias": ref.normal(47, (co,), 0.02),
+         "rightWeight": ref.normal(48, (cm, co), 1 / cm) / fc[:, None], "rightBias": ref.normal(49, (co,), 0.02),
+         "outputWeight": ref.normal(50, (co * co, cz), 1 / (co * co)), "outputBias": ref.normal(51, (cz,), 0.02)}
+    w = {k: np.asarray(v, np.float32) for k, v in w.items()}
+    expect = ref.opm(act, mask, w)
+    op = opm.OuterProductMean(S, L, cm, co, cz, msa_dtype=msa_dtype)
+    op.prepare(w)
+    flat = torch.zeros(act.size + shift, dtype=torch.float16 if msa_dtype == "f16" else torch.float32, device=dev)
+    flat[shift:] = torch.from_numpy(act).to(dev).reshape(-1)
+    out = op(flat[shift:].reshape(S, L, cm), torch.from_numpy(mask).to(dev)).cpu().numpy()
+    assert np.abs(out - expect).max() <= 1e-5 * np.abs(expect).max()
