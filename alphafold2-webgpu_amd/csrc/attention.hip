@@ -165,6 +165,10 @@ int validate(const afhip_attention_desc* dp) {
 // Kernels
 // --------------------------------------------------------------------------
 
+typedef short short4v __attribute__((ext_vector_type(4)));
+typedef short short8v __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) short4v lds_short4v;
+
 template <typename T> __device__ __forceinline__ float ld(const T* p, int64_t i) { return (float)p[i]; }
 
 // Weight preparation from the reference's packed f32 order
@@ -785,7 +789,7 @@ template <typename CT> int launch_flash_f32(const FlashArgs& fa, hipStream_t st)
 // offset as in the f32 kernel above; the output, still times v's power of two,
 // leaves as pairs for the output projection.
 // Bound: the loads (20 instructions a block over 32 rows each, for every wave
-// its own). Column attention over 508 sequences x 59 residues, 8 heads of 32:
+// its own), which the next kernel shares where there are blocks enough. Column attention over 508 sequences x 59 residues, 8 heads of 32:
 // 115 us, the f32 kernel 163; dropping a third of the vector instructions
 // (v_fma_mix_f32 in the split, no per-load bound) left it at 117.
 // log2: keeps small weights' l out of f16's last digits. A weight is at most
@@ -983,9 +987,195 @@ template <int STEPS, int LOAD> int launch_flash_pair_as(const FlashArgs& fa, hip
                 per_xcd);
 }
 
+// The same at head dimension 32 over more than 64 keys, with the key blocks
+// shared: the four waves of a workgroup take four query blocks of one (b, h) and
+// each loads and splits a quarter of a block's K and V into LDS planes of h and l
+// (K rows padded to 80 bytes for the fragment reads, V in 64-byte rows for the
+// transposing ones), double-buffered with one barrier a block. That takes the
+// loads of a block from 20 instructions over 32 rows a wave to two over four,
+// and two thirds of the splitting. Measured, column attention over 508 sequences
+// x 59 residues, 8 heads of 32: 116 us unshared, 83 shared.
+struct PairTile {
+  half_t k[2][32][40];  // [plane][key][channel]
+  half_t v[2][32][32];
+};
+
+template <bool BIAS>
+__global__ __launch_bounds__(64 * kF32Waves) void attention_flash_pair32_kernel(FlashArgs a, int qgroups, int64_t groups,
+                                                                             int64_t per_xcd) {
+  __shared__ __attribute__((aligned(16))) PairTile tiles[2];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, hi = lane >> 5;
+  const int64_t group = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (group >= groups) return;  // the whole workgroup
+  const int q0 = 32 * ((int)(group % qgroups) * kF32Waves + __builtin_amdgcn_readfirstlane(tid >> 6));
+  const int h = (int)(group / qgroups % a.H);
+  const int64_t b = group / qgroups / a.H;
+  const int Q = a.Q;
+  const uint32_t ldb = 16u * (uint32_t)a.C;  // bytes between rows
+  const char* rows = reinterpret_cast<const char*>(a.qkvg) + (b * Q * 4 * a.C + (int64_t)h * 32) * 4;
+  const char* keys = rows + (int64_t)a.C * 4;
+  const char* vals = keys + (int64_t)a.C * 4;
+  const float unit = a.logit_scale[h];
+  const bool active = q0 < Q;  // idle waves still load and meet every barrier
+
+  // This lane's piece of a block: key tid / 8, channels 4 (tid % 8)..; keys past
+  // the end repeat the last (their logits are dropped).
+  const int pkey = tid >> 3, pch = 4 * (tid & 7);
+  float4 pk, pv;
+  auto fetch = [&](int k0) {
+    const uint32_t off = (uint32_t)min(k0 + pkey, Q - 1) * ldb + 4u * pch;
+    pk = *reinterpret_cast<const float4*>(keys + off);
+    pv = *reinterpret_cast<const float4*>(vals + off);
+  };
+  auto stash = [&](PairTile& t) {
+    half2v h0, l0, h1, l1;
+    pair_split2(pk.x, pk.y, h0, l0);
+    pair_split2(pk.z, pk.w, h1, l1);
+    *reinterpret_cast<half4*>(&t.k[0][pkey][pch]) = half4{h0[0], h0[1], h1[0], h1[1]};
+    *reinterpret_cast<half4*>(&t.k[1][pkey][pch]) = half4{l0[0], l0[1], l1[0], l1[1]};
+    pair_split2(pv.x, pv.y, h0, l0);
+    pair_split2(pv.z, pv.w, h1, l1);
+    *reinterpret_cast<half4*>(&t.v[0][pkey][pch]) = half4{h0[0], h0[1], h1[0], h1[1]};
+    *reinterpret_cast<half4*>(&t.v[1][pkey][pch]) = half4{l0[0], l0[1], l1[0], l1[1]};
+  };
+  const int myq = q0 + col, qc = min(myq, Q - 1);
+  const float* kb_row = a.key_bias + b * a.stride;
+  const float* pb_row = BIAS ? a.bias + ((int64_t)h * Q + qc) * a.stride : nullptr;
+  auto load_bias = [&](const float* row, int k0, float (&f)[16]) {
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const float4 w = *reinterpret_cast<const float4*>(row + min(k0 + 8 * g + 4 * hi, a.stride - 4));
+      f[4 * g] = w.x, f[4 * g + 1] = w.y, f[4 * g + 2] = w.z, f[4 * g + 3] = w.w;
+    }
+  };
+  auto split8 = [&](const float* f, half8& hh, half8& ll) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      half2v h2, l2;
+      pair_split2(f[e], f[e + 1], h2, l2);
+      hh[e] = h2[0], hh[e + 1] = h2[1], ll[e] = l2[0], ll[e + 1] = l2[1];
+    }
+  };
+
+  fetch(0);
+  half8 qh[2], ql[2];
+  {
+    const float* p = reinterpret_cast<const float*>(rows + (uint32_t)qc * ldb) + 8 * hi;
+    float qf[16];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float4 w = *reinterpret_cast<const float4*>(p + 16 * (i >> 1) + 4 * (i & 1));
+      qf[4 * i] = w.x, qf[4 * i + 1] = w.y, qf[4 * i + 2] = w.z, qf[4 * i + 3] = w.w;
+    }
+#pragma unroll
+    for (int s = 0; s < 2; s++) split8(qf + 8 * s, qh[s], ql[s]);
+  }
+  float kb[16], pb[16];
+  load_bias(kb_row, 0, kb);
+  if constexpr (BIAS) load_bias(pb_row, 0, pb);
+  stash(tiles[0]);
+  fetch(32);
+  block_barrier();
+
+  // The transposing reads' addresses, as in the f16 kernels.
+  const int tr_key = 4 * hi + ((lane & 15) >> 2), tr_ch = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  floatx16 o = {};
+  float m = -1e30f, offset = 0.0f;
+  float sum = 0.0f;  // over this lane half's keys
+  for (int k0 = 0, buf = 0; k0 < Q; k0 += 32, buf ^= 1) {
+    const PairTile& t = tiles[buf];
+    if (active) {
+      floatx16 sc = {};
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const half8 kh = *reinterpret_cast<const half8*>(&t.k[0][col][16 * s + 8 * hi]);
+        const half8 kl = *reinterpret_cast<const half8*>(&t.k[1][col][16 * s + 8 * hi]);
+        sc = mfma_f16(kh, qh[s], sc);
+        sc = mfma_f16(kh, ql[s], sc);
+        sc = mfma_f16(kl, qh[s], sc);
+      }
+      float x[16];
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const float l = fmaf(sc[v], unit, kb[v]);
+        x[v] = __builtin_amdgcn_fmed3f(BIAS ? l + pb[v] : l, -a.clamp, a.clamp);
+      }
+      load_bias(kb_row, k0 + 32, kb);
+      if constexpr (BIAS) load_bias(pb_row, k0 + 32, pb);
+      if (k0 + 32 > Q) {
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+          if (k0 + 8 * (v >> 2) + 4 * hi + (v & 3) >= Q) x[v] = kDropped;
+      }
+      float mx = x[0];
+#pragma unroll
+      for (int v = 1; v < 16; v++) mx = fmaxf(mx, x[v]);
+      if (__builtin_amdgcn_ballot_w64(mx > m + kF32Slack)) {
+        const float to = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)));
+        const float f = __builtin_amdgcn_exp2f((m - to) * kLog2e);
+        sum *= f;
+#pragma unroll
+        for (int v = 0; v < 16; v++) o[v] *= f;
+        m = to;
+        offset = fmaf(-to, kLog2e, kPairWeight);
+      }
+#pragma unroll
+      for (int v = 0; v < 16; v++) x[v] = __builtin_amdgcn_exp2f(fmaf(x[v], kLog2e, offset));
+      sum += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])) +
+             (((x[8] + x[9]) + (x[10] + x[11])) + ((x[12] + x[13]) + (x[14] + x[15])));
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        half8 ph, pl, vt[2];
+        split8(x + 8 * s, ph, pl);
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+          const half_t* vp = &t.v[p][16 * s + tr_key][tr_ch];
+          const short4v x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)vp);
+          const short4v x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)(vp + 8 * 32));
+          vt[p] = __builtin_bit_cast(half8, short8v{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]});
+        }
+        o = mfma_f16(vt[0], ph, o);
+        o = mfma_f16(vt[0], pl, o);
+        o = mfma_f16(vt[1], ph, o);
+      }
+    }
+    // Block k0 + 32 goes to the buffer whose reads ended before the last
+    // barrier; block k0 + 64 starts on its way.
+    stash(tiles[buf ^ 1]);
+    fetch(k0 + 64);
+    block_barrier();
+  }
+  sum += __shfl_xor(sum, 32);
+  if (myq >= Q) return;
+  const float* gr = reinterpret_cast<const float*>(rows + (uint32_t)myq * ldb) + 3 * (int64_t)a.C;
+  const int64_t src = a.transpose ? (int64_t)myq * a.B + b : b * Q + myq;
+  half_t* out = reinterpret_cast<half_t*>(a.weighted) + src * 2 * a.C;
+  float4 gv[4];
+#pragma unroll
+  for (int g = 0; g < 4; g++) gv[g] = *reinterpret_cast<const float4*>(gr + 8 * g + 4 * hi);
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    half2v h0, l0, h1, l1;
+    pair_split2(o[4 * g] / sum * gv[g].x, o[4 * g + 1] / sum * gv[g].y, h0, l0);
+    pair_split2(o[4 * g + 2] / sum * gv[g].z, o[4 * g + 3] / sum * gv[g].w, h1, l1);
+    half_t* p = out + pair_index(h * 32 + 8 * g + 4 * hi);
+    *reinterpret_cast<half4*>(p) = half4{h0[0], h0[1], h1[0], h1[1]};
+    *reinterpret_cast<half4*>(p + 16) = half4{l0[0], l0[1], l1[0], l1[1]};
+  }
+}
+
+int launch_flash_pair32(const FlashArgs& fa, hipStream_t st) {
+  const int qgroups = (int)ceil_div(fa.Q, 32 * kF32Waves);
+  const int64_t groups = (int64_t)fa.B * fa.H * qgroups, per_xcd = ceil_div(groups, 8);
+  AFHIP_REQUIRE(per_xcd < ((int64_t)1 << 28), "attention grid too large");
+  auto k = fa.bias ? attention_flash_pair32_kernel<true> : attention_flash_pair32_kernel<false>;
+  return launch("attention.flash", k, dim3((unsigned)(8 * per_xcd)), dim3(64 * kF32Waves), 0, st, fa, qgroups, groups,
+                per_xcd);
+}
+
 int launch_flash_pair(const FlashArgs& fa, hipStream_t st) {
   if (fa.d % 4) return launch_flash_pair_as<2, 0>(fa, st);
-  if (fa.d == 32) return launch_flash_pair_as<2, 2>(fa, st);
+  if (fa.d == 32) return fa.Q > 64 ? launch_flash_pair32(fa, st) : launch_flash_pair_as<2, 2>(fa, st);
   return fa.d <= 16 ? launch_flash_pair_as<1, 1>(fa, st) : launch_flash_pair_as<2, 1>(fa, st);
 }
 
@@ -1024,10 +1214,6 @@ constexpr float kSlack = 8.0f;
 // Base-2 distance below the row maximum past which exp2 gives 0 in f32
 // (below 2^-149) and therefore in f16.
 constexpr float kClampReach = 160.0f;
-
-typedef short short4v __attribute__((ext_vector_type(4)));
-typedef short short8v __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) short4v lds_short4v;
 
 struct FlashTile {
   half_t k[kFlashBatch][32][40];   // [bi][key][channel], rows padded to 80 bytes

@@ -423,3 +423,22 @@ def test_f16_four_heads_of_eight(dev, name, S, L, scale, C, H):
                                                               for k, v in pb.items()})
     got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb, precision="f16", in_dtype="f16", out_dtype="f16")
     assert np.abs(got - expect).max() <= 1e-2 * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("name,S,L,scale", [("msa_column", 96, 2, 4), ("msa_column", 129, 3, 1), ("msa_row", 2, 161, 12),
+                                            ("triangle_end", 0, 130, 1)])
+def test_f32_pairs_shared_key_blocks(dev, name, S, L, scale):
+    # Head dimension 32 over more than 64 keys: three, four and five query blocks
+    # of 32 (workgroups with idle waves), ragged last blocks, a masked stretch and
+    # a masked tail, logits that spread (the pair bias or the queries scaled up)
+    # so that the offset moves in later blocks. The bound of the f32 flash edges.
+    C, H = 64, 2
+    x, mask, B, Q, tr, w, pb = case(name, S, L, C, H, Cp=16)
+    mask[-7:] = 0.0
+    if pb is None:
+        w["queryWeight"] = w["queryWeight"] * scale
+    else:
+        pb["projectionWeight"] = pb["projectionWeight"] * scale
+    expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
+    got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb)
+    assert np.abs(got - expect).max() <= 7e-5 * np.abs(expect).max()
