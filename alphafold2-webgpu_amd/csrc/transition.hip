@@ -129,74 +129,101 @@ __global__ void transition_prepare_kernel(const float* __restrict__ packed, int 
   }
 }
 
-// Weights of the pair path, one workgroup a row of W1 [H][C], then of W2 [C][H].
+// Weights of the pair path, one workgroup for 16 rows of W1 [H][C], then of W2
+// [C][H] (both lie transposed in the packed tensors: 16 neighbours a read, and
+// through an LDS tile on to whole rows).
 // With x_hat = (x - mean) rstd, |x_hat|_2 <= sqrt(C) for any row:
 //   W1'[h] = W1[h] diag(gamma) in double, scaled by 2^e to fill f16 (largest
-//   element in [2^14, 2^15)); x_hat is stored times 2^x_shift(C) <= 2^15;
+//   element in [2^14, 2^15)); x_hat is stored times 2^x_exp <= 2^15;
 //   b1' = b1 + W1 beta; the hidden unit h stays below
 //   B = sqrt(C) |W1'[h]|_2 + |b1'|, so its pairs hold it times 2^-u, B 2^-u in
 //   (2^14, 2^15]; W2's column h takes 2^u back.
 // The first linear's scale and bias carry 2^-u (it commutes with the ReLU).
+constexpr int kPrepRows = 16, kPrepInner = 64;
+
+// Rows n0.. of dst (pair rows of K) from src [K][N]: value(k, n, src[k][n]).
+template <typename F>
+__device__ __forceinline__ void pair_transpose(const float* __restrict__ src, int K, int N, int n0, half_t* dst,
+                                               float (*tile)[kPrepRows + 1], const F& value) {
+  const int a = threadIdx.x & 15, b = threadIdx.x >> 4;
+  for (int k0 = 0; k0 < K; k0 += kPrepInner) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPrepInner / 16; i++) {
+      const int k = b + 16 * i;
+      if (k0 + k < K) tile[k][a] = src[(int64_t)(k0 + k) * N + n0 + a];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPrepInner / 16; i++) {
+      const int k = a + 16 * i;
+      if (k0 + k < K) pair_store(dst + (int64_t)(n0 + b) * 2 * K, k0 + k, value(k0 + k, b, tile[k][b]));
+    }
+  }
+}
+
 __global__ __launch_bounds__(256) void pair_first_kernel(const float* __restrict__ packed, int C, int H, int x_exp,
                                                          half_t* __restrict__ w1, float* __restrict__ s1,
                                                          float* __restrict__ b1, int* __restrict__ shift) {
   const float* gamma = packed;
   const float* beta = gamma + C;
   const float* f = beta + C;  // [C][H]
-  const int h = blockIdx.x;
+  const int h0 = blockIdx.x * kPrepRows, r = threadIdx.x & 15, part = threadIdx.x >> 4;
   float most = 0.0f;
   double squares = 0.0, offset = 0.0;
-  for (int c = threadIdx.x; c < C; c += 256) {
-    const double w = f[(size_t)c * H + h], g = w * gamma[c];
+  for (int c = part; c < C; c += 16) {
+    const double w = f[(size_t)c * H + h0 + r], g = w * gamma[c];
     most = fmaxf(most, fabsf((float)g));
     squares += g * g;
     offset += w * beta[c];
   }
-  __shared__ float m_part[4];
-  __shared__ double s_part[4], o_part[4];
-  for (int o = 32; o > 0; o >>= 1) {
-    most = fmaxf(most, __shfl_xor(most, o));
-    squares += __shfl_xor(squares, o);
-    offset += __shfl_xor(offset, o);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    m_part[threadIdx.x >> 6] = most;
-    s_part[threadIdx.x >> 6] = squares;
-    o_part[threadIdx.x >> 6] = offset;
-  }
+  __shared__ float m_part[16][16], tile[kPrepInner][kPrepRows + 1];
+  __shared__ double s_part[16][16], o_part[16][16];
+  __shared__ int exps[16];
+  m_part[part][r] = most;
+  s_part[part][r] = squares;
+  o_part[part][r] = offset;
   __syncthreads();
-  most = fmaxf(fmaxf(m_part[0], m_part[1]), fmaxf(m_part[2], m_part[3]));
-  squares = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
-  const double bias = f[(size_t)C * H + h] + ((o_part[0] + o_part[1]) + (o_part[2] + o_part[3]));
-  const int e = pair_exponent(most);
-  const int u = -pair_exponent((float)(sqrt((double)C * squares) + fabs(bias)));
-  for (int c = threadIdx.x; c < C; c += 256)
-    pair_store(w1 + (int64_t)h * 2 * C, c, (float)ldexp((double)f[(size_t)c * H + h] * gamma[c], e));
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 16) {
+    const int h = h0 + r;
+    for (int p = 1; p < 16; p++) {
+      most = fmaxf(most, m_part[p][r]);
+      squares += s_part[p][r];
+      offset += o_part[p][r];
+    }
+    const double bias = f[(size_t)C * H + h] + offset;
+    const int e = pair_exponent(most);
+    const int u = -pair_exponent((float)(sqrt((double)C * squares) + fabs(bias)));
     s1[h] = ldexpf(1.0f, -(x_exp + e + u));
     b1[h] = (float)ldexp(bias, -u);
     shift[h] = u;
+    exps[r] = e;
   }
+  __syncthreads();
+  pair_transpose(f, C, H, h0, w1, tile,
+                 [&](int c, int row, float w) { return (float)ldexp((double)w * gamma[c], exps[row]); });
 }
 
 __global__ __launch_bounds__(256) void pair_second_kernel(const float* __restrict__ packed, int C, int H,
                                                           const int* __restrict__ shift, half_t* __restrict__ w2,
                                                           float* __restrict__ s2, float* __restrict__ b2) {
   const float* g = packed + 2 * (size_t)C + (size_t)C * H + H;  // [H][C]
-  const int c = blockIdx.x;
+  const int c0 = blockIdx.x * kPrepRows, r = threadIdx.x & 15, part = threadIdx.x >> 4;
   float most = 0.0f;
-  for (int h = threadIdx.x; h < H; h += 256) most = fmaxf(most, fabsf(ldexpf(g[(size_t)h * C + c], shift[h])));
-  __shared__ float part[4];
-  for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = most;
+  for (int h = part; h < H; h += 16) most = fmaxf(most, fabsf(ldexpf(g[(size_t)h * C + c0 + r], shift[h])));
+  __shared__ float m_part[16][16], tile[kPrepInner][kPrepRows + 1];
+  __shared__ int exps[16];
+  m_part[part][r] = most;
   __syncthreads();
-  const int e = pair_exponent(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
-  for (int h = threadIdx.x; h < H; h += 256)
-    pair_store(w2 + (int64_t)c * 2 * H, h, ldexpf(g[(size_t)h * C + c], shift[h] + e));
-  if (threadIdx.x == 0) {
-    s2[c] = ldexpf(1.0f, -e);
+  if (threadIdx.x < 16) {
+    const int c = c0 + r;
+    for (int p = 1; p < 16; p++) most = fmaxf(most, m_part[p][r]);
+    exps[r] = pair_exponent(most);
+    s2[c] = ldexpf(1.0f, -exps[r]);
     b2[c] = g[(size_t)H * C + c];
   }
+  __syncthreads();
+  pair_transpose(g, H, C, c0, w2, tile, [&](int h, int row, float w) { return ldexpf(w, shift[h] + exps[row]); });
 }
 
 // The LayerNorm without its affine, rows written as pairs of x_hat 2^x_exp;
@@ -449,11 +476,11 @@ int afhip_transition_prepare_weights(const afhip_transition_desc* desc, const fl
     return AFHIP_OK;
   }
   if (pair_shape(d)) {
-    if (int s = launch("transition.prepare", pair_first_kernel, dim3(d.hidden), dim3(256), 0, st, packed, d.channels,
+    if (int s = launch("transition.prepare", pair_first_kernel, dim3(d.hidden / kPrepRows), dim3(256), 0, st, packed, d.channels,
                        d.hidden, pair_norm_exponent(d.channels), (half_t*)(b + w.w1), (float*)(b + w.s1),
                        (float*)(b + w.b1), (int*)(b + w.shift)))
       return s;
-    return launch("transition.prepare", pair_second_kernel, dim3(d.channels), dim3(256), 0, st, packed, d.channels,
+    return launch("transition.prepare", pair_second_kernel, dim3(d.channels / kPrepRows), dim3(256), 0, st, packed, d.channels,
                   d.hidden, (const int*)(b + w.shift), (half_t*)(b + w.w2), (float*)(b + w.s2), (float*)(b + w.b2));
   }
   return launch("transition.prepare", transition_prepare_kernel<float>, dim3(1024), dim3(256), 0, st, packed,
