@@ -88,6 +88,7 @@ typedef float f32x8v __attribute__((ext_vector_type(8)));
 // mean's output projection run on the finished contraction tile.
 constexpr int kEpiGeneric = 0;
 constexpr int kEpiOpmFused = 1;
+constexpr int kEpiAttention = 2;  // generic, with the attention blocks in the row-wise epilogue
 
 template <int BM, int BN, int STAGES, int WM, int WN, bool PIPE, typename TC, int EPI = kEpiGeneric, int LW = 16,
           bool AK = false, bool AF = false, bool FP32 = false, bool PAIRS = false>
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(64 * WM * WN, FP32 && STAGES == 2 ? 4 : PAIRS && ST
   // stage and is rounded to f16 as the fragments are read.
   // f32 arithmetic (FP32): A and B both f32 in 128-byte rows, on the f32
   // MFMA (32 x 32 x 2), with the register-staged kernel's k pairing.
-  static_assert(!AF || (LW == 16 && !AK && EPI == kEpiGeneric), "f32 A tiles");
+  static_assert(!AF || (LW == 16 && !AK && EPI != kEpiOpmFused), "f32 A tiles");
   static_assert(!FP32 || (LW == 16 && !AK && !AF && EPI == kEpiGeneric), "f32 tiles");
   constexpr bool A4 = AF || FP32;  // A rows of 4-byte elements
   constexpr int AROW = A4 ? 2 * kRowBytes : kRowBytes;    // bytes of a k-contiguous A row
@@ -792,10 +793,12 @@ __global__ __launch_bounds__(64 * WM * WN, FP32 && STAGES == 2 ? 4 : PAIRS && ST
       return;
     }
   }
-  // The attention blocks lengthen the row-wise epilogue of every call; the
-  // four-stage f32 tiles, whose calls take 10 us, leave them out (launch_typed
-  // sends no such call there).
-  constexpr bool kAttention = !FP32 || STAGES == 2;
+  // The attention blocks lengthen the row-wise epilogue of every call (f16
+  // linears of 9000 x 256 x 1024 and 30000 x 64 x 256 took 28.0 and 18.3 us
+  // with them on MI355X, 25.0 and 16.2 without), so f16 tiles have them in an
+  // instance of their own (launch_tile), and the four-stage f32 tiles, whose
+  // calls take 10 us, leave them out (launch_typed sends no such call there).
+  constexpr bool kAttention = EPI == kEpiAttention || (FP32 && STAGES == 2);
   if (gemm_detail::rowwise_epilogue(g) && (kAttention || !(g.flags & AFHIP_EPILOGUE_ATTENTION))) {
     // Row-wise epilogues (plain, scale, bias, attention blocks, ReLU,
     // residual, the outer-product-mean output's bias / (eps + count)) straight
@@ -885,7 +888,7 @@ __global__ __launch_bounds__(64 * WM * WN, FP32 && STAGES == 2 ? 4 : PAIRS && ST
           const int col = n0 + wn + 32 * j + 8 * g4 + 4 * (lane >> 5);
           if (col >= g.N) continue;
           float y[4] = {acc[i][j][4 * g4], acc[i][j][4 * g4 + 1], acc[i][j][4 * g4 + 2], acc[i][j][4 * g4 + 3]};
-          gemm_detail::epilogue_row4<TC>(g, bt, row, col, y, min(4, g.N - col), vec4);
+          gemm_detail::epilogue_row4<TC, kAttention>(g, bt, row, col, y, min(4, g.N - col), vec4);
         }
     }
     return;
@@ -969,6 +972,11 @@ int launch_tile(const GemmArgs& g, const char* label, hipStream_t s) {
   ka.per_xcd = (int)ceil_div(total, 8);
   const size_t shared = (size_t)STAGES * dma_stage_bytes(BM, BN, AF || FP32, FP32);
   auto kernel = gemm_dma_kernel<BM, BN, STAGES, WM, WN, PIPE, TC, kEpiGeneric, LW, AK, AF, FP32, PAIRS>;
+  // The attention projections write f16 from k-contiguous 16-byte rows; any
+  // other form passes its blocks through the element-wise epilogue.
+  if constexpr (LW == 16 && !AK && !FP32 && !PAIRS && sizeof(TC) == 2)
+    if (g.flags & AFHIP_EPILOGUE_ATTENTION)
+      kernel = gemm_dma_kernel<BM, BN, STAGES, WM, WN, PIPE, TC, kEpiAttention, LW, AK, AF, FP32, PAIRS>;
   if (int st = allow_lds((const void*)kernel, shared)) return st;
   return launch(label, kernel, dim3((unsigned)(ka.per_xcd * 8)), dim3(64 * WM * WN), shared, s, ka);
 }

@@ -236,13 +236,13 @@ __device__ __forceinline__ int attention_block4(const GemmArgs& g, int col) {
 // steps in the same order with the same roundings, written with one vector
 // access when `vec` (all four columns present, row start and ldc aligned to
 // four elements).
-template <typename TC>
+template <typename TC, bool ATTENTION>
 __device__ __forceinline__ void epilogue_row4(const GemmArgs& g, int b, int row, int col, float* y, int n, bool vec) {
 #pragma clang fp contract(off)
   const uint32_t flags = g.flags;
   float denom = 0.0f;
   if (flags & EPILOGUE_OPM_OUTPUT) denom = g.opm_eps + g.opm_count[(int64_t)g.opm_row0 + row];
-  const int block = flags & AFHIP_EPILOGUE_ATTENTION ? attention_block4(g, col) : 0;
+  const int block = ATTENTION && (flags & AFHIP_EPILOGUE_ATTENTION) ? attention_block4(g, col) : 0;
 #pragma unroll
   for (int e = 0; e < 4; e++) {
     if (e >= n) break;
