@@ -1147,6 +1147,14 @@ template <typename TC> int launch_pairs(const GemmArgs& g, const char* label, hi
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   if (!al16(g.a) || !al16(g.b))  // 4-byte loads, as for f16 rows off 16 bytes
     return launch_tile<128, 128, 5, 2, 2, false, TC, 4, false, false, false, true>(g, label, s);
+  // Fewer tiles than CUs leave each a serial chain on part of the chip: 64 x 64
+  // tiles, six stages of 8 KiB (80 k ahead), give four times the workgroups.
+  // Whole f32 transitions on MI355X (128 x 128 / this rule), us: 3000 x 64 x 256
+  // 26.4 / 15.9, 2100 x 128 x 512 35.1 / 21.2, 5000 x 256 x 1024 (80 tiles in the
+  // second linear) 57.1 / 45.7.
+  const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  if (ceil_div(g.M, 128) * ceil_div(g.N, 128) < cus)
+    return launch_tile<64, 64, 6, 2, 2, false, TC, 16, false, false, false, true>(g, label, s);
   return launch_tile<128, 128, 3, 2, 2, false, TC, 16, false, false, false, true>(g, label, s);
 }
 }  // namespace
