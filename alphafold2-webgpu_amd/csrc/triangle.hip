@@ -271,6 +271,7 @@ struct OutputArgs {
   int pairs;        // pairs in this block
   int cz, ch, czp, chp;
   int residual;
+  int in_place;  // out overlaps z (read by the launch)
   float eps;
   float x_scale, h_scale;  // the pair kernels' x_hat of z and of the contracted values
 };
@@ -734,14 +735,18 @@ template <typename ZT> int launch_project_pair(const ProjectArgs& pa, hipStream_
                 (int)rows_on_four(pa.z, pa.cz, sizeof(ZT)));
 }
 
+// In place one workgroup takes a tile's columns: every workgroup of a tile reads
+// all channels of its rows of z for the gate, and nothing orders those reads
+// before another one's stores of the same rows.
 template <typename ZT, typename OT> int launch_output_pair(const OutputArgs& oa, hipStream_t s) {
   const int64_t tiles = ceil_div(oa.pairs, kPairRows);
+  const unsigned splits = oa.in_place ? 1u : column_splits(tiles, (oa.cz + 31) / 32);
   const size_t shared =
       (size_t)kPairRows * (pair_pitch(oa.czp / 16) + pair_pitch(oa.chp / 16)) * 2 + 2 * 32 * 32 * 4;
   auto k = tri_output_pair_kernel<ZT, OT>;
   if (int st = allow_lds((const void*)k, shared)) return st;
-  return launch("triangle.output", k, dim3((unsigned)tiles, column_splits(tiles, (oa.cz + 31) / 32)), dim3(256), shared,
-                s, oa, (int)rows_on_four(oa.z, oa.cz, sizeof(ZT)));
+  return launch("triangle.output", k, dim3((unsigned)tiles, splits), dim3(256), shared, s, oa,
+                (int)rows_on_four(oa.z, oa.cz, sizeof(ZT)));
 }
 
 int dispatch_project(bool f16, int zd, const ProjectArgs& pa, size_t shared, hipStream_t s) {
@@ -925,6 +930,10 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
   const void* col_op = pa.incoming ? pa.out_a : pa.out_b;
   const size_t es = f16 ? 2 : 4;
   GemmTypes types{d.precision, f16 ? AFHIP_F16 : AFHIP_F32, f16 ? AFHIP_F16 : AFHIP_F32, f16 ? AFHIP_F16 : AFHIP_F32};
+  const size_t elements = (size_t)P * d.c_z;
+  const uintptr_t zb = reinterpret_cast<uintptr_t>(z), ob = reinterpret_cast<uintptr_t>(out);
+  const bool in_place = ob < zb + elements * (d.pair_dtype == AFHIP_F16 ? 2 : 4) &&
+                        zb < ob + elements * (d.out_dtype == AFHIP_F16 ? 2 : 4);
   const int kmax = std::max(w.chp, w.czp);
   const size_t osh = round_up((int64_t)kmax * (kRows + 1) * 4, 16) + (size_t)kRows * (kmax + 8) * 2;
   for (int i0 = 0; i0 < L; i0 += ws.block_rows) {
@@ -970,6 +979,7 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
     oa.czp = w.czp;
     oa.chp = w.chp;
     oa.residual = d.residual;
+    oa.in_place = in_place;
     oa.eps = d.epsilon;
     if (fast) {
       FastOutputArgs fo{};

@@ -318,3 +318,30 @@ def test_evoformer_block_f16_at_alphafold_widths(dev):
     assert np.abs(tm.float().cpu().numpy() - em).max() <= 1e-2 * np.abs(em).max()
     assert np.abs(tz.float().cpu().numpy() - ez).max() <= 1e-2 * np.abs(ez).max()
     ex.release()
+
+
+def test_evoformer_block_f32_at_alphafold_widths(dev):
+    # f32 at AlphaFold's widths (the kernels over pairs of f16), everything in
+    # place: column attention over more than 64 sequences, triangle tiles whose
+    # columns would be split over workgroups out of place. The bound of the small
+    # f32 block.
+    from afhip.execution import EvoformerBlock, Execution
+
+    L, S, cm, co, cz, ch = 41, 70, 256, 32, 128, 128
+    w = _block_weights(0xAF2700, cz, ch, cm, co, 4 * cz)
+    w.update(_msa_weights(0xAF2800, cm, cz))
+    msa = ref.normal(17, (S, L, cm))
+    msa_mask = (ref.uniform(18, (S, L), 0, 1) > 0.1).astype(np.float32)
+    pair_mask = (ref.uniform(19, (L, L), 0, 1) > 0.15).astype(np.float32)
+    z = ref.normal(20, (L, L, cz))
+    em, ez = _oracle_block(msa, msa_mask, z, pair_mask, w, S, L, cm, cz, False)
+    ex = Execution()
+    blk = EvoformerBlock(ex, L, sequences=S, c_m=cm, c_z=cz, c_outer=co, c_hidden=ch, precision="f32", dtype="f32")
+    blk.prepare(w)
+    pm, pmm = ex.upload("msa", msa), ex.upload("msa-mask", msa_mask)
+    pz, pzm = ex.upload("pair", z), ex.upload("pair-mask", pair_mask)
+    blk(pm, pmm, pz, pzm)
+    gm, gz = ex.download(pm, (S, L, cm)), ex.download(pz, (L, L, cz))
+    assert np.abs(gm - em).max() <= 1e-4 * np.abs(em).max()
+    assert np.abs(gz - ez).max() <= 1e-4 * np.abs(ez).max()
+    ex.release()

@@ -218,3 +218,30 @@ def test_f32_pair_kernels(dev, direction, length, cz, ch, pair_dtype, out_dtype,
     mask = torch.from_numpy(np.ascontiguousarray(inp["mask"], np.float32)).to(dev)
     out = op(place(z, pair_dtype), mask, out=place(old, out_dtype)).float().cpu().numpy()
     assert np.abs(out - expect).max() <= (1e-5 if out_dtype == "f32" else 1e-5 + 2.0 ** -11) * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("direction", ["outgoing", "incoming"])
+@pytest.mark.parametrize("length,ch,storage,block_rows", [
+    (59, 128, "f32", 0), (128, 128, "f32", 0), (100, 256, "f32", 0), (128, 256, "f16", 0), (90, 256, "f32", 0),
+    (59, 256, "f16", 7), (150, 128, "f32", 32)])
+def test_f32_in_place_is_bit_identical(dev, direction, length, ch, storage, block_rows):
+    # The pair stack runs the triangle with z as its output. Out of place, up to
+    # four workgroups share a tile of 64 pairs and each reads all 128 channels of
+    # its rows of z; in place one has to read them all before any of them is
+    # stored, and at 256 hidden channels more workgroups than the chip holds at
+    # once would be launched otherwise. The same arithmetic either way.
+    import torch
+
+    from afhip import triangle
+
+    cz = 128
+    inp = ref.deterministic_triangle_input(length, cz, ch, seed=length + ch)
+    z = torch.from_numpy(ref.round_f16(inp["z"])).to(dev)
+    z = z.half() if storage == "f16" else z
+    mask = torch.from_numpy(np.ascontiguousarray(inp["mask"], np.float32)).to(dev)
+    op = triangle.TriangleMultiplication(length, cz, ch, direction=direction, precision="f32", pair_dtype=storage,
+                                         out_dtype=storage, residual=True, block_rows=block_rows)
+    op.prepare(inp["weights"])
+    expect = op(z, mask, out=z.clone())
+    got = op(z, mask, out=z)
+    assert torch.equal(got, expect)
