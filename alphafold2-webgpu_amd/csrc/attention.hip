@@ -29,7 +29,7 @@
 // carry a factor log2(e)), which changes nothing but the rounding:
 // exp2(log2(e) x) = exp(x).
 //
-// At f32 precision with channels a multiple of 16 every product runs on the
+// At f32 precision with 64 channels or more, a multiple of 16, every product runs on the
 // f16 MFMA over pairs of f16 (gemm.h), the scales powers of two from bounds
 // that hold for any input (attention_pair_*_kernel). Any other width, or f16
 // precision with another head dimension, runs the two products of the
@@ -54,11 +54,12 @@ bool fast_path(const afhip_attention_desc& d) {
   return d.precision == AFHIP_PRECISION_F16 && (d.channels / d.heads) % 8 == 0;
 }
 
-// f32 precision over pairs: whole 16-channel blocks, and byte offsets within a
+// f32 precision over pairs: whole 16-channel blocks, projections with sums long
+// enough for it (gemm.h), and byte offsets within a
 // batch entry's f32 q, k, v, g rows in 32 bits (the flash kernel's, which
 // fetches up to 63 rows past the last before it cuts an offset back).
 bool pair_path(const afhip_attention_desc& d) {
-  return d.precision == AFHIP_PRECISION_F32 && d.channels % 16 == 0 &&
+  return d.precision == AFHIP_PRECISION_F32 && d.channels % 16 == 0 && d.channels >= kPairMinK &&
          ((int64_t)d.queries + 64) * 16 * d.channels <= (int64_t)UINT32_MAX;
 }
 

@@ -90,6 +90,14 @@ inline int pair_norm_exponent(int C) {
   while ((int64_t)1 << (2 * root) < C) root++;  // sqrt(C) <= 2^root
   return 15 - root;
 }
+// Below this many products a sum stays on the f32 MFMA. The pairs keep 22 to 24
+// bits of an operand and drop the l l term (2^-24 of a product), but a third as
+// many f32 roundings accumulate, which is worth less the shorter the sum.
+// Measured against 64 bits, operators over pairs / on the f32 MFMA (rms error):
+// transition 16 x 16 1.30, 32 x 32 1.15, 64 x 64 0.99, 256 x 1024 0.83; triangle
+// 16 x 16 1.13, 32 x 32 1.02, 64 x 64 0.91; attention over 20 keys, 16 channels
+// 1.16, 32 1.05, 64 0.93, 256 0.74; outer-product mean 16 channels 1.06, 64 0.99.
+constexpr int kPairMinK = 64;
 // The output as pairs (rows of ldc elements, 2 ldc halves) instead of TC.
 constexpr uint32_t EPILOGUE_PAIRS = 1u << 18;
 
@@ -97,9 +105,7 @@ constexpr uint32_t EPILOGUE_PAIRS = 1u << 18;
 // rows of K elements, f32 accumulation, epilogue SCALE, BIAS, ATTENTION (the
 // gate's sigmoid; q as it is), RELU and RESIDUAL (f32 or f16 outputs only) in
 // that order. N, ldc and head_cols multiples of 16, operands on 4 bytes (16 for
-// the wide loads), no batch. Against 64 bits its error is no larger than the f32 MFMA's from
-// K = 64 on: the dropped l l term is 2^-24 of a product, a third as many f32
-// roundings accumulate.
+// the wide loads), no batch, K at least kPairMinK.
 int run_gemm_pairs(const GemmArgs& args, int c_dtype, const char* label, hipStream_t stream);
 
 struct GemmTypes {

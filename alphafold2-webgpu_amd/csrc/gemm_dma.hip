@@ -1164,7 +1164,7 @@ int run_gemm_pairs(const GemmArgs& args, int c_dtype, const char* label, hipStre
   const uint32_t allowed = AFHIP_EPILOGUE_SCALE | AFHIP_EPILOGUE_BIAS | AFHIP_EPILOGUE_ATTENTION | AFHIP_EPILOGUE_RELU |
                            AFHIP_EPILOGUE_RESIDUAL | EPILOGUE_PAIRS;
   const bool pairs_out = args.flags & EPILOGUE_PAIRS;
-  if (args.M <= 0 || args.N <= 0 || args.K <= 0 || args.K % 16 || args.N % 16 || args.ldc % 16 || args.ldc < args.N ||
+  if (args.M <= 0 || args.N <= 0 || args.K < kPairMinK || args.K % 16 || args.N % 16 || args.ldc % 16 || args.ldc < args.N ||
       args.batch != 1 || !al4(args.a) || !al4(args.b) || (args.flags & ~allowed) || args.c_column_major ||
       (pairs_out && (!al4(args.c) || (args.flags & AFHIP_EPILOGUE_RESIDUAL))) ||
       ((args.flags & AFHIP_EPILOGUE_ATTENTION) && args.head_cols % 16) ||

@@ -47,6 +47,9 @@ bool fused_ok(const afhip_opm_desc& d) {
   return d.precision == AFHIP_PRECISION_F16 && d.c_outer == 32 && d.c_z > 96 && d.c_z <= 128;
 }
 
+// f32 precision projects over pairs of f16 where its sums are long enough (gemm.h).
+bool opm_pairs(const afhip_opm_desc& d) { return d.precision == AFHIP_PRECISION_F32 && d.c_m >= kPairMinK; }
+
 struct OpmWeights {
   size_t ln_scale, ln_offset, w_lr, b_lr, w_out, b_out, total;
   size_t s_lr;  // f32 precision: the pair projection's output scales
@@ -73,7 +76,7 @@ OpmWeights opm_layout(const afhip_opm_desc& d) {
   w.b_lr = take(4 * (size_t)w.cop);
   w.w_out = take(es * (size_t)w.czp * d.c_outer * d.c_outer);
   w.b_out = take(4 * (size_t)w.czp);
-  if (d.precision == AFHIP_PRECISION_F32) w.s_lr = take(4 * (size_t)w.cop);
+  if (opm_pairs(d)) w.s_lr = take(4 * (size_t)w.cop);
   w.total = at;
   return w;
 }
@@ -120,16 +123,16 @@ struct ProjectArgs {
   float eps;
 };
 
-template <typename MT>
+template <typename MT, bool F16MATH>
 __global__ __launch_bounds__(256) void opm_project_kernel(ProjectArgs a) {
-  using CT = half_t;
+  using CT = typename std::conditional<F16MATH, half_t, float>::type;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int xpitch = kRows + 1;
   float* xs = reinterpret_cast<float*>(smem);
   size_t off = round_up((int64_t)a.cmp * xpitch * 4, 16);
   CT* an = reinterpret_cast<CT*>(smem + off);
   const int apitch = a.cmp + 8;
-  off += round_up((int64_t)kRows * apitch * 2, 16);
+  if (F16MATH) off += round_up((int64_t)kRows * apitch * 2, 16);
   CT* stage = reinterpret_cast<CT*>(smem + off);
   constexpr int spitch = kRows + 8;
 
@@ -166,7 +169,8 @@ __global__ __launch_bounds__(256) void opm_project_kernel(ProjectArgs a) {
     const float rstd = fast_rsqrt(var / (float)a.cm + a.eps);
     for (int c = part; c < a.cmp; c += 4) {
       float v = c < a.cm ? (xs[c * xpitch + q] - mean) * rstd * a.ln_scale[c] + a.ln_offset[c] : 0.0f;
-      an[q * apitch + c] = (CT)v;
+      if (F16MATH) an[q * apitch + c] = (CT)v;
+      else xs[c * xpitch + q] = v;
     }
   }
   __syncthreads();
@@ -179,11 +183,18 @@ __global__ __launch_bounds__(256) void opm_project_kernel(ProjectArgs a) {
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[v] = 0.0f;
     const int n = nc + (lane & 31);
-    for (int k = 0; k < a.cmp; k += 16) {
-      const int kk = k + 8 * (lane >> 5);
-      half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
-      half8 bf = *reinterpret_cast<const half8*>(W + (size_t)n * a.cmp + kk);
-      acc = mfma_f16(af, bf, acc);
+    if constexpr (F16MATH) {
+      for (int k = 0; k < a.cmp; k += 16) {
+        const int kk = k + 8 * (lane >> 5);
+        half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
+        half8 bf = *reinterpret_cast<const half8*>(W + (size_t)n * a.cmp + kk);
+        acc = mfma_f16(af, bf, acc);
+      }
+    } else {
+      for (int k = 0; k < a.cmp; k += 2) {
+        const int kk = k + (lane >> 5);
+        acc = mfma_f32(xs[kk * xpitch + rw + (lane & 31)], W[(size_t)n * a.cmp + kk], acc);
+      }
     }
     const float bias = a.b_lr[n];
 #pragma unroll
@@ -213,7 +224,7 @@ __global__ __launch_bounds__(256) void opm_project_kernel(ProjectArgs a) {
   }
 }
 
-// f32 precision: the projection over pairs of f16 (pairs.h), any c_m <= 512.
+// f32 precision, c_m >= 64: the projection over pairs of f16 (pairs.h).
 // Wave (rows 32 (w % 2).., column block w / 2 of each two) computes W x_hat^T, so
 // a lane ends with one (residue, sequence) row and 16 channels and each store
 // of a channel is up to 32 consecutive sequences. Before, 64-row tiles on the
@@ -635,9 +646,12 @@ template <typename MT> int launch_project_pair(const ProjectArgs& pa, hipStream_
   return pa.cmp <= 256 ? launch_project_pair_steps<MT, 16>(pa, s) : launch_project_pair_steps<MT, 32>(pa, s);
 }
 
-template <typename MT> int launch_project(const ProjectArgs& pa, size_t shared, hipStream_t s) {
-  if (int st = allow_lds((const void*)opm_project_kernel<MT>, shared)) return st;
-  return launch("opm.project", opm_project_kernel<MT>, dim3((unsigned)ceil_div((int64_t)pa.S * pa.L, kRows)),
+template <typename MT, bool F16MATH> int launch_project(const ProjectArgs& pa, hipStream_t s) {
+  const size_t shared = round_up((int64_t)pa.cmp * (kRows + 1) * 4, 16) +
+                        (F16MATH ? round_up((int64_t)kRows * (pa.cmp + 8) * 2, 16) : 0) +
+                        (size_t)64 * (kRows + 8) * (F16MATH ? 2 : 4);
+  if (int st = allow_lds((const void*)opm_project_kernel<MT, F16MATH>, shared)) return st;
+  return launch("opm.project", opm_project_kernel<MT, F16MATH>, dim3((unsigned)ceil_div((int64_t)pa.S * pa.L, kRows)),
                 dim3(256), shared, s, pa);
 }
 
@@ -685,6 +699,7 @@ int afhip_opm_prepare_weights(const afhip_opm_desc* desc, const float* packed, v
                        (float*)(base + w.w_out), (float*)(base + w.b_out), ln_s, ln_o, false))
       return s;
     // The projection's weights again, as pairs over the f32 ones.
+    if (!opm_pairs(d)) return AFHIP_OK;
     if (int s = launch("opm.prepare", opm_pair_prepare_kernel, dim3(w.cop), dim3(64), 0, st, packed, d.c_m, d.c_outer,
                        w.cmp, pair_norm_exponent(d.c_m), (half_t*)(base + w.w_lr), (float*)(base + w.s_lr),
                        (float*)(base + w.b_lr)))
@@ -728,8 +743,6 @@ int afhip_opm_run(const afhip_opm_desc* desc, const void* activations, const flo
   pa.eps = d.layer_norm_epsilon;
   pa.s_lr = (const float*)(wb + w.s_lr);
   pa.x_scale = ldexpf(1.0f, pair_norm_exponent(d.c_m));
-  const size_t psh = round_up((int64_t)w.cmp * (kRows + 1) * 4, 16) + round_up((int64_t)kRows * (w.cmp + 8) * 2, 16) +
-                     (size_t)64 * (kRows + 8) * 2;
   int s;
   float* count = (float*)(wsb + ws.count);
   // The fast projection computes the pair counts in the same launch.
@@ -737,7 +750,9 @@ int afhip_opm_run(const afhip_opm_desc* desc, const void* activations, const flo
   if (fast)
     s = d.msa_dtype == AFHIP_F32 ? launch_fast_cm<float>(pa, count, st) : launch_fast_cm<half_t>(pa, count, st);
   else if (f16)
-    s = d.msa_dtype == AFHIP_F32 ? launch_project<float>(pa, psh, st) : launch_project<half_t>(pa, psh, st);
+    s = d.msa_dtype == AFHIP_F32 ? launch_project<float, true>(pa, st) : launch_project<half_t, true>(pa, st);
+  else if (!opm_pairs(d))
+    s = d.msa_dtype == AFHIP_F32 ? launch_project<float, false>(pa, st) : launch_project<half_t, false>(pa, st);
   else
     s = d.msa_dtype == AFHIP_F32 ? launch_project_pair<float>(pa, st) : launch_project_pair<half_t>(pa, st);
   if (s) return s;

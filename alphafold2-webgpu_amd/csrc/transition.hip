@@ -23,10 +23,11 @@ struct TransitionWeights {
   size_t s1, s2, shift;  // the pair path's output scales and hidden exponents
 };
 
-// The pair path (f32 precision): whole 16-channel blocks both ways.
+// The pair path (f32 precision): whole 16-channel blocks both ways, sums long
+// enough for it (gemm.h).
 bool pair_shape(const afhip_transition_desc& d) {
-  return d.precision == AFHIP_PRECISION_F32 && d.channels % 16 == 0 && d.hidden % 16 == 0 && d.channels <= (1 << 16) &&
-         d.hidden <= (1 << 20);
+  return d.precision == AFHIP_PRECISION_F32 && d.channels % 16 == 0 && d.hidden % 16 == 0 &&
+         std::min(d.channels, d.hidden) >= kPairMinK && d.channels <= (1 << 16) && d.hidden <= (1 << 20);
 }
 
 TransitionWeights layout(const afhip_transition_desc& d) {

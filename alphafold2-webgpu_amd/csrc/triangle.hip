@@ -18,8 +18,8 @@
 //     of z are normalised and projected by linearG; out = (p + bz)*sig(g + bg).
 //     The gate is recomputed here from z rather than stored and re-read.
 //
-// At f32 precision 1 and 3 multiply pairs of f16 on the f16 MFMA (gemm.h; the
-// tri_*_pair kernels below); the contraction is the f32 GEMM.
+// At f32 precision with 64 channels or more 1 and 3 multiply pairs of f16 on the
+// f16 MFMA (gemm.h; the tri_*_pair kernels below); the contraction is the f32 GEMM.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -35,11 +35,18 @@ namespace {
 constexpr int kRows = 64;  // pair rows per workgroup in the projection kernels
 constexpr int kC = 128;    // the fast path's c_z = c_hidden
 
+// The projections' products. f32 precision multiplies pairs of f16 where both
+// of its sums are long enough (gemm.h).
+enum class Products { kF16, kF32, kPairs };
+bool tri_pairs(const afhip_triangle_desc& d) {
+  return d.precision == AFHIP_PRECISION_F32 && std::min(d.c_z, d.c_hidden) >= kPairMinK;
+}
+
 struct TriWeights {
   // Offsets in bytes into the prepared buffer.
   size_t ln_in_w, ln_in_b, w_proj, b_proj, ln_out_w, ln_out_b, w_z, b_z, w_g, b_g;
   size_t fold_w, fold_b;  // the f16 fast path's folded weights (0 when not eligible)
-  size_t s_proj, s_z, s_g;  // f32 precision: output scales of the pair products
+  size_t s_proj, s_z, s_g;  // over pairs: output scales of the pair products
   size_t total;
   int czp, chp, czo;  // padded input width (multiple of 32), padded hidden, padded output rows
 };
@@ -66,7 +73,7 @@ TriWeights tri_layout(const afhip_triangle_desc& d) {
   w.b_z = take(4 * (size_t)w.czo);
   w.w_g = take(es * (size_t)w.czo * w.czp);
   w.b_g = take(4 * (size_t)w.czo);
-  if (d.precision == AFHIP_PRECISION_F32) {
+  if (tri_pairs(d)) {
     w.s_proj = take(4 * 4 * (size_t)w.chp);
     w.s_z = take(4 * (size_t)w.czo);
     w.s_g = take(4 * (size_t)w.czo);
@@ -158,18 +165,18 @@ struct ProjectArgs {
   float x_scale;  // the pair kernels hold x_hat times this
 };
 
-template <typename ZT>
+template <typename ZT, bool F16MATH>
 __global__ __launch_bounds__(256) void tri_project_kernel(ProjectArgs a) {
-  using CT = half_t;
+  using CT = typename std::conditional<F16MATH, half_t, float>::type;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  // xs: f32 [czp][kRows + 1], channel-major raw z; an: CT [kRows][czp + 8];
+  // xs: f32 [czp][kRows + 1], channel-major raw z; an: CT [kRows][czp + 8] (f16 only);
   // stage: CT [64][kRows + 8] output transpose.
   const int xpitch = kRows + 1;
   float* xs = reinterpret_cast<float*>(smem);
   size_t off = round_up((int64_t)a.czp * xpitch * 4, 16);
   CT* an = reinterpret_cast<CT*>(smem + off);
   const int apitch = a.czp + 8;
-  off += round_up((int64_t)kRows * apitch * 2, 16);
+  if (F16MATH) off += round_up((int64_t)kRows * apitch * 2, 16);
   CT* stage = reinterpret_cast<CT*>(smem + off);
   constexpr int spitch = kRows + 8;
 
@@ -195,7 +202,8 @@ __global__ __launch_bounds__(256) void tri_project_kernel(ProjectArgs a) {
     const int q = tid >> 2, part = tid & 3;
     for (int c = part; c < a.czp; c += 4) {
       float v = c < a.cz ? (xs[c * xpitch + q] - mean) * rstd * a.ln_w[c] + a.ln_b[c] : 0.0f;
-      an[q * apitch + c] = (CT)v;
+      if (F16MATH) an[q * apitch + c] = (CT)v;
+      else xs[c * xpitch + q] = v;
     }
   }
   __syncthreads();
@@ -215,13 +223,22 @@ __global__ __launch_bounds__(256) void tri_project_kernel(ProjectArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; v++) accp[v] = accg[v] = 0.0f;
         const int n = hc + (lane & 31);
-        for (int k = 0; k < a.czp; k += 16) {
-          const int kk = k + 8 * (lane >> 5);
-          half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
-          half8 bpf = *reinterpret_cast<const half8*>(wp + (size_t)n * a.czp + kk);
-          half8 bgf = *reinterpret_cast<const half8*>(wg + (size_t)n * a.czp + kk);
-          accp = mfma_f16(af, bpf, accp);
-          accg = mfma_f16(af, bgf, accg);
+        if constexpr (F16MATH) {
+          for (int k = 0; k < a.czp; k += 16) {
+            const int kk = k + 8 * (lane >> 5);
+            half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
+            half8 bpf = *reinterpret_cast<const half8*>(wp + (size_t)n * a.czp + kk);
+            half8 bgf = *reinterpret_cast<const half8*>(wg + (size_t)n * a.czp + kk);
+            accp = mfma_f16(af, bpf, accp);
+            accg = mfma_f16(af, bgf, accg);
+          }
+        } else {
+          for (int k = 0; k < a.czp; k += 2) {
+            const int kk = k + (lane >> 5);
+            float af = xs[kk * xpitch + rw + (lane & 31)];
+            accp = mfma_f32(af, wp[(size_t)n * a.czp + kk], accp);
+            accg = mfma_f32(af, wg[(size_t)n * a.czp + kk], accg);
+          }
         }
         const float bpv = bp[n], bgv = bg[n];
 #pragma unroll
@@ -276,9 +293,10 @@ struct OutputArgs {
   float x_scale, h_scale;  // the pair kernels' x_hat of z and of the contracted values
 };
 
-// Normalises 64 columns of a channel-major tile (xs[c][q]) into an[q][c].
-// Returns after a barrier.
-__device__ __forceinline__ void normalize_tile(float* xs, int xpitch, half_t* an, int apitch, int channels, int padded,
+// Loads 64 columns of a channel-major tile (xs[c][q]) and normalises them in
+// place (f32) or into an[q][c] (f16). Returns after a barrier.
+template <typename CT, bool F16MATH>
+__device__ __forceinline__ void normalize_tile(float* xs, int xpitch, CT* an, int apitch, int channels, int padded,
                                                const float* w, const float* b, float eps, int tid) {
   float mean, rstd;
   column_stats(xs, xpitch, channels, eps, tid, mean, rstd);
@@ -286,32 +304,41 @@ __device__ __forceinline__ void normalize_tile(float* xs, int xpitch, half_t* an
   __syncthreads();
   for (int c = part; c < padded; c += 4) {
     float v = c < channels ? (xs[c * xpitch + q] - mean) * rstd * w[c] + b[c] : 0.0f;
-    an[q * apitch + c] = (half_t)v;
+    if (F16MATH) an[q * apitch + c] = (CT)v;
+    else xs[c * xpitch + q] = v;
   }
   __syncthreads();
 }
 
 // acc[t] += A (64 x K from LDS) * W^T for the wave's column tiles.
-__device__ __forceinline__ void tile_gemm(floatx16 (&acc)[2], const half_t* an, int apitch, const half_t* W, int K,
-                                          int czo, int lane, int wave) {
+template <typename CT, bool F16MATH>
+__device__ __forceinline__ void tile_gemm(floatx16 (&acc)[2], const float* xs, int xpitch, const CT* an, int apitch,
+                                          const CT* W, int K, int czo, int lane, int wave) {
   const int rw = 32 * (wave & 1);
 #pragma unroll
   for (int t = 0; t < 2; t++) {
     const int j = (wave >> 1) + 2 * t;
     if (32 * j >= czo) continue;
     const int n = 32 * j + (lane & 31);
-    for (int k = 0; k < K; k += 16) {
-      const int kk = k + 8 * (lane >> 5);
-      half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
-      half8 bf = *reinterpret_cast<const half8*>(W + (size_t)n * K + kk);
-      acc[t] = mfma_f16(af, bf, acc[t]);
+    if constexpr (F16MATH) {
+      for (int k = 0; k < K; k += 16) {
+        const int kk = k + 8 * (lane >> 5);
+        half8 af = *reinterpret_cast<const half8*>(an + (rw + (lane & 31)) * apitch + kk);
+        half8 bf = *reinterpret_cast<const half8*>(W + (size_t)n * K + kk);
+        acc[t] = mfma_f16(af, bf, acc[t]);
+      }
+    } else {
+      for (int k = 0; k < K; k += 2) {
+        const int kk = k + (lane >> 5);
+        acc[t] = mfma_f32(xs[kk * xpitch + rw + (lane & 31)], W[(size_t)n * K + kk], acc[t]);
+      }
     }
   }
 }
 
-template <typename ZT, typename OT>
+template <typename ZT, typename OT, bool F16MATH>
 __global__ __launch_bounds__(256) void tri_output_kernel(OutputArgs a) {
-  using CT = half_t;
+  using CT = typename std::conditional<F16MATH, half_t, float>::type;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int xpitch = kRows + 1;
   const int kmax = a.chp > a.czp ? a.chp : a.czp;
@@ -332,13 +359,14 @@ __global__ __launch_bounds__(256) void tri_output_kernel(OutputArgs a) {
     xs[c * xpitch + q] = v;
   }
   __syncthreads();
-  normalize_tile(xs, xpitch, an, apitch, a.ch, a.chp, a.ln_out_w, a.ln_out_b, a.eps, tid);
+  normalize_tile<CT, F16MATH>(xs, xpitch, an, apitch, a.ch, a.chp, a.ln_out_w, a.ln_out_b, a.eps, tid);
   floatx16 accz[2], accg[2];
 #pragma unroll
   for (int t = 0; t < 2; t++)
 #pragma unroll
     for (int v = 0; v < 16; v++) accz[t][v] = accg[t][v] = 0.0f;
-  tile_gemm(accz, an, apitch, reinterpret_cast<const CT*>(a.w_z), a.chp, (int)round_up(a.cz, 32), lane, wave);
+  tile_gemm<CT, F16MATH>(accz, xs, xpitch, an, apitch, reinterpret_cast<const CT*>(a.w_z), a.chp,
+                         (int)round_up(a.cz, 32), lane, wave);
   __syncthreads();
 
   // Phase 2: the same pairs of z, transposed to channel-major.
@@ -349,8 +377,9 @@ __global__ __launch_bounds__(256) void tri_output_kernel(OutputArgs a) {
     xs[c * xpitch + q] = v;
   }
   __syncthreads();
-  normalize_tile(xs, xpitch, an, apitch, a.cz, a.czp, a.ln_in_w, a.ln_in_b, a.eps, tid);
-  tile_gemm(accg, an, apitch, reinterpret_cast<const CT*>(a.w_g), a.czp, (int)round_up(a.cz, 32), lane, wave);
+  normalize_tile<CT, F16MATH>(xs, xpitch, an, apitch, a.cz, a.czp, a.ln_in_w, a.ln_in_b, a.eps, tid);
+  tile_gemm<CT, F16MATH>(accg, xs, xpitch, an, apitch, reinterpret_cast<const CT*>(a.w_g), a.czp,
+                         (int)round_up(a.cz, 32), lane, wave);
 
   OT* out = reinterpret_cast<OT*>(a.out);
   const int rw = 32 * (wave & 1);
@@ -373,10 +402,10 @@ __global__ __launch_bounds__(256) void tri_output_kernel(OutputArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// f32 precision: both projections over pairs of f16
+// f32 precision, c_z and c_hidden >= 64: both projections over pairs of f16
 // ---------------------------------------------------------------------------
 //
-// The f32 kernels before these ran the f32 MFMA, one 64-pair tile a workgroup
+// The f32 kernels above run the f32 MFMA, one 64-pair tile a workgroup
 // through all four (two) matrices, with the weights read element by element in
 // the middle of the MFMA chain: at L = 59, 55 of 256 CUs worked through 32k
 // cycles of MFMA each. Here a tile's columns are split over as many workgroups
@@ -707,16 +736,18 @@ int validate(const afhip_triangle_desc* d) {
   return AFHIP_OK;
 }
 
-template <typename ZT> int launch_project(const ProjectArgs& pa, size_t shared, hipStream_t s) {
-  if (int st = allow_lds((const void*)tri_project_kernel<ZT>, shared)) return st;
-  return launch("triangle.project", tri_project_kernel<ZT>, dim3((unsigned)ceil_div(pa.P, kRows)), dim3(256), shared, s,
-                pa);
+template <typename ZT, bool F16MATH>
+int launch_project(const ProjectArgs& pa, size_t shared, hipStream_t s) {
+  if (int st = allow_lds((const void*)tri_project_kernel<ZT, F16MATH>, shared)) return st;
+  return launch("triangle.project", tri_project_kernel<ZT, F16MATH>, dim3((unsigned)ceil_div(pa.P, kRows)),
+                dim3(256), shared, s, pa);
 }
 
-template <typename ZT, typename OT> int launch_output(const OutputArgs& oa, size_t shared, hipStream_t s) {
-  if (int st = allow_lds((const void*)tri_output_kernel<ZT, OT>, shared)) return st;
-  return launch("triangle.output", tri_output_kernel<ZT, OT>, dim3((unsigned)ceil_div(oa.pairs, kRows)), dim3(256),
-                shared, s, oa);
+template <typename ZT, typename OT, bool F16MATH>
+int launch_output(const OutputArgs& oa, size_t shared, hipStream_t s) {
+  if (int st = allow_lds((const void*)tri_output_kernel<ZT, OT, F16MATH>, shared)) return st;
+  return launch("triangle.output", tri_output_kernel<ZT, OT, F16MATH>, dim3((unsigned)ceil_div(oa.pairs, kRows)),
+                dim3(256), shared, s, oa);
 }
 
 // How many workgroups share a tile's column blocks: enough for two a CU, as
@@ -749,19 +780,20 @@ template <typename ZT, typename OT> int launch_output_pair(const OutputArgs& oa,
                 (int)rows_on_four(oa.z, oa.cz, sizeof(ZT)));
 }
 
-int dispatch_project(bool f16, int zd, const ProjectArgs& pa, size_t shared, hipStream_t s) {
-  if (!f16) return zd == AFHIP_F32 ? launch_project_pair<float>(pa, s) : launch_project_pair<half_t>(pa, s);
-  return zd == AFHIP_F32 ? launch_project<float>(pa, shared, s) : launch_project<half_t>(pa, shared, s);
+template <bool F16MATH, typename ZT> int launch_output_to(int od, const OutputArgs& oa, size_t shared, hipStream_t s) {
+  return od == AFHIP_F32 ? launch_output<ZT, float, F16MATH>(oa, shared, s)
+                         : launch_output<ZT, half_t, F16MATH>(oa, shared, s);
 }
 
-template <typename ZT> int dispatch_output_to(bool f16, int od, const OutputArgs& oa, size_t shared, hipStream_t s) {
-  if (!f16) return od == AFHIP_F32 ? launch_output_pair<ZT, float>(oa, s) : launch_output_pair<ZT, half_t>(oa, s);
-  return od == AFHIP_F32 ? launch_output<ZT, float>(oa, shared, s) : launch_output<ZT, half_t>(oa, shared, s);
+template <typename ZT> int dispatch_project(Products p, const ProjectArgs& pa, size_t shared, hipStream_t s) {
+  if (p == Products::kPairs) return launch_project_pair<ZT>(pa, s);
+  return p == Products::kF16 ? launch_project<ZT, true>(pa, shared, s) : launch_project<ZT, false>(pa, shared, s);
 }
 
-int dispatch_output(bool f16, int zd, int od, const OutputArgs& oa, size_t shared, hipStream_t s) {
-  return zd == AFHIP_F32 ? dispatch_output_to<float>(f16, od, oa, shared, s)
-                         : dispatch_output_to<half_t>(f16, od, oa, shared, s);
+template <typename ZT> int dispatch_output(Products p, int od, const OutputArgs& oa, size_t shared, hipStream_t s) {
+  if (p == Products::kPairs) return od == AFHIP_F32 ? launch_output_pair<ZT, float>(oa, s) : launch_output_pair<ZT, half_t>(oa, s);
+  return p == Products::kF16 ? launch_output_to<true, ZT>(od, oa, shared, s)
+                             : launch_output_to<false, ZT>(od, oa, shared, s);
 }
 
 }  // namespace
@@ -809,7 +841,7 @@ int afhip_triangle_prepare_weights(const afhip_triangle_desc* desc, const float*
   o[0] = 0;
   for (int i = 0; i < 16; i++) o[i + 1] = o[i] + sizes[i];
   char* base = (char*)prepared;
-  if (d.precision == AFHIP_PRECISION_F32) {
+  if (tri_pairs(d)) {
     // ORDER indices as below; the pair kernels need nothing else.
     PairSources src{};
     auto matrix = [&](int at, int index, int norm, int rows, int cols, int padded, int steps, size_t out, size_t scale,
@@ -825,9 +857,11 @@ int afhip_triangle_prepare_weights(const afhip_triangle_desc* desc, const float*
     matrix(5, 14, 0, cz, cz, w.czo, w.czp / 16, w.w_g, w.s_g, w.b_g);
     return launch("tri_prepare", tri_pair_prepare_kernel, dim3((unsigned)std::max(w.chp, w.czo), 6), dim3(64), 0, st, src);
   }
-  const size_t es = 2;
+  const bool f16 = d.precision == AFHIP_PRECISION_F16;
+  const size_t es = f16 ? 2 : 4;
   auto mat = [&](int index, int rows, int cols, size_t dst, int prow, int pcol) {
-    return pad_matrix<half_t>(packed + o[index], rows, cols, base + dst, prow, pcol, st);
+    return f16 ? pad_matrix<half_t>(packed + o[index], rows, cols, base + dst, prow, pcol, st)
+               : pad_matrix<float>(packed + o[index], rows, cols, base + dst, prow, pcol, st);
   };
   int s;
   if ((s = pad_vector(packed + o[0], cz, base + w.ln_in_w, cz, st))) return s;
@@ -875,6 +909,7 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
                 workspace_bytes, ws.total);
   hipStream_t st = (hipStream_t)stream;
   const bool f16 = d.precision == AFHIP_PRECISION_F16;
+  const Products products = f16 ? Products::kF16 : tri_pairs(d) ? Products::kPairs : Products::kF32;
   const char* wb = (const char*)prepared;
   char* wsb = (char*)workspace;
   const int L = d.length;
@@ -920,8 +955,9 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
     s = launch_triangle_project_f16(fa, d.pair_dtype, st);
   } else {
     const size_t psh = round_up((int64_t)w.czp * (kRows + 1) * 4, 16) +
-                       round_up((int64_t)kRows * (w.czp + 8) * 2, 16) + (size_t)64 * (kRows + 8) * 2;
-    s = dispatch_project(f16, d.pair_dtype, pa, psh, st);
+                       (f16 ? round_up((int64_t)kRows * (w.czp + 8) * 2, 16) : 0) + (size_t)64 * (kRows + 8) * (f16 ? 2 : 4);
+    s = d.pair_dtype == AFHIP_F32 ? dispatch_project<float>(products, pa, psh, st)
+                                  : dispatch_project<half_t>(products, pa, psh, st);
   }
   if (s) return s;
 
@@ -935,7 +971,7 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
   const bool in_place = ob < zb + elements * (d.pair_dtype == AFHIP_F16 ? 2 : 4) &&
                         zb < ob + elements * (d.out_dtype == AFHIP_F16 ? 2 : 4);
   const int kmax = std::max(w.chp, w.czp);
-  const size_t osh = round_up((int64_t)kmax * (kRows + 1) * 4, 16) + (size_t)kRows * (kmax + 8) * 2;
+  const size_t osh = round_up((int64_t)kmax * (kRows + 1) * 4, 16) + (f16 ? (size_t)kRows * (kmax + 8) * 2 : 0);
   for (int i0 = 0; i0 < L; i0 += ws.block_rows) {
     const int count = std::min(ws.block_rows, L - i0);
     GemmArgs g;
@@ -997,7 +1033,8 @@ int afhip_triangle_run(const afhip_triangle_desc* desc, const void* z, const flo
       fo.eps = d.epsilon;
       s = launch_triangle_output_f16(fo, d.pair_dtype, d.out_dtype, st);
     } else {
-      s = dispatch_output(f16, d.pair_dtype, d.out_dtype, oa, osh, st);
+      s = d.pair_dtype == AFHIP_F32 ? dispatch_output<float>(products, d.out_dtype, oa, osh, st)
+                                    : dispatch_output<half_t>(products, d.out_dtype, oa, osh, st);
     }
     if (s) return s;
   }

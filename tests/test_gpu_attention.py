@@ -356,12 +356,12 @@ def test_f32_mfma_flash_edges(dev, name, S, L, C, H, precision):
     assert np.abs(got - expect).max() <= (7e-5 if precision == "f32" else 1e-2) * np.abs(expect).max()
 
 
-@pytest.mark.parametrize("C,H", [(16, 4), (80, 16), (48, 4), (64, 4), (112, 4), (128, 4), (96, 32)])
+@pytest.mark.parametrize("C,H", [(16, 4), (80, 16), (48, 4), (64, 4), (112, 4), (128, 4), (96, 32), (144, 12), (64, 16)])
 @pytest.mark.parametrize("name,S,L,residual,shift", [("msa_column", 33, 2, True, 1), ("triangle_start", 0, 65, False, 0),
                                                      ("triangle_end", 0, 31, True, 0), ("msa_row", 3, 32, False, 1)])
 def test_f32_pairs_attention(dev, name, S, L, residual, shift, C, H):
-    # f32 precision over pairs of f16: head dimensions 4, 5, 12, 16, 28, 32 and
-    # 3 (chunked and element-wise loads, one and two steps of 16 channels),
+    # f32 precision over pairs of f16 (16 and 48 channels stay on the f32 MFMA):
+    # head dimensions 4, 5, 12, 16, 28, 32 and 3 (chunked and element-wise loads, one and two steps of 16 channels),
     # ragged query and key blocks, fully masked rows, the residual, and the
     # weights and the workspace on 4 bytes (shift). The LayerNorm scales and the
     # projections' columns carry factors of 1e-6 to 1e6 that cancel (queries
@@ -442,3 +442,20 @@ def test_f32_pairs_shared_key_blocks(dev, name, S, L, scale):
     expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
     got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb)
     assert np.abs(got - expect).max() <= 7e-5 * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("C,H", [(16, 1), (32, 4), (48, 12)])
+def test_f32_keeps_every_bit_of_short_sums(dev, C, H):
+    # Below 64 channels the products stay on the f32 MFMA: with rows that the
+    # LayerNorm takes to +-1, one key, one weight a value channel, open gates and an identity for
+    # the output projection, the outputs are those weights, all 24 bits of them.
+    # Pairs of f16 hold one in four to 23 bits.
+    B = 5
+    x = np.where(np.indices((B, C)).sum(0) % 2 == 0, 2.0 ** 20, -2.0 ** 20).astype(np.float32)
+    v = np.float32(1) + (2 * np.floor(ref.uniform(C, (C,), 0, 2 ** 22)) + 1).astype(np.float32) * np.float32(2 ** -23)
+    w = {"queryNormScale": np.ones(C, np.float32), "queryNormOffset": np.zeros(C, np.float32),
+         **{k + "Weight": np.zeros((C, C), np.float32) for k in ("query", "key", "gating")},
+         "valueWeight": np.diag(v), "gatingBias": np.full(C, 200, np.float32),
+         "outputWeight": np.eye(C, dtype=np.float32), "outputBias": np.zeros(C, np.float32)}
+    got = run_case(dev, x.reshape(-1), np.ones(B, np.float32), B, 1, C, H, True, w, None)
+    assert np.array_equal(got.reshape(B, C), np.sign(x) * v)

@@ -344,11 +344,13 @@ def test_invalid_opm_and_transition_raise(dev):
 @pytest.mark.parametrize("rows,c,h,in_dt,out_dt,residual,shift", [
     (1, 16, 16, "f32", "f32", False, 0), (31, 16, 48, "f32", "f32", True, 1), (129, 48, 80, "f32", "f32", False, 1),
     (300, 64, 256, "f16", "f32", True, 0), (257, 128, 512, "f32", "f16", True, 1), (130, 256, 1024, "f32", "f32", True, 0),
-    (65, 40, 64, "f32", "f32", False, 0), (16500, 16, 272, "f32", "f32", False, 0), (16500, 256, 64, "f32", "f32", True, 0)])
+    (65, 40, 64, "f32", "f32", False, 0), (16500, 16, 272, "f32", "f32", False, 0), (16500, 256, 64, "f32", "f32", True, 0),
+    (1, 64, 64, "f32", "f32", False, 0), (31, 64, 80, "f32", "f32", True, 1), (129, 112, 144, "f32", "f32", False, 1),
+    (16500, 80, 272, "f32", "f32", True, 1)])
 def test_transition_f32_pairs(dev, rows, c, h, in_dt, out_dt, residual, shift):
     # f32 precision on the f16 matrix units: ragged row and column tiles, both
     # LayerNorm kernels, activations and outputs off 16-byte alignment (shift
-    # elements; the workspace and the weights then lie on 4 bytes), f16 in or out, the residual; 40 channels keep the f32
+    # elements; the workspace and the weights then lie on 4 bytes), f16 in or out, the residual. 16, 40 and 48 channels keep the f32
     # GEMM, and 16500 rows fill the chip with 128 x 128 tiles (fewer run on 64 x 64). The LayerNorm scales, the first linear's columns and the
     # second's rows carry factors of 1e-6 to 1e6 that cancel in the result, as
     # any weight may: the powers of two that the pairs are stored with follow
@@ -387,11 +389,12 @@ def test_transition_f32_pairs(dev, rows, c, h, in_dt, out_dt, residual, shift):
 
 
 @pytest.mark.parametrize("S,L,cm,co,cz,msa_dtype,shift", [(1, 3, 512, 32, 16, "f32", 0), (65, 2, 300, 20, 8, "f16", 1),
-                                                          (31, 9, 17, 40, 12, "f32", 3), (64, 70, 64, 32, 128, "f32", 0)])
+                                                          (31, 9, 17, 40, 12, "f32", 3), (64, 70, 64, 32, 128, "f32", 0),
+                                                          (31, 9, 67, 40, 12, "f32", 3)])
 def test_opm_f32_pair_projection(dev, S, L, cm, co, cz, msa_dtype, shift):
     # f32 precision's projection over pairs of f16: one to two column blocks of
     # 64, ragged tiles whose rows cross residues, channels short of their padding
-    # and up to 512, the MSA off 16-byte alignment (shift elements). The
+    # and up to 512 (17 stay on the f32 MFMA), the MSA off 16-byte alignment (shift elements). The
     # LayerNorm's scales and the columns of the weights it feeds carry factors of
     # 1e-6 to 1e6 that cancel. The f32 bound of the other tests.
     import torch
@@ -413,3 +416,60 @@ def test_opm_f32_pair_projection(dev, S, L, cm, co, cz, msa_dtype, shift):
     flat[shift:] = torch.from_numpy(act).to(dev).reshape(-1)
     out = op(flat[shift:].reshape(S, L, cm), torch.from_numpy(mask).to(dev)).cpu().numpy()
     assert np.abs(out - expect).max() <= 1e-5 * np.abs(expect).max()
+
+
+def _exact_weights(n, seed):
+    # 24-bit significands, the last bit set
+    return np.float32(1) + (2 * np.floor(ref.uniform(seed, (n,), 0, 2 ** 22)) + 1).astype(np.float32) * np.float32(2 ** -23)
+
+
+def _signs(shape, scale=2.0 ** 20):
+    # Rows that a LayerNorm takes to +-1 exactly: mean 0, variance scale^2.
+    return np.where(np.indices(shape).sum(0) % 2 == 0, scale, -scale).astype(np.float32)
+
+
+@pytest.mark.parametrize("c,h", [(16, 16), (32, 128), (48, 64), (64, 48), (256, 16), (16, 1024)])
+def test_transition_f32_keeps_every_bit_of_short_sums(dev, c, h):
+    # Below 64 products the sums stay on the f32 MFMA: with rows of +-1 and one
+    # weight a hidden unit the outputs are the weights, all 24 bits of them, and zero where the
+    # ReLU cuts. Pairs of f16 hold one in four of these to 23 bits.
+    import torch
+
+    from afhip import transition
+
+    x = _signs((6, c))
+    n = min(c, h)
+    w = {"layerNormScale": np.ones(c, np.float32), "layerNormOffset": np.zeros(c, np.float32),
+         "firstWeight": np.zeros((c, h), np.float32), "firstBias": np.zeros(h, np.float32),
+         "secondWeight": np.zeros((h, c), np.float32), "secondBias": np.zeros(c, np.float32)}
+    v = _exact_weights(n, 31 + c)
+    w["firstWeight"][np.arange(n), np.arange(n)] = v
+    w["secondWeight"][np.arange(n), np.arange(n)] = 1
+    expect = np.zeros((6, c), np.float32)
+    expect[:, :n] = np.maximum(np.sign(x[:, :n]) * v, 0)
+    op = transition.Transition(6, c, h)
+    op.prepare(w)
+    assert np.array_equal(op(torch.from_numpy(x).to(dev)).cpu().numpy(), expect)
+
+
+@pytest.mark.parametrize("cm", [16, 34, 62])
+def test_opm_f32_keeps_every_bit_of_short_sums(dev, cm):
+    # As above: one sequence, one weight a left channel, right channels of 1.
+    import torch
+
+    from afhip import opm
+
+    L, co = 3, 8
+    m = _signs((1, L, cm))
+    v = _exact_weights(co, 57 + cm)
+    w = {"layerNormScale": np.ones(cm, np.float32), "layerNormOffset": np.zeros(cm, np.float32),
+         "leftWeight": np.zeros((cm, co), np.float32), "leftBias": np.zeros(co, np.float32),
+         "rightWeight": np.zeros((cm, co), np.float32), "rightBias": np.ones(co, np.float32),
+         "outputWeight": np.zeros((co * co, co), np.float32), "outputBias": np.zeros(co, np.float32)}
+    w["leftWeight"][np.arange(co), np.arange(co)] = v
+    w["outputWeight"][np.arange(co) * co, np.arange(co)] = 1
+    expect = np.repeat((np.sign(m[0, :, :co]) * v)[:, None], L, 1)
+    op = opm.OuterProductMean(1, L, cm, co, co, normalization_epsilon=0.0)
+    op.prepare(w)
+    got = op(torch.from_numpy(m).to(dev), torch.ones(1, L, device=dev)).cpu().numpy()
+    assert np.array_equal(got, expect)

@@ -180,9 +180,11 @@ def test_invalid_input_raises_range_error(dev):
 @pytest.mark.parametrize("direction", ["outgoing", "incoming"])
 @pytest.mark.parametrize("length,cz,ch,pair_dtype,out_dtype,residual,shift", [
     (1, 4, 8, "f32", "f32", False, 0), (8, 31, 33, "f32", "f32", True, 1), (9, 128, 256, "f16", "f32", False, 0),
-    (33, 100, 72, "f32", "f16", True, 1), (23, 64, 224, "f16", "f32", True, 3), (90, 128, 128, "f32", "f32", False, 0)])
+    (33, 100, 72, "f32", "f16", True, 1), (23, 64, 224, "f16", "f32", True, 3), (90, 128, 128, "f32", "f32", False, 0),
+    (1, 64, 65, "f32", "f32", False, 0), (8, 67, 97, "f32", "f32", True, 1)])
 def test_f32_pair_kernels(dev, direction, length, cz, ch, pair_dtype, out_dtype, residual, shift):
-    # f32 precision's projection and output kernels over pairs of f16: ragged
+    # f32 precision's projection and output kernels, over pairs of f16 from 64
+    # channels on both sides and on the f32 MFMA below: ragged
     # tiles of 64 pairs, channels short of their 32-wide padding, one to four
     # column splits, z and the output off 16-byte alignment (shift elements),
     # f16 storage, the residual. The input LayerNorm's scales and the columns of
@@ -245,3 +247,30 @@ def test_f32_in_place_is_bit_identical(dev, direction, length, ch, storage, bloc
     expect = op(z, mask, out=z.clone())
     got = op(z, mask, out=z)
     assert torch.equal(got, expect)
+
+
+@pytest.mark.parametrize("cz,ch", [(16, 16), (48, 48), (32, 128), (128, 32)])
+def test_f32_keeps_every_bit_of_short_sums(dev, cz, ch):
+    # Below 64 channels the products stay on the f32 MFMA. A contraction of
+    # +-2^20 leaves its LayerNorm as +-1, so with one weight a row of linearZ and
+    # open gates the outputs are those weights, all 24 bits of them; pairs of f16
+    # hold one in four to 23 bits.
+    import torch
+
+    from afhip import triangle
+
+    inp = ref.deterministic_triangle_input(1, cz, ch, seed=cz + ch)
+    w = {k: np.zeros_like(np.asarray(v, np.float32)) for k, v in inp["weights"].items()}
+    sign = np.where(np.arange(ch) % 2 == 0, 1, -1).astype(np.float32)
+    v = np.float32(1) + (2 * np.floor(ref.uniform(cz, (cz,), 0, 2 ** 22)) + 1).astype(np.float32) * np.float32(2 ** -23)
+    w["layerNormInWeight"] += 1
+    w["layerNormOutWeight"] += 1
+    w["linearAPBias"] += 2 ** 10 * sign
+    w["linearBPBias"] += 2 ** 10
+    for name in ("linearAGBias", "linearBGBias", "linearGBias"):
+        w[name] += 200
+    w["linearZWeight"][np.arange(cz), np.arange(cz) % ch] = v
+    op = triangle.TriangleMultiplication(1, cz, ch)
+    op.prepare(w)
+    got = op(torch.from_numpy(inp["z"]).to(dev), torch.ones(1, 1, device=dev)).cpu().numpy().reshape(-1)
+    assert np.array_equal(got, v * sign[np.arange(cz) % ch])
