@@ -66,8 +66,8 @@ bool pair_path(const afhip_attention_desc& d) {
 // Prepared weights: everything the kernels read, in their dtypes.
 struct AttentionWeights {
   size_t ln_scale, ln_offset, w_proj, b_proj, w_out, b_out, pair_scale, pair_offset, w_bias, total;
-  // The pair path: output scales of the two products, each head's logit scale
-  // and value exponent, and the bounds they were taken from.
+  // The pair path: output scales of the two products, each head's logit scale,
+  // each channel's value exponent, and the bounds they were taken from.
   size_t s_proj, s_out, logit_scale, v_exp, bound;
 };
 
@@ -95,7 +95,7 @@ AttentionWeights weights_layout(const afhip_attention_desc& d) {
     w.s_proj = take(4 * 4 * C);
     w.s_out = take(4 * C);
     w.logit_scale = take(4 * (size_t)d.heads);
-    w.v_exp = take(4 * (size_t)d.heads);
+    w.v_exp = take(4 * C);
     w.bound = take(4 * 4 * C);
   }
   w.total = at;
@@ -287,32 +287,42 @@ __global__ __launch_bounds__(256) void attention_pair_project_kernel(const float
   }
 }
 
-// One wave a head: q, k and v leave the projection times the power of two that
-// takes the head's largest bound to [2^14, 2^15], so the flash kernel's pairs
-// hold them whatever the input; the logits carry 2^(q + k) back, and v's
-// exponent, which the attention's output keeps, goes into the output weights.
+// One wave a head: q, k and v leave the projection times powers of two, one a
+// channel, under which the flash kernel's pairs hold them whatever the input. Of
+// a channel's q and k only the product counts, and weights may put any factor
+// into one and its inverse into the other: their exponents add up to one S for
+// the head, which the logits carry back. The channel with the largest product of
+// bounds is at 2^15 in both, the others balanced below it. A channel of v
+// has an exponent of its own, which the attention's output keeps and the output
+// weights take back.
 __global__ __launch_bounds__(64) void attention_pair_heads_kernel(int C, int H, const float* __restrict__ bound,
                                                                   float* __restrict__ s_proj,
                                                                   float* __restrict__ b_proj,
                                                                   float* __restrict__ logit_scale,
                                                                   int* __restrict__ v_exp) {
   const int h = blockIdx.x, lane = threadIdx.x, d = C / H;  // d <= 32
-  int exps[3];
+  const int n = h * d + lane;
+  const bool in = lane < d;
+  int e[3];  // takes each bound to 2^15
 #pragma unroll
-  for (int part = 0; part < 3; part++) {
-    const int n = part * C + h * d + lane;
-    float most = lane < d ? bound[n] : 0.0f;
-    for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
-    exps[part] = pair_exponent(most);
-    if (lane < d) {
-      s_proj[n] = ldexpf(s_proj[n], exps[part]);
-      b_proj[n] = ldexpf(b_proj[n], exps[part]);
+  for (int part = 0; part < 3; part++) e[part] = in ? pair_exponent(bound[part * C + n]) : 0;
+  const bool product = in && bound[n] > 0.0f && bound[C + n] > 0.0f;
+  constexpr int kNone = 1 << 20;
+  int S = product ? e[0] + e[1] : kNone;
+  for (int o = 32; o > 0; o >>= 1) S = min(S, __shfl_xor(S, o));
+  if (product) {  // S <= e[0] + e[1]: both exponents go down
+    e[0] -= (e[0] + e[1] - S + 1) / 2;
+    e[1] = S - e[0];
+  }
+  if (in) {
+#pragma unroll
+    for (int part = 0; part < 3; part++) {
+      s_proj[part * C + n] = ldexpf(s_proj[part * C + n], e[part]);
+      b_proj[part * C + n] = ldexpf(b_proj[part * C + n], e[part]);
     }
+    v_exp[n] = e[2];
   }
-  if (lane == 0) {
-    logit_scale[h] = ldexpf(1.0f, min(max(-(exps[0] + exps[1]), -120), 120));
-    v_exp[h] = exps[2];
-  }
+  if (lane == 0) logit_scale[h] = S == kNone ? 1.0f : ldexpf(1.0f, min(max(-S, -120), 120));
 }
 
 // The output projection, one workgroup a row n of [C][C], and the tensors that
@@ -321,9 +331,9 @@ __global__ __launch_bounds__(256) void attention_pair_output_kernel(const float*
                                                                     int separate, int has_bias,
                                                                     const int* __restrict__ v_exp,
                                                                     AttentionPairOut o) {
-  const int n = blockIdx.x, d = C / H;
+  const int n = blockIdx.x;
   const float* w = packed + 3 * (int64_t)C + 4 * (int64_t)C * C;  // [k][C]
-  auto value = [&](int k) { return ldexpf(w[(int64_t)k * C + n], -v_exp[k / d]); };
+  auto value = [&](int k) { return ldexpf(w[(int64_t)k * C + n], -v_exp[k]); };
   float most = 0.0f;
   for (int k = threadIdx.x; k < C; k += 256) most = fmaxf(most, fabsf(value(k)));
   __shared__ float part[4];

@@ -459,3 +459,22 @@ def test_f32_keeps_every_bit_of_short_sums(dev, C, H):
          "outputWeight": np.eye(C, dtype=np.float32), "outputBias": np.zeros(C, np.float32)}
     got = run_case(dev, x.reshape(-1), np.ones(B, np.float32), B, 1, C, H, True, w, None)
     assert np.array_equal(got.reshape(B, C), np.sign(x) * v)
+
+
+@pytest.mark.parametrize("C,H", [(64, 2), (64, 8), (80, 16)])
+@pytest.mark.parametrize("name,S,L", [("msa_column", 97, 2), ("msa_row", 3, 33)])
+def test_f32_channels_of_any_scale(dev, name, S, L, C, H):
+    # Query channels times 1e-6 to 1e6 and the key channels divided by the same,
+    # values likewise against the output weights' rows: each channel of a head
+    # has its own factor, and none of them is in the result. The f32 bound.
+    x, mask, B, Q, tr, w, pb = case(name, S, L, C, H, Cp=12)
+    fk, fv = 10.0 ** ref.uniform(95, (C,), -6, 6), 10.0 ** ref.uniform(96, (C,), -6, 6)
+    w = {k: np.array(v, np.float64).reshape(v.shape) for k, v in w.items()}
+    w["queryWeight"] = w["queryWeight"] * fk
+    w["keyWeight"] = w["keyWeight"] / fk
+    w["valueWeight"] = w["valueWeight"] * fv
+    w["outputWeight"] = w["outputWeight"] / fv[:, None]
+    w = {k: v.astype(np.float32) for k, v in w.items()}
+    expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
+    got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb)
+    assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()
