@@ -795,7 +795,7 @@ template <typename CT> int launch_flash_f32(const FlashArgs& fa, hipStream_t st)
 // The same attention over pairs of f16 (f32 precision): q, k and v arrive in f32,
 // scaled by powers of two that keep them below 2^15 (attention_pair_heads_kernel),
 // and are split into h + l as they are loaded; the weights e^(x - m) are split
-// times 2^kPairWeight. Three products (h h, h l, l h) a step of 16 on the f16 MFMA, 384
+// times 2^pair_weight_exponent. Three products (h h, h l, l h) a step of 16 on the f16 MFMA, 384
 // cycles a block at head dimension 32 against 2,048. Loads, key order, clamp and
 // offset as in the f32 kernel above; the output, still times v's power of two,
 // leaves as pairs for the output projection.
@@ -803,10 +803,12 @@ template <typename CT> int launch_flash_f32(const FlashArgs& fa, hipStream_t st)
 // its own), which the next kernel shares where there are blocks enough. Column attention over 508 sequences x 59 residues, 8 heads of 32:
 // 115 us, the f32 kernel 163; dropping a third of the vector instructions
 // (v_fma_mix_f32 in the split, no per-load bound) left it at 117.
-// log2: keeps small weights' l out of f16's last digits. A weight is at most
-// 2^(kPairWeight + 2.9) (the slack), times 2^8 where every key is masked: there
-// x = m = -1e8, and the rounding of `offset` is up to 8. That is below 65504.
-constexpr float kPairWeight = 4.0f;
+// The weights' exponent under the offset m. A weight is at most 2^2.9 (the slack)
+// times 2^12, below f16's largest, and the error of its pairs is 2^-37, so that
+// thousands of small ones beside a large one still add up. Past |m| = 2^17 (masked
+// keys: m = -1e8) the rounding of `offset` scales the weights by up to 2^8 either
+// way, and the exponent leaves room for that.
+__device__ __forceinline__ float pair_weight_exponent(float m) { return fabsf(m) < 131072.0f ? 12.0f : 4.0f; }
 
 // LOAD: a lane's channels element by element (0), in 16-byte chunks (1, head
 // dimension a multiple of four) or in whole steps (2, exactly 16 STEPS channels).
@@ -942,12 +944,13 @@ __global__ __launch_bounds__(64 * kF32Waves) void attention_flash_pair_kernel(Fl
     for (int v = 1; v < 16; v++) mx = fmaxf(mx, x[v]);
     if (__builtin_amdgcn_ballot_w64(mx > m + kF32Slack)) {
       const float to = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)));
-      const float f = __builtin_amdgcn_exp2f((m - to) * kLog2e);
+      const float exponent = pair_weight_exponent(to);
+      const float f = __builtin_amdgcn_exp2f(fmaf(m - to, kLog2e, exponent - pair_weight_exponent(m)));
       sum *= f;
 #pragma unroll
       for (int v = 0; v < 16; v++) o[v] *= f;
       m = to;
-      offset = fmaf(-to, kLog2e, kPairWeight);
+      offset = fmaf(-to, kLog2e, exponent);
     }
 #pragma unroll
     for (int v = 0; v < 16; v++) x[v] = __builtin_amdgcn_exp2f(fmaf(x[v], kLog2e, offset));
@@ -1123,12 +1126,13 @@ __global__ __launch_bounds__(64 * kF32Waves) void attention_flash_pair32_kernel(
       for (int v = 1; v < 16; v++) mx = fmaxf(mx, x[v]);
       if (__builtin_amdgcn_ballot_w64(mx > m + kF32Slack)) {
         const float to = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)));
-        const float f = __builtin_amdgcn_exp2f((m - to) * kLog2e);
+        const float exponent = pair_weight_exponent(to);
+        const float f = __builtin_amdgcn_exp2f(fmaf(m - to, kLog2e, exponent - pair_weight_exponent(m)));
         sum *= f;
 #pragma unroll
         for (int v = 0; v < 16; v++) o[v] *= f;
         m = to;
-        offset = fmaf(-to, kLog2e, kPairWeight);
+        offset = fmaf(-to, kLog2e, exponent);
       }
 #pragma unroll
       for (int v = 0; v < 16; v++) x[v] = __builtin_amdgcn_exp2f(fmaf(x[v], kLog2e, offset));

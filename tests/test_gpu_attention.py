@@ -478,3 +478,29 @@ def test_f32_channels_of_any_scale(dev, name, S, L, C, H):
     expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
     got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb)
     assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("C,H", [(64, 2), (64, 8)])
+def test_f32_many_small_weights(dev, C, H):
+    # One key 20.45 above 2,047 others, whose value in channel 5 is 500 times that
+    # key's: their weights, e^-20.45 = 2^-29.5 each, make 1.3e-3 of the result. An
+    # error of 2^-25 in weights that are held times 2^12 moves it by 2^-7.5 of
+    # that, 7e-6.
+    Q, j = 2048, 5
+    x = np.full((Q, C), -1, np.float32)
+    x[:, j] = C - 1
+    x[0] = np.where(np.arange(C) % 2 == 0, 1, -1)
+    x[0, j], x[0, j - 1] = 1 / 64, -1 / 64
+    act = np.where(np.arange(Q)[None, :, None] == 0, 1, -1) * np.array([1, 1, -1, -1]) * np.ones((Q, 1, 1))
+    pb = {"source": "separate", "activations": (1024 * act).astype(np.float32), "channels": 4,
+          "layerNormScale": np.ones(4, np.float32), "layerNormOffset": np.zeros(4, np.float32),
+          "projectionWeight": np.repeat(np.array([[1], [1], [-1], [-1]], np.float32) * np.float32(20.45 / 8), H, 1)}
+    w = {"queryNormScale": np.ones(C, np.float32), "queryNormOffset": np.zeros(C, np.float32),
+         **{k + "Weight": np.zeros((C, C), np.float32) for k in ("query", "key", "gating")},
+         "valueWeight": np.eye(C, dtype=np.float32), "gatingBias": np.full(C, 200, np.float32),
+         "outputWeight": np.eye(C, dtype=np.float32), "outputBias": np.zeros(C, np.float32)}
+    x = (1024 * x).astype(np.float32)
+    mask = np.ones(Q, np.float32)
+    expect = ref.attention(x.reshape(-1), mask, w, 1, Q, C, H, pair_bias=pb).reshape(Q, C)[:, j]
+    got = run_case(dev, x.reshape(-1), mask, 1, Q, C, H, False, w, pb).reshape(Q, C)[:, j]
+    assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()
