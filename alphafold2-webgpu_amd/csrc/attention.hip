@@ -305,7 +305,8 @@ __global__ __launch_bounds__(64) void attention_pair_heads_kernel(int C, int H, 
   const bool in = lane < d;
   int e[3];  // takes each bound to 2^15
 #pragma unroll
-  for (int part = 0; part < 3; part++) e[part] = in ? pair_exponent(bound[part * C + n]) : 0;
+  for (int part = 0; part < 3; part++) e[part] = in ? pair_exponent_of(bound[part * C + n]) : 0;
+  e[2] = min(e[2], 110);  // the output weights take it back
   const bool product = in && bound[n] > 0.0f && bound[C + n] > 0.0f;
   constexpr int kNone = 1 << 20;
   int S = product ? e[0] + e[1] : kNone;

@@ -75,14 +75,16 @@ __device__ __forceinline__ void pair_store(half_t* row, int64_t k, float x) {
   row[pair_index(k) + 16] = l;
 }
 // The power of two (its exponent) that takes values of magnitude up to `most`
-// into (-2^15, 2^15), the largest past 2^14; 0 where there are none or they are
-// not finite. Bounded so that the exponents a result adds up stay in f32.
-__device__ __forceinline__ int pair_exponent(float most) {
-  if (!(most > 0.0f) || !isfinite(most)) return 0;
+// into [-2^15, 2^15], the largest past 2^14; 0 where there are none. An infinite
+// `most` is a bound past the largest f32 on values that are none of them past it.
+__device__ __forceinline__ int pair_exponent_of(float most) {
+  if (!(most > 0.0f)) return 0;
   int p;
-  frexpf(most, &p);  // most = m 2^p, m in [1/2, 1)
-  return min(max(15 - p, -110), 110);
+  frexpf(fminf(most, 3.402823466e38f), &p);  // m 2^p, m in [1/2, 1)
+  return 15 - p;
 }
+// Bounded so that the exponents a result adds up stay in f32.
+__device__ __forceinline__ int pair_exponent(float most) { return min(pair_exponent_of(most), 110); }
 // A LayerNorm's output before its affine: C values of magnitude at most
 // sqrt(C), stored times 2^pair_norm_exponent(C), at most 2^15.
 inline int pair_norm_exponent(int C) {

@@ -9,6 +9,7 @@
 // at 64, 128 or 256 channels, one wave per row otherwise) and both linears run
 // through the shared GEMM.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 
 #include "gemm.h"
@@ -195,14 +196,19 @@ __global__ __launch_bounds__(256) void pair_first_kernel(const float* __restrict
     const double bias = f[(size_t)C * H + h] + offset;
     const int e = pair_exponent(most);
     const int u = -pair_exponent((float)(sqrt((double)C * squares) + fabs(bias)));
+    // An infinite weight's pairs are NaN, which the ReLU would make zero: its unit
+    // is infinite whatever the row.
+    const bool infinite = most == INFINITY;
     s1[h] = ldexpf(1.0f, -(x_exp + e + u));
-    b1[h] = (float)ldexp(bias, -u);
-    shift[h] = u;
-    exps[r] = e;
+    b1[h] = infinite ? INFINITY : (float)ldexp(bias, -u);
+    shift[h] = infinite ? 0 : u;
+    exps[r] = infinite ? INT_MIN : e;
   }
   __syncthreads();
   pair_transpose(f, C, H, h0, w1, tile,
-                 [&](int c, int row, float w) { return (float)ldexp((double)w * gamma[c], exps[row]); });
+                 [&](int c, int row, float w) {
+                   return exps[row] == INT_MIN ? 0.0f : (float)ldexp((double)w * gamma[c], exps[row]);
+                 });
 }
 
 __global__ __launch_bounds__(256) void pair_second_kernel(const float* __restrict__ packed, int C, int H,

@@ -504,3 +504,21 @@ def test_f32_many_small_weights(dev, C, H):
     expect = ref.attention(x.reshape(-1), mask, w, 1, Q, C, H, pair_bias=pb).reshape(Q, C)[:, j]
     got = run_case(dev, x.reshape(-1), mask, 1, Q, C, H, False, w, pb).reshape(Q, C)[:, j]
     assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("C,H", [(64, 2), (64, 8)])
+def test_f32_largest_weights(dev, C, H):
+    # A query and a value channel with one weight of 1.6e38 each: the logits are
+    # all clamped, to either side, and v, up to 1e37, meets output weights of 1e-36. A
+    # bound on either channel from its weights' norm passes the largest f32. The f32 bound.
+    x, mask, B, Q, tr, w, pb = case("msa_column", 70, 2, C, H, Cp=12)
+    w = {k: np.array(v, np.float32).reshape(v.shape) for k, v in w.items()}
+    x = x.reshape(-1, C).copy()
+    x[:, 0] = ref.uniform(97, (len(x),), -0.01, 0.01)
+    for name in ("queryWeight", "valueWeight"):
+        w[name][:, 3] = 0
+        w[name][0, 3] = 1.6e38
+    w["outputWeight"][3] *= 1e-36
+    expect = ref.attention(x.reshape(-1), mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
+    got = run_case(dev, x.reshape(-1), mask, B, Q, C, H, tr, w, pb)
+    assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()

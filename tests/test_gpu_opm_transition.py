@@ -473,3 +473,52 @@ def test_opm_f32_keeps_every_bit_of_short_sums(dev, cm):
     op.prepare(w)
     got = op(torch.from_numpy(m).to(dev), torch.ones(1, L, device=dev)).cpu().numpy()
     assert np.array_equal(got, expect)
+
+
+@pytest.mark.parametrize("big,small", [(1.6e38, 1e-37), (np.inf, 1.0)])
+def test_transition_f32_largest_weights(dev, big, small):
+    # A hidden unit with one weight of 1.6e38 against output weights of 1e-37:
+    # the unit reaches 2e38 and a bound on it from the weights' norm passes the
+    # largest f32. The f32 bound. An infinite weight shows: no row of it is finite.
+    import torch
+
+    from afhip import transition
+
+    inp = transition_case(130, 64, 64, 3)
+    x, w = inp["activations"].copy(), {k: np.array(v, np.float32) for k, v in inp["weights"].items()}
+    x[:, 0] = ref.uniform(98, (len(x),), -1, 1)
+    w["firstWeight"][:, 5] = 0
+    w["firstWeight"][0, 5] = big
+    w["secondWeight"][5] *= small
+    expect = ref.transition(x, w)
+    op = transition.Transition(130, 64, 64)
+    op.prepare(w)
+    got = op(torch.from_numpy(x).to(dev)).cpu().numpy()
+    if np.isfinite(big):
+        assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()
+    else:
+        assert not np.isfinite(expect).all() and not np.isfinite(got).any()
+
+
+def test_opm_f32_largest_weights(dev):
+    # As above: a left channel's weight against its output weights.
+    import torch
+
+    from afhip import opm
+
+    S, L, cm, co, cz = 4, 5, 64, 8, 16
+    m, mask = ref.normal(61, (S, L, cm)), np.ones((S, L), np.float32)
+    m[..., 0] = ref.uniform(62, (S, L), -1, 1)
+    w = {"layerNormScale": ref.normal(63, (cm,), 0.01, 1.0), "layerNormOffset": ref.normal(64, (cm,), 0.01),
+         "leftWeight": ref.normal(65, (cm, co), 1 / cm), "leftBias": ref.normal(66, (co,), 0.02),
+         "rightWeight": ref.normal(67, (cm, co), 1e-4 / cm), "rightBias": ref.normal(68, (co,), 1e-4),
+         "outputWeight": ref.normal(69, (co * co, cz), 1 / (co * co)), "outputBias": ref.normal(70, (cz,), 0.02)}
+    w = {k: np.array(v, np.float32) for k, v in w.items()}
+    w["leftWeight"][:, 5] = 0
+    w["leftWeight"][0, 5] = 1.6e38
+    w["outputWeight"][5 * co:6 * co] *= 1e-37
+    expect = ref.opm(m, mask, w)
+    op = opm.OuterProductMean(S, L, cm, co, cz)
+    op.prepare(w)
+    got = op(torch.from_numpy(m).to(dev), torch.from_numpy(mask).to(dev)).cpu().numpy()
+    assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()

@@ -274,3 +274,28 @@ def test_f32_keeps_every_bit_of_short_sums(dev, cz, ch):
     op.prepare(w)
     got = op(torch.from_numpy(inp["z"]).to(dev), torch.ones(1, 1, device=dev)).cpu().numpy().reshape(-1)
     assert np.array_equal(got, v * sign[np.arange(cz) % ch])
+
+
+def test_f32_largest_weights(dev):
+    # Weights of 1.6e38 in a gate, which they open or shut, and of 4.5e37 in
+    # linearZ, whose channel is compared by itself. The f32 bound.
+    import torch
+
+    from afhip import triangle
+
+    length, cz, ch = 9, 64, 64
+    inp = ref.deterministic_triangle_input(length, cz, ch, seed=5)
+    w = {k: np.array(v, np.float32) for k, v in inp["weights"].items()}
+    w["linearAGWeight"][7, 0] = 1.6e38
+    w["linearZWeight"][9] = 0
+    w["linearZWeight"][9, 3] = 4.5e37
+    mask = np.ascontiguousarray(inp["mask"], np.float32)
+    expect = ref.triangle("outgoing", inp["z"], mask, w)
+    op = triangle.TriangleMultiplication(length, cz, ch)
+    op.prepare(w)
+    got = op(torch.from_numpy(np.ascontiguousarray(inp["z"], np.float32)).to(dev), torch.from_numpy(mask).to(dev))
+    got = got.cpu().numpy().reshape(expect.shape)
+    assert np.isfinite(expect).all() and np.abs(expect[..., 9]).max() > 1e37
+    assert rel_max(got[..., 9] / 1e30, expect[..., 9] / 1e30) <= 1e-5
+    rest = np.arange(cz) != 9
+    assert rel_max(got[..., rest], expect[..., rest]) <= 1e-5
