@@ -405,9 +405,12 @@ def test_f32_pairs_attention(dev, name, S, L, residual, shift, C, H):
 @pytest.mark.parametrize("C,H", [(32, 4), (64, 8), (96, 12)])
 @pytest.mark.parametrize("name,S,L,scale", [("msa_row", 3, 1, 1), ("msa_row", 2, 33, 12), ("msa_column", 31, 3, 4),
                                             ("msa_column", 97, 2, 4), ("triangle_end", 0, 64, 1),
-                                            ("triangle_start", 0, 65, 12)])
+                                            ("triangle_start", 0, 65, 12), ("msa_row", 520, 1, 1),
+                                            ("msa_row", 600, 33, 12), ("msa_column", 31, 520, 4),
+                                            ("msa_column", 97, 200, 4), ("triangle_start", 0, 130, 12)])
 def test_f16_four_heads_of_eight(dev, name, S, L, scale, C, H):
-    # Head dimension 8 with heads in fours: ragged blocks of 32 queries and
+    # Head dimension 8 with heads in fours, in calls of 512 tiles of 32 queries or
+    # more by a kernel of their own: ragged blocks of 32 queries and
     # keys, fully masked rows, and logits that spread (the pair bias, or the
     # queries, scaled up) so that the softmax offset moves in later blocks. Above
     # 64 queries a masked tail too. The general f16 bound of 1e-2.
