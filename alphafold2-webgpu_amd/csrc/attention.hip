@@ -2222,10 +2222,13 @@ int afhip_attention_run(const afhip_attention_desc* desc, const void* activation
       g.flags |= AFHIP_EPILOGUE_SCALE;
       if ((s = run_gemm_pairs(g, AFHIP_F32, "attention.project", st))) return s;
     } else if (const afhip_variant v = select_variant(t, g.M, g.N, g.K, 1);
-               v.source == 0 && C == 64 && g.M >= 16384 && stream_eligible(g, t)) {
-      // 256 columns are few for STREAM's rule (heuristic_variant), but a K of 64 is all
-      // output: 60416 x 64 x 256 on MI355X 14.5 us against 26 on LDS_DMA tiles,
-      // 153600 rows 20 against 56.
+               v.source == 0 && C == 64 && stream_eligible(g, t)) {
+      // Of the widths STREAM takes, 64 channels make 256 columns, too few for the
+      // GEMM plans' rule (heuristic_variant); but a K of 64 is all output, and a tile
+      // of the other kernels is two steps of loads with nothing beside them. Whole
+      // calls on MI355X, 8 heads, STREAM / as selected, us: 50 rows 17.7 / 29.3,
+      // 2,000 19.1 / 30.9, 8,000 21.0 / 31.0, 26,000 36.9 / 37.1, 32,000 39.4 / 38.7,
+      // 60,400 45 / 63, 153,600 76 / 112.
       if ((s = run_gemm_stream(g, t, "attention.project", st))) return s;
     } else if ((s = run_gemm(g, t, v, "attention.project", st))) {
       return s;
