@@ -70,8 +70,10 @@ OpmWeights opm_layout(const afhip_opm_desc& d) {
     at = round_up((int64_t)(at + bytes), 256);
     return here;
   };
-  w.ln_scale = take(4 * (size_t)d.c_m);
-  w.ln_offset = take(4 * (size_t)d.c_m);
+  if (!opm_pairs(d)) {  // the pair projection's weights hold the LayerNorm's affine
+    w.ln_scale = take(4 * (size_t)d.c_m);
+    w.ln_offset = take(4 * (size_t)d.c_m);
+  }
   w.w_lr = take(es * (size_t)w.cop * w.cmp);
   w.b_lr = take(4 * (size_t)w.cop);
   w.w_out = take(es * (size_t)w.czp * d.c_outer * d.c_outer);
@@ -576,11 +578,12 @@ template <typename MT> int launch_fast_cm(const ProjectArgs& pa, float* count, h
   return launch_fast<256, MT>(pa, count, s);
 }
 
+// `projection` false: the output weights alone (the projection's are prepared as pairs).
 template <typename CT>
 __global__ void opm_prepare_kernel(const float* __restrict__ packed, int cm, int co, int cz, int cmp, int cop, int czp,
                                    CT* __restrict__ w_lr, float* __restrict__ b_lr, CT* __restrict__ w_out,
                                    float* __restrict__ b_out, float* __restrict__ ln_s, float* __restrict__ ln_o,
-                                   bool fused) {
+                                   bool fused, bool projection) {
   const float* ln_scale = packed;
   const float* ln_offset = ln_scale + cm;
   const float* left_w = ln_offset + cm;
@@ -591,7 +594,9 @@ __global__ void opm_prepare_kernel(const float* __restrict__ packed, int cm, int
   const float* out_b = out_w + (size_t)co * co * cz;
   const int64_t n_lr = (int64_t)cop * cmp, n_out = (int64_t)czp * co * co;
   const int64_t total = n_lr + n_out + cop + czp + 2 * cm;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+  const int64_t first = projection ? 0 : n_lr;
+  for (int64_t i = first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
+       i += (int64_t)gridDim.x * blockDim.x) {
     if (i < n_lr) {  // [cop][cmp] <- left/right [cm][co] transposed
       const int n = (int)(i / cmp), k = (int)(i % cmp);
       float v = 0.0f;
@@ -606,11 +611,11 @@ __global__ void opm_prepare_kernel(const float* __restrict__ packed, int cm, int
       w_out[at] = (CT)(n < cz ? out_w[(size_t)k * cz + n] : 0.0f);
     } else if (i < n_lr + n_out + cop) {
       const int n = (int)(i - n_lr - n_out);
-      b_lr[n] = n < co ? left_b[n] : (n < 2 * co ? right_b[n - co] : 0.0f);
+      if (projection) b_lr[n] = n < co ? left_b[n] : (n < 2 * co ? right_b[n - co] : 0.0f);
     } else if (i < n_lr + n_out + cop + czp) {
       const int n = (int)(i - n_lr - n_out - cop);
       b_out[n] = n < cz ? out_b[n] : 0.0f;
-    } else {
+    } else if (projection) {
       const int c = (int)(i - n_lr - n_out - cop - czp);
       if (c < cm) ln_s[c] = ln_scale[c];
       else ln_o[c - cm] = ln_offset[c - cm];
@@ -691,14 +696,13 @@ int afhip_opm_prepare_weights(const afhip_opm_desc* desc, const float* packed, v
   if (d.precision == AFHIP_PRECISION_F16) {
     if (int s = launch("opm.prepare", opm_prepare_kernel<half_t>, grid, block, 0, st, packed, d.c_m, d.c_outer, d.c_z,
                        w.cmp, w.cop, w.czp, (half_t*)(base + w.w_lr), (float*)(base + w.b_lr),
-                       (half_t*)(base + w.w_out), (float*)(base + w.b_out), ln_s, ln_o, fused_ok(d)))
+                       (half_t*)(base + w.w_out), (float*)(base + w.b_out), ln_s, ln_o, fused_ok(d), true))
       return s;
   } else {
     if (int s = launch("opm.prepare", opm_prepare_kernel<float>, grid, block, 0, st, packed, d.c_m, d.c_outer, d.c_z,
                        w.cmp, w.cop, w.czp, (float*)(base + w.w_lr), (float*)(base + w.b_lr),
-                       (float*)(base + w.w_out), (float*)(base + w.b_out), ln_s, ln_o, false))
+                       (float*)(base + w.w_out), (float*)(base + w.b_out), ln_s, ln_o, false, !opm_pairs(d)))
       return s;
-    // The projection's weights again, as pairs over the f32 ones.
     if (!opm_pairs(d)) return AFHIP_OK;
     if (int s = launch("opm.prepare", opm_pair_prepare_kernel, dim3(w.cop), dim3(64), 0, st, packed, d.c_m, d.c_outer,
                        w.cmp, pair_norm_exponent(d.c_m), (half_t*)(base + w.w_lr), (float*)(base + w.s_lr),

@@ -40,8 +40,10 @@ TransitionWeights layout(const afhip_transition_desc& d) {
     at = round_up((int64_t)(at + bytes), 256);
     return here;
   };
-  w.scale = take(4 * (size_t)d.channels);
-  w.offset = take(4 * (size_t)d.channels);
+  if (!pair_shape(d)) {  // the pair path's first linear holds the LayerNorm's affine
+    w.scale = take(4 * (size_t)d.channels);
+    w.offset = take(4 * (size_t)d.channels);
+  }
   w.w1 = take(es * (size_t)d.hidden * d.channels);  // [H][C]
   w.b1 = take(4 * (size_t)d.hidden);
   w.w2 = take(es * (size_t)d.channels * d.hidden);  // [C][H]

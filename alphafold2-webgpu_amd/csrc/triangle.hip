@@ -63,12 +63,14 @@ TriWeights tri_layout(const afhip_triangle_desc& d) {
     at = round_up((int64_t)(at + bytes), 256);
     return here;
   };
-  w.ln_in_w = take(4 * (size_t)d.c_z);
-  w.ln_in_b = take(4 * (size_t)d.c_z);
+  if (!tri_pairs(d)) {  // the pair products' weights hold the LayerNorms' affines
+    w.ln_in_w = take(4 * (size_t)d.c_z);
+    w.ln_in_b = take(4 * (size_t)d.c_z);
+    w.ln_out_w = take(4 * (size_t)d.c_hidden);
+    w.ln_out_b = take(4 * (size_t)d.c_hidden);
+  }
   w.w_proj = take(es * 4 * (size_t)w.chp * w.czp);
   w.b_proj = take(4 * 4 * (size_t)w.chp);
-  w.ln_out_w = take(4 * (size_t)d.c_hidden);
-  w.ln_out_b = take(4 * (size_t)d.c_hidden);
   w.w_z = take(es * (size_t)w.czo * w.chp);
   w.b_z = take(4 * (size_t)w.czo);
   w.w_g = take(es * (size_t)w.czo * w.czp);
