@@ -124,7 +124,7 @@ def test_attention_gpu_run_mirrors_the_reference_call(dev):
 
 @pytest.mark.parametrize("C,H", [(32, 1), (15, 3), (64, 2), (24, 24)])
 def test_general_head_dimensions_f32(dev, C, H):
-    # head dimensions 32, 5, 32 and 1 through the general kernel's instances
+    # head dimensions 32, 5 and 1 on the f32 MFMA, and 32 over pairs of f16 (64 channels)
     x, mask, B, Q, tr, w, pb = case("triangle_start", S=0, L=13, C=C, H=H)
     expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
     got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb)
@@ -338,13 +338,14 @@ def test_f16_mfma_narrow_heads(dev, name, C, H):
 
 
 @pytest.mark.parametrize("C,H,precision", [(64, 16, "f32"), (36, 3, "f32"), (40, 2, "f32"), (84, 3, "f32"), (64, 2, "f32"),
-                                           (10, 1, "f32"), (21, 3, "f16")])
+                                           (10, 1, "f32"), (21, 3, "f16"), (12, 3, "f32"), (24, 3, "f32"), (16, 4, "f32"),
+                                           (48, 3, "f32"), (32, 1, "f32")])
 @pytest.mark.parametrize("name,S,L", [("msa_column", 33, 2), ("msa_column", 65, 3), ("triangle_end", 0, 32),
                                       ("msa_row", 2, 31), ("msa_row", 3, 1)])
 def test_f32_mfma_flash_edges(dev, name, S, L, C, H, precision):
     # The f32 flash kernel at the edges of its 32-query and 32-key blocks and
-    # of its channel paddings (head dimensions 4, 12, 20, 28, 32, 10; 7 in
-    # f16 storage). The query weights are scaled up so that logits
+    # of its channel paddings (head dimensions 12, 20, 28, 10, 4, 8, 16 and 32; 7 in
+    # f16 storage). (64, 16) and (64, 2) run over pairs of f16 instead. The query weights are scaled up so that logits
     # spread over tens of units and the softmax offset moves in later
     # blocks. f32: 16 roundings of logits below 128 (2^-18 each) move a weight
     # by at most 6e-5, the rest is the 1e-5 of the other f32 tests; f16
@@ -524,4 +525,17 @@ def test_f32_largest_weights(dev, C, H):
     w["outputWeight"][3] *= 1e-36
     expect = ref.attention(x.reshape(-1), mask, w, B, Q, C, H, transpose=tr, pair_bias=pb)
     got = run_case(dev, x.reshape(-1), mask, B, Q, C, H, tr, w, pb)
+    assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()
+
+
+@pytest.mark.parametrize("C,H,S,L", [(64, 2, 33, 1000), (128, 4, 29, 300), (256, 8, 40, 110)])
+def test_f32_pairs_large_products(dev, C, H, S, L):
+    # Rows enough for the pair GEMM's 128 x 128 tiles: the projection with its
+    # attention blocks (256 columns: 16,384 rows; 512: 8,192; 1,024: 4,096) and, at
+    # 33,000 rows, the output projection with the residual; ragged last tiles.
+    # The f32 bound of the other tests.
+    x, mask, B, Q, tr, w, pb = case("msa_column", S, L, C, H, Cp=12)
+    old = ref.normal(18, (B * Q * C,))
+    expect = ref.attention(x, mask, w, B, Q, C, H, transpose=tr, pair_bias=pb) + old
+    got = run_case(dev, x, mask, B, Q, C, H, tr, w, pb, residual=old)
     assert np.abs(got - expect).max() <= 1e-5 * np.abs(expect).max()
