@@ -329,13 +329,14 @@ int launch_pair_norm(const void* x, int64_t rows, int C, float eps, void* y, hip
   const float x_scale = ldexpf(1.0f, pair_norm_exponent(C));
   const IT* xi = (const IT*)x;
   half_t* yo = (half_t*)y;
-  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  const unsigned grid = (unsigned)std::min<int64_t>(ceil_div(rows, 4 * (64 / std::max(1, C / 8)) * 4), (int64_t)cus * 8);
   const char* label = "transition.layer_norm";
-  if ((reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
-    if (C == 64) return launch(label, pair_norm_rows_kernel<IT, 8>, dim3(grid), dim3(256), 0, st, xi, rows, eps, x_scale, yo);
-    if (C == 128) return launch(label, pair_norm_rows_kernel<IT, 16>, dim3(grid), dim3(256), 0, st, xi, rows, eps, x_scale, yo);
-    if (C == 256) return launch(label, pair_norm_rows_kernel<IT, 32>, dim3(grid), dim3(256), 0, st, xi, rows, eps, x_scale, yo);
+  const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+  if (aligned && (C == 64 || C == 128 || C == 256)) {
+    const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const int64_t rows_per_block = 4 * (64 / (C / 8)) * 4;  // four waves, four rows in flight per lane
+    const dim3 grid((unsigned)std::min<int64_t>(ceil_div(rows, rows_per_block), (int64_t)cus * 8));
+    auto k = C == 64 ? pair_norm_rows_kernel<IT, 8> : C == 128 ? pair_norm_rows_kernel<IT, 16> : pair_norm_rows_kernel<IT, 32>;
+    return launch(label, k, grid, dim3(256), 0, st, xi, rows, eps, x_scale, yo);
   }
   return launch(label, pair_norm_kernel<IT>, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, st, xi, rows, C, eps,
                 x_scale, yo);

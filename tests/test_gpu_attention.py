@@ -357,7 +357,7 @@ def test_f32_mfma_flash_edges(dev, name, S, L, C, H, precision):
     assert np.abs(got - expect).max() <= (7e-5 if precision == "f32" else 1e-2) * np.abs(expect).max()
 
 
-@pytest.mark.parametrize("C,H", [(16, 4), (80, 16), (48, 4), (64, 4), (112, 4), (128, 4), (96, 32), (144, 12), (64, 16)])
+@pytest.mark.parametrize("C,H", [(16, 4), (80, 16), (48, 4), (64, 4), (112, 4), (128, 4), (96, 32), (144, 12), (64, 16), (544, 17)])
 @pytest.mark.parametrize("name,S,L,residual,shift", [("msa_column", 33, 2, True, 1), ("triangle_start", 0, 65, False, 0),
                                                      ("triangle_end", 0, 31, True, 0), ("msa_row", 3, 32, False, 1)])
 def test_f32_pairs_attention(dev, name, S, L, residual, shift, C, H):

@@ -346,12 +346,12 @@ def test_invalid_opm_and_transition_raise(dev):
     (300, 64, 256, "f16", "f32", True, 0), (257, 128, 512, "f32", "f16", True, 1), (130, 256, 1024, "f32", "f32", True, 0),
     (65, 40, 64, "f32", "f32", False, 0), (16500, 16, 272, "f32", "f32", False, 0), (16500, 256, 64, "f32", "f32", True, 0),
     (1, 64, 64, "f32", "f32", False, 0), (31, 64, 80, "f32", "f32", True, 1), (129, 112, 144, "f32", "f32", False, 1),
-    (16500, 80, 272, "f32", "f32", True, 1)])
+    (16500, 80, 272, "f32", "f32", True, 1), (67, 528, 64, "f32", "f32", False, 0), (33, 1024, 4096, "f32", "f32", True, 0)])
 def test_transition_f32_pairs(dev, rows, c, h, in_dt, out_dt, residual, shift):
     # f32 precision on the f16 matrix units: ragged row and column tiles, both
     # LayerNorm kernels, activations and outputs off 16-byte alignment (shift
     # elements; the workspace and the weights then lie on 4 bytes), f16 in or out, the residual. 16, 40 and 48 channels keep the f32
-    # GEMM, and 16500 rows fill the chip with 128 x 128 tiles (fewer run on 64 x 64). The LayerNorm scales, the first linear's columns and the
+    # GEMM, and 16500 rows fill the chip with 128 x 128 tiles (fewer run on 64 x 64). Widths past the row kernel's 512 channels. The LayerNorm scales, the first linear's columns and the
     # second's rows carry factors of 1e-6 to 1e6 that cancel in the result, as
     # any weight may: the powers of two that the pairs are stored with follow
     # them. f32 out: the f32 bound of the other tests; f16 out: half an ulp of
