@@ -140,9 +140,12 @@ class _TriangleMultiplicationGpu:
     def run(self, inp: dict, options: dict | None = None) -> dict:
         """run(input, {precision?, blockRows?, pairStorage?}) (webgpu.ts:56-201).
 
-        precision "f32" keeps every product and sum in f32; "f16" rounds the
-        operands of every product to f16 and accumulates in f32. The output is
-        f32, as the reference returns a Float32Array.
+        precision "f32" keeps every sum in f32, and every product; from 64
+        channels on both sides the projections' products are taken over pairs
+        of f16 that hold an operand to 22 to 24 bits, with an error against 64
+        bits no larger than the f32 products'. "f16" rounds the operands of
+        every product to f16 and accumulates in f32. The output is f32, as the
+        reference returns a Float32Array.
         """
         import torch
 

@@ -616,9 +616,9 @@ struct FlashArgs {
 // the registers its last use just freed. No LDS, no barrier, up to four waves
 // a SIMD. Four waves of a workgroup take consecutive query blocks, so K and V
 // reach a CU about once; workgroup ids give each XCD a contiguous range.
-// Measured, column attention over 508 sequences x 59 residues, 8 heads of 32
-// (15.6 GFLOP, 101 us at the f32 rate of a large product): 163 us; one thread
-// a query took 1,493 us.
+// Measured over 508 sequences x 59 residues, column attention: 9 heads of 28 200 us.
+// 8 heads of 32 (15.6 GFLOP, 101 us at the f32 rate of a large product) took 163 us
+// here, before pairs of f16 took them (below), and 1,493 us by one thread a query.
 constexpr int kF32Waves = 4;
 constexpr float kF32Slack = 2.0f;
 constexpr float kDropped = -1e30f;    // the logit of a key past the end
@@ -804,10 +804,11 @@ template <typename CT> int launch_flash_f32(const FlashArgs& fa, hipStream_t st)
 // cycles a block at head dimension 32 against 2,048. Loads, key order, clamp and
 // offset as in the f32 kernel above; the output, still times v's power of two,
 // leaves as pairs for the output projection.
-// Bound: the loads (20 instructions a block over 32 rows each, for every wave
-// its own), which the next kernel shares where there are blocks enough. Column attention over 508 sequences x 59 residues, 8 heads of 32:
-// 115 us, the f32 kernel 163; dropping a third of the vector instructions
-// (v_fma_mix_f32 in the split, no per-load bound) left it at 117.
+// Bound: vector instructions, for every wave splits K and V for itself: 16 heads
+// of 16 over 508 sequences x 59 residues 178 us, 50-90% of the cycles in them, 20%
+// in MFMAs. At 8 heads of 32, 115 us (the f32 kernel 163), the loads (20 instructions
+// a block over 32 rows each) bound it as much: a third fewer vector instructions
+// left 117. The next kernel shares both where there are blocks enough.
 // The weights' exponent under the offset m. A weight is at most 2^2.9 (the slack)
 // times 2^12, below f16's largest, and the error of its pairs is 2^-37, so that
 // thousands of small ones beside a large one still add up. Past |m| = 2^17 (masked
@@ -1013,7 +1014,9 @@ template <int STEPS, int LOAD> int launch_flash_pair_as(const FlashArgs& fa, hip
 // transposing ones), double-buffered with one barrier a block. That takes the
 // loads of a block from 20 instructions over 32 rows a wave to two over four,
 // and two thirds of the splitting. Measured, column attention over 508 sequences
-// x 59 residues, 8 heads of 32: 116 us unshared, 83 shared.
+// x 59 residues, 8 heads of 32: 116 us unshared, 83-86 shared. Bound: vector
+// instructions still, 40-73% of the cycles (the softmax and the weights' splitting),
+// MFMAs 27%.
 struct PairTile {
   half_t k[2][32][40];  // [plane][key][channel]
   half_t v[2][32][32];
@@ -1193,6 +1196,11 @@ int launch_flash_pair32(const FlashArgs& fa, hipStream_t st) {
                 per_xcd);
 }
 
+// Shared key blocks above two of them. Whole calls on MI355X, 4 heads of 32 without
+// a bias, unshared over shared, 8 / 59 / 256 batch entries: 64 keys 1.07 1.05 1.01,
+// 65 1.07 1.04 1.04, 128 1.03 1.02 1.07, 129 1.06 1.06 0.97, 160 1.05 1.06 0.99, 200
+// 1.05 1.07 1.09, 256 1.04 1.09 1.16, 508 1.04 1.20 1.24; 2 and 8 heads and a bias
+// are alike. Up to two blocks sharing saves little but the launches' latency.
 int launch_flash_pair(const FlashArgs& fa, hipStream_t st) {
   if (fa.d % 4) return launch_flash_pair_as<2, 0>(fa, st);
   if (fa.d == 32) return fa.Q > 64 ? launch_flash_pair32(fa, st) : launch_flash_pair_as<2, 2>(fa, st);

@@ -46,8 +46,10 @@ constexpr uint32_t EPILOGUE_OPM_CONTRACT = 1u << 16;
 constexpr uint32_t EPILOGUE_OPM_OUTPUT = 1u << 17;
 
 // f32 matrices as pairs of f16 (the pair GEMM, gemm_dma.hip): x = h + l with
-// h = f16(x), l = f16(x - h), 22 to 24 bits of x wherever |x| <= 65504 and x is
-// not tiny beside 2^-14, which the callers see to with power-of-two scales. A
+// h = f16(x), l = f16(x - h), 22 to 24 bits of x wherever 2^-3 <= |x| <= 65504, and
+// within 2^-25 below. The callers hold each row's largest element (or a bound on
+// it) in [2^14, 2^15) with power-of-two scales, so an element keeps its bits down
+// to 2^-17 of that and is within 2^-39 of it below. A
 // row keeps each 16 consecutive k as 16 h, then 16 l (64 bytes); a matrix takes
 // the bytes it takes in f32. K is a multiple of 16.
 __host__ __device__ inline int64_t pair_index(int64_t k) { return 32 * (k >> 4) + (k & 15); }  // of h; l is 16 on

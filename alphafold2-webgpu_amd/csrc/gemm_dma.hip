@@ -11,9 +11,10 @@
 // the outer-product-mean contraction and the f16 projections.
 //
 // PAIRS: f32 operands held as pairs of f16 (gemm.h), three products on the f16
-// MFMA: 96 cycles for 32 x 32 x 16 against 512 of the f32 MFMA. Bound by the
-// LDS reads beside the MFMAs (8 KiB a wave for 384 cycles of MFMA) and, with
-// pairs or f32 out, the output's bytes.
+// MFMA: 96 cycles for 32 x 32 x 16 against 512 of the f32 MFMA. No one unit
+// bounds it: at 29,972 x 256 x 1,024 (69 us) MFMAs are busy 37% of the time,
+// vector instructions (the epilogue's scales and splitting) 25-46%, LDS 21%, and
+// a wave waits a third of its time; K = 256 is 16 steps between a ramp-up and that epilogue.
 //
 // Design:
 //  - One workgroup of WM x WN wave64s owns a BM x BN output tile (each wave

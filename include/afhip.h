@@ -54,7 +54,11 @@ extern "C" {
 #define AFHIP_I8 2
 
 /* Arithmetic of a kernel's products and accumulator.
- * F32: f32 operands, f32 products and sums (MFMA f32).
+ * F32: f32 operands, f32 products and sums (MFMA f32). The transition, the
+ *      attention, the triangle's projections and the outer-product mean's take
+ *      sums of 64 products or more over operands held as two f16 values (22 to
+ *      24 bits; three MFMA f16 products, f32 sums), whose error against 64 bits
+ *      is no larger.
  * F16: operands rounded to f16, f32 accumulation (MFMA f16); the reference's
  *      "matrix" precision with an f16 unit (src/runtime/gemm.ts:150-206).
  * Pure f16 accumulation is never offered, as SHIPPABLE_GEMM_PRECISIONS
@@ -243,7 +247,10 @@ AFHIP_API int afhip_gemm_select(const afhip_gemm_desc* desc, afhip_variant* out)
  * returned (source 0), as the reference keeps its f32 kernel. */
 AFHIP_API int afhip_gemm_calibrate(const afhip_gemm_desc* desc, afhip_variant* out);
 /* Pins a variant for every plan created afterwards (NULL unpins); the
- * counterpart of forceGemmVariant (gemm-selection.ts:122-125). */
+ * counterpart of forceGemmVariant (gemm-selection.ts:122-125). The products that
+ * the operators run as plans take a pinned or calibrated variant too; kernels of
+ * an operator's own (fused ones, and f32 precision's products over pairs of f16)
+ * have no variants. */
 AFHIP_API int afhip_gemm_force_variant(const afhip_variant* variant);
 /* Calibration document (JSON, keyed by device, driver and shape class);
  * the counterpart of readCalibration/writeCalibration
