@@ -1688,24 +1688,23 @@ bool heads8_eligible(const afhip_attention_desc& d) {
 // It has a quarter of the other kernel's waves, each with four heads in turn, and
 // shares nothing between them: it needs waves enough, more of them the longer a
 // wave runs, and every batch entry reads the pair bias again, which from 200 keys
-// on costs more than the barriers did, and sooner where its rows all start at
-// the same place of a cache line. Whole calls on MI355X, 8 heads of 8, the other
-// kernel's time over this one's, batch x keys (tiles):
+// on costs more than the barriers did, and sooner where its rows lie a multiple of
+// 256 bytes apart. Whole calls on MI355X, 8 heads of 8, the other kernel's time
+// over this one's, batch x keys (tiles):
 //   no bias: 59 x 16 (118) 0.95, 59 x 64 (236) 0.95, 30 x 160 (300) 0.93, 59 x 100
 //   (472) 1.06, 100 x 160 (1,000) 1.34, 300 x 256 (4,800) 1.24, 1,024 x 384 (24,576)
-//   1.35; long: 4 x 2,048 (512) 0.71, 59 x 384 (1,416) 0.96, 59 x 1,024 (3,776) 1.10,
-//   59 x 4,096 (15,104) 1.16
+//   1.35; long: 4 x 2,048 (512) 0.71, 59 x 384 (1,416) 0.96, 14 x 4,096 (3,584) 0.99,
+//   29 x 2,048 (3,712) 1.06, 59 x 1,024 (3,776) 1.10
 //   bias: 59 x 59 (236) 0.96, 59 x 100 (472) 0.99, 100 x 100 (800) 1.11, 1,024 x 150
-//   (10,240) 1.47, 1,024 x 200 (14,336) 1.21, x 208 1.13, x 240 1.03, x 384 0.67; rows
-//   of whole lines: 150 x 128 (1,200) 0.91, 1,024 x 128 (8,192) 1.07, x 160 1.08,
-//   x 192 0.93, x 224 0.85, x 256 0.75
+//   (10,240) 1.47, x 160 1.08, x 200 1.21, x 208 1.13, x 240 1.03, x 384 0.67; rows 256
+//   bytes apart: 512 x 64 (2,048) 1.16, 150 x 128 (1,200) 0.91, 1,024 x 128 (8,192)
+//   1.07, x 192 0.93, x 256 0.75
 bool heads8_better(const afhip_attention_desc& d) {
-  const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256, full = 16 * cus;  // waves the chip holds
+  const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;  // 16 waves fit each
   const int64_t Q = d.queries, tiles = (int64_t)d.batch * (d.heads / 4) * ceil_div(Q, 32);
-  if (!d.pair_bias) return tiles >= std::max(2 * cus, std::min(4 * Q, full));
-  const bool whole_lines = Q % 32 == 0;
-  if (Q > (whole_lines ? 160 : 200)) return false;
-  return tiles >= (whole_lines && Q >= 128 ? full : std::max(2 * cus, 5 * Q));
+  if (!d.pair_bias) return tiles >= std::max(2 * cus, std::min(4 * Q, 14 * cus));
+  if (Q % 64 == 0 && Q >= 128) return Q == 128 && tiles >= 16 * cus;
+  return Q <= 200 && tiles >= std::max(2 * cus, 5 * Q);
 }
 
 int launch_flash_heads8(const FlashArgs& fa, hipStream_t st) {
